@@ -21,8 +21,12 @@
 // iteration both right-hand sides vanish, so the coupled and the segregated
 // (SIMPLE) iterations share their fixed point.
 //
-// Storage (device numbering): block CSR, diagonal blocks apart, each block 16
-// contiguous values row-major; vectors interleaved [n][4] = (p, u, v, w).
+// Storage (device numbering): of an off-diagonal block's 16 entries eight are
+// zero and the others are five numbers -- the pressure-matrix entry (0, 0), the
+// momentum-matrix entry (1..3, 1..3) and one coupling per component, the same
+// in (0, k) and (k, 0) -- kept as five arrays over the slots of the scalar
+// pattern (sliced ELL, entry pairs); a diagonal block is its two scalar
+// diagonals and six couplings.  Vectors interleaved [n][4] = (p, u, v, w).
 // Solver: FP64 BiCGStab, right-preconditioned by a SIMPLE-type block
 // factorisation whose Schur-complement step is one FP32 V-cycle of the scalar
 // pressure hierarchy (see precond below).
@@ -39,19 +43,15 @@ struct Coupled {
     bool built = false;
     int n = 0;
     int64_t nnzb = 0;                           // off-diagonal blocks
-    // fine level (device numbering), FP64
-    std::vector<int> h_ptr, h_col;
-    DBuf<int> ptr, col, fslot_own, fslot_nbr;   // per internal face: block index in row owner / neighbour
-    DBuf<double> val, diag, rhs;                // [nnzb][16], [n][16], [n][4]
-    DBuf<double> mval, mdiag, mrhs, pval, pdiag, prhs;   // scalar momentum / pressure systems
+    DBuf<double> rhs;                           // [n][4]
+    // the blocks, FP64: momentum / pressure entries and couplings per slot
+    // (mval, pval [nv], gval [3][nv]; padding slots of gval hold 0), the
+    // diagonal blocks' scalar entries and their couplings (0, 1..3), (1..3, 0)
+    // (dval [6][n])
+    DBuf<double> mval, mdiag, mrhs, pval, pdiag, prhs, gval, dval;
     DBuf<double> x;                             // [n][4] last solution
-    // the couplings the preconditioner reads, FP32.  gc [3][nv]: per slot of
-    // the scalar pattern (the sliced ELL of the pressure and momentum
-    // matrices, entry pairs) the off-diagonal block's continuity-row u'
-    // entries (0, 1..3); its momentum rows' p' entries (1..3, 0) are the same
-    // three numbers (k_cpl_row writes both as sg n_k A w_j).  Padding slots
-    // hold 0.  dd [6][n]: the diagonal block's (0, 1..3) and (1..3, 0)
-    // entries.  im [n]: 1 / diag(M).
+    // the couplings the preconditioner reads, FP32 (gval and dval rounded:
+    // gc [3][nv], dd [6][n]) and im [n] = 1 / diag(M)
     DBuf<float> gc, dd;
     DBuf<double> im;
     DBuf<double> kv;                            // Krylov vectors
@@ -66,65 +66,51 @@ void coupled_free(Coupled* p) { delete p; }
 namespace {
 
 // ---------------------------------------------------------------- assembly --
+// Forms the couplings and the right-hand side; the scalar entries are the two
+// assembled systems' own arrays.  (Writing 16-value blocks instead took 665 us
+// on 1.05M cells, 1.0 GB of stores; the couplings alone 233 us.)
 __global__ void __launch_bounds__(TPB) k_cpl_row(
-    int nc, int nif, int nbf, const int* __restrict__ cf_sl, const int* __restrict__ cf_ell,
-    const int* __restrict__ owner, const int* __restrict__ nbr, const int* __restrict__ bpatch,
+    int nc, int nif, const int* __restrict__ cf_sl, const int* __restrict__ cf_ell, const int* __restrict__ bpatch,
     const semo_patch_bc* __restrict__ bcs, const double* __restrict__ nrm, const double* __restrict__ area,
     const double* __restrict__ wCv, const int* __restrict__ slot_own, const int* __restrict__ slot_nbr,
-    const int* __restrict__ fso, const int* __restrict__ fsn, const double* __restrict__ mval,
-    const double* __restrict__ mdiag, const double* __restrict__ pval, const double* __restrict__ pdiag,
-    const double* __restrict__ mrhs, const double* __restrict__ prhs, const double* __restrict__ U,
-    const double* __restrict__ V, const double* __restrict__ W, double* __restrict__ val, double* __restrict__ diag, double* __restrict__ rhs, int64_t nv,
+    const double* __restrict__ mdiag, const double* __restrict__ mrhs, const double* __restrict__ prhs,
+    const double* __restrict__ U, const double* __restrict__ V, const double* __restrict__ W,
+    double* __restrict__ gval, double* __restrict__ dval, double* __restrict__ rhs, int64_t nv,
     float* __restrict__ gc, float* __restrict__ dd, double* __restrict__ im) {
     int i = xcd_block() * blockDim.x + threadIdx.x;
     if (i >= nc) return;
-    double D[16];
-    for (int q = 0; q < 16; ++q) D[q] = 0.0;
+    double D[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};    // continuity row's u'_k, momentum rows' p'
     double uc[3] = {U[i], V[i], W[i]};
     CELL_FACES_BEGIN(i, cf_sl, cf_ell, f, own)
         const double* n = nrm + 3 * (size_t)f;
         double A = area[f];
         if (f < nif) {
             double wC = wCv[f];
-            // the block of this face's neighbour in row i: no other face
-            // adds to it (one face per pair of cells), so it is formed in
-            // registers and stored once, 16-byte stores
-            double B[16];
-            for (int q = 0; q < 16; ++q) B[q] = 0.0;
+            // no other face adds to this slot (one face per pair of cells)
             int slot = own ? slot_own[f] : slot_nbr[f];
-            double a = mval[slot];
-            double q = pval[slot];
-            B[0] += q;
-            for (int k = 1; k < 4; ++k) B[5 * k] += a;
             double wi = own ? wC : 1.0 - wC, wj = 1.0 - wi, sg = own ? 1.0 : -1.0;
-            for (int k = 1; k < 4; ++k) {
-                double g = sg * n[k - 1] * A;
-                D[k] += g * wi;       // continuity row, u'_k of this cell
-                B[k] += g * wj;
-                gc[(k - 1) * nv + slot] = (float)B[k];
-                D[4 * k] += g * wi;   // momentum row k, p' of this cell
-                B[4 * k] += g * wj;
+            for (int k = 0; k < 3; ++k) {
+                double g = sg * n[k] * A;
+                D[k] += g * wi;
+                D[3 + k] += g * wi;
+                double gj = g * wj;
+                gval[k * nv + slot] = gj;
+                gc[k * nv + slot] = (float)gj;
             }
-            double2* Bo = reinterpret_cast<double2*>(val + 16 * (size_t)(own ? fso[f] : fsn[f]));
-            for (int q = 0; q < 8; ++q) Bo[q] = make_double2(B[2 * q], B[2 * q + 1]);
             continue;
         }
         semo_patch_bc bc = bcs[bpatch[f - nif]];
         if (bc.p_type != SEMO_BC_FIXED_VALUE)
-            for (int k = 1; k < 4; ++k) D[4 * k] += n[k - 1] * A;
+            for (int k = 0; k < 3; ++k) D[3 + k] += n[k] * A;
         bool flux = bc.u_type == SEMO_BC_ZERO_GRADIENT ||
                     (bc.u_type == SEMO_BC_INLET_OUTLET && uc[0] * n[0] + uc[1] * n[1] + uc[2] * n[2] > 0.0);
         if (flux)
-            for (int k = 1; k < 4; ++k) D[k] += n[k - 1] * A;
+            for (int k = 0; k < 3; ++k) D[k] += n[k] * A;
     }
-    D[0] += pdiag[i];
-    for (int k = 1; k < 4; ++k) D[5 * k] += mdiag[i];
-    double2* Do = reinterpret_cast<double2*>(diag + 16 * (size_t)i);
-    for (int q = 0; q < 8; ++q) Do[q] = make_double2(D[2 * q], D[2 * q + 1]);
     size_t N = (size_t)nc;
-    for (int k = 0; k < 3; ++k) {
-        dd[k * N + i] = (float)D[1 + k];
-        dd[(3 + k) * N + i] = (float)D[4 * (1 + k)];
+    for (int k = 0; k < 6; ++k) {
+        dval[k * N + i] = D[k];
+        dd[k * N + i] = (float)D[k];
     }
     im[i] = 1.0 / mdiag[i];
     double2* Ro = reinterpret_cast<double2*>(rhs + 4 * (size_t)i);
@@ -132,28 +118,88 @@ __global__ void __launch_bounds__(TPB) k_cpl_row(
     Ro[1] = make_double2(mrhs[N + i], mrhs[2 * N + i]);
 }
 
-// ------------------------------------------------------------- block SpMV --
-// Four lanes per block row: lane q owns output component q and reads row q of
-// every block (4 contiguous values), so a quad reads each 16-value block as
-// one contiguous run; x_j (4 values) is shared by the quad.
-// OP 0: y = A x;  OP 1: y = b - A x
-template <class T, int OP>
-__global__ void __launch_bounds__(TPB) k_bsr(int n, const int* __restrict__ ptr, const int* __restrict__ col,
-                                             const T* __restrict__ val, const T* __restrict__ diag,
-                                             const T* __restrict__ x, const T* __restrict__ b, T* __restrict__ y) {
-    int gid = xcd_block() * blockDim.x + threadIdx.x;
-    int i = gid >> 2, q = gid & 3;
-    if (i >= n) return;
-    const T* d = diag + 16 * (size_t)i + 4 * q;
-    const T* xi = x + 4 * (size_t)i;
-    T s = d[0] * xi[0] + d[1] * xi[1] + d[2] * xi[2] + d[3] * xi[3];
-    for (int e = ptr[i]; e < ptr[i + 1]; ++e) {
-        const T* a = val + 16 * (size_t)e + 4 * q;
-        const T* xj = x + 4 * (size_t)col[e];
-        s += a[0] * xj[0] + a[1] * xj[1] + a[2] * xj[2] + a[3] * xj[3];
+// the columns of entries e, e + 1 (e even) of the scalar pattern, from
+// int16 offsets column - row or from int32 columns
+template <bool NARROW>
+__device__ inline int2 pat_cols(const int* __restrict__ col, const int16_t* __restrict__ dcol, int e, int row) {
+    if constexpr (NARROW) {
+        int w = *reinterpret_cast<const int*>(dcol + e);
+        return make_int2(row + (int)(int16_t)(w & 0xffff), row + (w >> 16));
+    } else {
+        return *reinterpret_cast<const int2*>(col + e);
     }
-    size_t o = 4 * (size_t)i + q;
-    y[o] = OP == 0 ? s : b[o] - s;
+}
+
+// ------------------------------------------------------------- block product --
+// the block matrix as the product reads it
+struct BlkMat {
+    const int* __restrict__ sl_ptr;
+    const int* __restrict__ col;
+    const int16_t* __restrict__ dcol;
+    const double* __restrict__ m;       // momentum entries per slot
+    const double* __restrict__ p;       // pressure entries per slot
+    const double* __restrict__ g;       // couplings [3][nv]
+    const double* __restrict__ md;      // scalar diagonals
+    const double* __restrict__ pd;
+    const double* __restrict__ d;       // the diagonal blocks' couplings [6][n]
+    int64_t nv;
+};
+
+// OP 0: y = A x;  OP 1: y = b - A x.  One lane per block row: a wavefront's
+// load of each of the five value arrays is one contiguous 1 KB run, a
+// neighbour costs one 32-byte gather.  Bound by HBM: 40 B per off-diagonal
+// block and 128 B per row with the vectors, against 132 B and 192 B when full
+// 16-value blocks were read (four lanes per row, block CSR): 1.05M cells
+// 200 -> 79 us a product, 5.0 TB/s.  The omitted products are by exact zeros, and the
+// rest are added in the same order.
+template <int OP, bool NARROW>
+__global__ void __launch_bounds__(TPB) k_blk(int n, BlkMat a, const double* __restrict__ x,
+                                             const double* __restrict__ b, double* __restrict__ y) {
+    int row = xcd_block() * TPB + threadIdx.x;
+    int s = row >> 6, lane = row & (SL - 1);
+    if (s >= (n + SL - 1) / SL) return;
+    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+    if (row < n) {
+        size_t N = (size_t)n;
+        double2 xa = *reinterpret_cast<const double2*>(x + 4 * (size_t)row);
+        double2 xb = *reinterpret_cast<const double2*>(x + 4 * (size_t)row + 2);
+        double dm = a.md[row];
+        s0 = a.pd[row] * xa.x + a.d[row] * xa.y + a.d[N + row] * xb.x + a.d[2 * N + row] * xb.y;
+        s1 = a.d[3 * N + row] * xa.x + dm * xa.y;
+        s2 = a.d[4 * N + row] * xa.x + dm * xb.x;
+        s3 = a.d[5 * N + row] * xa.x + dm * xb.y;
+    }
+    int end = a.sl_ptr[s + 1];
+    const double* g1 = a.g + a.nv;
+    const double* g2 = g1 + a.nv;
+    for (int e = a.sl_ptr[s] + 2 * lane; e < end; e += 2 * SL) {
+        int2 j = pat_cols<NARROW>(a.col, a.dcol, e, row);
+        double2 q = *reinterpret_cast<const double2*>(a.p + e);
+        double2 m = *reinterpret_cast<const double2*>(a.m + e);
+        double2 c0 = *reinterpret_cast<const double2*>(a.g + e);
+        double2 c1 = *reinterpret_cast<const double2*>(g1 + e);
+        double2 c2 = *reinterpret_cast<const double2*>(g2 + e);
+        double2 u0 = *reinterpret_cast<const double2*>(x + 4 * (size_t)j.x);
+        double2 u1 = *reinterpret_cast<const double2*>(x + 4 * (size_t)j.x + 2);
+        double2 v0 = *reinterpret_cast<const double2*>(x + 4 * (size_t)j.y);
+        double2 v1 = *reinterpret_cast<const double2*>(x + 4 * (size_t)j.y + 2);
+        s0 += q.x * u0.x + c0.x * u0.y + c1.x * u1.x + c2.x * u1.y;
+        s1 += c0.x * u0.x + m.x * u0.y;
+        s2 += c1.x * u0.x + m.x * u1.x;
+        s3 += c2.x * u0.x + m.x * u1.y;
+        s0 += q.y * v0.x + c0.y * v0.y + c1.y * v1.x + c2.y * v1.y;
+        s1 += c0.y * v0.x + m.y * v0.y;
+        s2 += c1.y * v0.x + m.y * v1.x;
+        s3 += c2.y * v0.x + m.y * v1.y;
+    }
+    if (row >= n) return;
+    if constexpr (OP == 1) {
+        double2 ba = *reinterpret_cast<const double2*>(b + 4 * (size_t)row);
+        double2 bb = *reinterpret_cast<const double2*>(b + 4 * (size_t)row + 2);
+        s0 = ba.x - s0; s1 = ba.y - s1; s2 = bb.x - s2; s3 = bb.y - s3;
+    }
+    *reinterpret_cast<double2*>(y + 4 * (size_t)row) = make_double2(s0, s1);
+    *reinterpret_cast<double2*>(y + 4 * (size_t)row + 2) = make_double2(s2, s3);
 }
 
 // ------------------------------------------ SIMPLE-type block preconditioner --
@@ -171,18 +217,6 @@ __global__ void __launch_bounds__(TPB) k_bsr(int n, const int* __restrict__ ptr,
 // are one 8-byte load per lane per pair, a wavefront's load one contiguous
 // run); u* is formed where it is read (r_u 1/diag(M), the same product the
 // correction forms), so no pass writes it.
-
-// the columns of entries e, e + 1 (e even) of the scalar pattern, from
-// int16 offsets column - row or from int32 columns
-template <bool NARROW>
-__device__ inline int2 pat_cols(const int* __restrict__ col, const int16_t* __restrict__ dcol, int e, int row) {
-    if constexpr (NARROW) {
-        int w = *reinterpret_cast<const int*>(dcol + e);
-        return make_int2(row + (int)(int16_t)(w & 0xffff), row + (w >> 16));
-    } else {
-        return *reinterpret_cast<const int2*>(col + e);
-    }
-}
 
 constexpr int PC_PAIRS = 2;   // entry pairs per trip: their loads, then their gathers
 
@@ -465,44 +499,35 @@ void precond(semo_ctx* c, Coupled& C, const double* r, double* z) {
                     dim3(TPB), n, A.sl_ptr.p, A.col.p, A.dcol.p, C.gc.p, nv, C.dd.p, r, C.im.p, C.zp.p, z);
 }
 
+BlkMat blk_mat(semo_ctx* c, const Coupled& C) {
+    const DevSell<double>& A = c->Amat;
+    return BlkMat{A.sl_ptr.p, A.col.p, A.dcol.p, C.mval.p, C.pval.p, C.gval.p, C.mdiag.p, C.pdiag.p, C.dval.p,
+                  (int64_t)c->pat.col.size()};
+}
+// y = A x (OP 0) or y = b - A x (OP 1)
+template <int OP>
+void blk_product(semo_ctx* c, Coupled& C, const double* x, const double* b, double* y, const char* tag) {
+    bool narrow = c->Amat.dcol.p != nullptr;
+    double bytes = (40.0 + (narrow ? 2.0 : 4.0)) * C.nnzb + (64.0 + 64.0 + (OP ? 32.0 : 0.0)) * C.n;
+    dim3 g(nblk((long)c->pat.nslices * SL)), t(TPB);
+    BlkMat a = blk_mat(c, C);
+    if (narrow) SEMO_LAUNCH(c, tag, bytes, (k_blk<OP, true>), g, t, C.n, a, x, b, y);
+    else SEMO_LAUNCH(c, tag, bytes, (k_blk<OP, false>), g, t, C.n, a, x, b, y);
+}
 void spmv64(semo_ctx* c, Coupled& C, const double* x, double* y) {
-    SEMO_LAUNCH(c, "cpl_bsr_spmv", 4.0 * C.n + 132.0 * C.nnzb + 128.0 * C.n + 64.0 * C.n, (k_bsr<double, 0>),
-                dim3(nblk(4 * (long)C.n)), dim3(TPB), C.n, C.ptr.p, C.col.p, C.val.p, C.diag.p, x,
-                (const double*)nullptr, y);
+    blk_product<0>(c, C, x, nullptr, y, "cpl_blk_spmv");
 }
 
-// fine pattern and face -> block maps (once per mesh)
+// work arrays (once per mesh)
 void coupled_setup(semo_ctx* c, Coupled& C) {
-    int n = c->nc, nif = c->nif;
+    int n = c->nc;
     C.n = n;
-    std::vector<int> ptr(n + 1, 0);
-    for (int f = 0; f < nif; ++f) { ptr[c->h_owner[f] + 1]++; ptr[c->h_nbr[f] + 1]++; }
-    for (int i = 0; i < n; ++i) ptr[i + 1] += ptr[i];
-    std::vector<std::pair<int, int>> ent(ptr[n]);
-    {
-        std::vector<int> pos(ptr.begin(), ptr.end() - 1);
-        for (int f = 0; f < nif; ++f) {
-            ent[pos[c->h_owner[f]]++] = {c->h_nbr[f], f};
-            ent[pos[c->h_nbr[f]]++] = {c->h_owner[f], ~f};
-        }
-    }
-    std::vector<int> col(ptr[n]), fso(std::max(nif, 1)), fsn(std::max(nif, 1));
-    for (int i = 0; i < n; ++i) {
-        std::sort(ent.begin() + ptr[i], ent.begin() + ptr[i + 1]);
-        for (int k = ptr[i]; k < ptr[i + 1]; ++k) {
-            col[k] = ent[k].first;
-            int f = ent[k].second;
-            if (f >= 0) fso[f] = k; else fsn[~f] = k;
-        }
-    }
-    C.h_ptr = ptr; C.h_col = col;
+    C.nnzb = 2 * (int64_t)c->nif;
     hipStream_t s = c->stream;
-    C.ptr.upload(ptr, s); C.col.upload(col, s); C.fslot_own.upload(fso, s); C.fslot_nbr.upload(fsn, s);
-    size_t nnzb = col.size();
-    C.val.alloc(16 * std::max<size_t>(nnzb, 1)); C.diag.alloc(16 * (size_t)n); C.rhs.alloc(4 * (size_t)n);
+    size_t nv = std::max<size_t>(c->pat.col.size(), 1);
+    C.rhs.alloc(4 * (size_t)n);
     C.x.alloc(4 * (size_t)n); C.x.zero(s);
-    size_t nv = c->pat.col.size();
-    for (DBuf<double>* b : {&C.mval, &C.pval}) b->alloc(std::max<size_t>(nv, 1));
+    for (DBuf<double>* b : {&C.mval, &C.pval}) b->alloc(nv);
     for (DBuf<double>* b : {&C.mdiag, &C.pdiag, &C.prhs}) b->alloc(n);
     C.mrhs.alloc(3 * (size_t)n);
     C.kv.alloc(8 * 4 * (size_t)n);
@@ -510,11 +535,9 @@ void coupled_setup(semo_ctx* c, Coupled& C) {
     C.part.alloc(2 * 2048 + 64);
     C.red.alloc(2 * (size_t)nblk(4 * (long)n) + 64);
     C.sc.alloc(16);
-
-    C.nnzb = (int64_t)nnzb;
-    C.gc.alloc(3 * std::max<size_t>(nv, 1));
-    C.gc.zero(s);                               // padding slots stay 0
-    C.dd.alloc(6 * (size_t)n);
+    C.gval.alloc(3 * nv); C.gval.zero(s);       // padding slots stay 0
+    C.gc.alloc(3 * nv); C.gc.zero(s);
+    C.dval.alloc(6 * (size_t)n); C.dd.alloc(6 * (size_t)n);
     C.im.alloc(n);
     SEMO_HIP(hipStreamSynchronize(s));
     C.built = true;
@@ -545,12 +568,10 @@ void assemble_coupled(semo_ctx* c) {
     copy_d(c, C.mdiag.p, c->Amat.diag.p, n);
     copy_d(c, C.mrhs.p, c->Bvec.p, 3 * (size_t)n);
     SEMO_LAUNCH(c, "cpl_assemble",
-                cell_faces_bytes(c, 56.0) + 32.0 * c->nif + 128.0 * ((double)n + C.nnzb) + 104.0 * n +
-                    24.0 * c->nif + 32.0 * n,
-                k_cpl_row, dim3(nblk(n)), dim3(TPB), n, c->nif, c->nbf, c->d_cf_sl.p, c->d_cf_ell.p, c->d_owner.p,
-                c->d_nbr.p, c->d_bpatch.p, c->d_bcs.p, c->f_nrm.p, c->f_area.p, c->f_wC.p, c->d_slot_own.p,
-                c->d_slot_nbr.p, C.fslot_own.p, C.fslot_nbr.p, C.mval.p, C.mdiag.p, C.pval.p, C.pdiag.p, C.mrhs.p,
-                C.prhs.p, c->U.p, c->V.p, c->W.p, C.val.p, C.diag.p, C.rhs.p, (int64_t)nv, C.gc.p, C.dd.p,
+                cell_faces_bytes(c, 48.0) + (8.0 + 72.0) * c->nif + (24.0 + 8.0 + 32.0 + 72.0 + 8.0 + 32.0) * n,
+                k_cpl_row, dim3(nblk(n)), dim3(TPB), n, c->nif, c->d_cf_sl.p, c->d_cf_ell.p, c->d_bpatch.p,
+                c->d_bcs.p, c->f_nrm.p, c->f_area.p, c->f_wC.p, c->d_slot_own.p, c->d_slot_nbr.p, C.mdiag.p,
+                C.mrhs.p, C.prhs.p, c->U.p, c->V.p, c->W.p, C.gval.p, C.dval.p, C.rhs.p, (int64_t)nv, C.gc.p, C.dd.p,
                 C.im.p);
     c->last_eq = 3;
 }
@@ -611,9 +632,7 @@ void coupled_solve(semo_ctx* c, const double* b, double* x, semo_solve_stats* st
             if (cc.done(it)) break;
             if (cc.r1 < 0.25 * best) { best = cc.r1; since = 0; }       // squared residuals
             else if (++since >= RESTART_AFTER) {
-                SEMO_LAUNCH(c, "cpl_bsr_resid", 4.0 * C.n + 132.0 * C.nnzb + 128.0 * C.n + 64.0 * C.n + 32.0 * C.n,
-                            (k_bsr<double, 1>), dim3(nblk(4 * (long)C.n)), dim3(TPB), C.n, C.ptr.p, C.col.p, C.val.p,
-                            C.diag.p, x, b, r);
+                blk_product<1>(c, C, x, b, r, "cpl_blk_resid");
                 SEMO_LAUNCH(c, "cpl_bicg_restart", 32.0 * N, k_cb_restart, dim3(nbv), dim3(TPB), N, r, rh, p, v,
                             C.red.p);
                 fin(nbv, F_RESTART);
@@ -623,9 +642,7 @@ void coupled_solve(semo_ctx* c, const double* b, double* x, semo_solve_stats* st
         }
         it = std::min(it, c->sp.maxit_u);
         // true residual
-        SEMO_LAUNCH(c, "cpl_bsr_resid", 4.0 * C.n + 132.0 * C.nnzb + 128.0 * C.n + 64.0 * C.n + 32.0 * C.n,
-                    (k_bsr<double, 1>), dim3(nblk(4 * (long)C.n)), dim3(TPB), C.n, C.ptr.p, C.col.p, C.val.p,
-                    C.diag.p, x, b, r);
+        blk_product<1>(c, C, x, b, r, "cpl_blk_resid");
         double rr = dot2(c, C, N, r, r, nullptr, nullptr).x;
         C.last_relres = std::sqrt(rr) / nb;
     } else {
@@ -665,19 +682,37 @@ void coupled_export(semo_ctx* c, std::vector<int>& rows, std::vector<int>& cols,
     SEMO_CHECK(c->cpl && c->cpl->built, SEMO_ESTATE, "no coupled system assembled");
     Coupled& C = *c->cpl;
     int n = C.n;
-    size_t nnzb = C.h_col.size();
-    std::vector<double> d(16 * (size_t)n), v(16 * nnzb);
-    rhs.resize(4 * (size_t)n);
-    C.diag.download(d.data(), d.size(), c->stream);
-    if (nnzb) C.val.download(v.data(), v.size(), c->stream);
+    size_t nv = c->pat.col.size(), N = (size_t)n;
+    std::vector<double> mv(nv), pv(nv), gv(3 * nv), dv(6 * N), md(N), pd(N);
+    rhs.resize(4 * N);
+    C.mval.download(mv.data(), nv, c->stream); C.pval.download(pv.data(), nv, c->stream);
+    C.gval.download(gv.data(), 3 * nv, c->stream); C.dval.download(dv.data(), 6 * N, c->stream);
+    C.mdiag.download(md.data(), N, c->stream); C.pdiag.download(pd.data(), N, c->stream);
     C.rhs.download(rhs.data(), rhs.size(), c->stream);
     SEMO_HIP(hipStreamSynchronize(c->stream));
-    rows.clear(); cols.clear(); blocks.clear();
-    for (int i = 0; i < n; ++i) { rows.push_back(i); cols.push_back(i); }
-    blocks = d;
-    for (int i = 0; i < n; ++i)
-        for (int k = C.h_ptr[i]; k < C.h_ptr[i + 1]; ++k) { rows.push_back(i); cols.push_back(C.h_col[k]); }
-    blocks.insert(blocks.end(), v.begin(), v.end());
+    rows.clear(); cols.clear();
+    size_t nb = N + (size_t)C.nnzb;
+    rows.reserve(nb); cols.reserve(nb);
+    blocks.assign(16 * nb, 0.0);
+    auto block = [&](int i, int j, double p, double m) {
+        double* B = blocks.data() + 16 * rows.size();
+        rows.push_back(i); cols.push_back(j);
+        B[0] = p; B[5] = B[10] = B[15] = m;
+        return B;
+    };
+    for (int i = 0; i < n; ++i) {
+        double* B = block(i, i, pd[i], md[i]);
+        for (int k = 0; k < 3; ++k) { B[1 + k] = dv[k * N + i]; B[4 * (1 + k)] = dv[(3 + k) * N + i]; }
+    }
+    for (int i = 0; i < n; ++i) {
+        int base = c->pat.sl_ptr[i / SL], w = (c->pat.sl_ptr[i / SL + 1] - base) / SL;
+        for (int q = 0; q < w; ++q) {
+            int e = sell_pos(base, q, i % SL);
+            if (c->pat.col[e] == i) break;                  // padding follows a row's last entry
+            double* B = block(i, c->pat.col[e], pv[e], mv[e]);
+            for (int k = 0; k < 3; ++k) B[1 + k] = B[4 * (1 + k)] = gv[k * nv + e];
+        }
+    }
 }
 
 }  // namespace semo

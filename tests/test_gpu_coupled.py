@@ -16,7 +16,7 @@ import numpy as np
 import pytest
 import scipy.sparse as sp
 
-from semo_mesh_amd.cases import cavity_case
+from semo_mesh_amd.cases import BC_FIXED_VALUE, PatchBC, cavity_case
 from semo_mesh_amd.mesh import cavity_mesh
 
 pytestmark = pytest.mark.gpu
@@ -108,6 +108,33 @@ def test_bsr4_spmv_equals_expanded_csr(system):
     x = np.random.default_rng(3).standard_normal((4, mesh.n_cells))
     y = g.coupled_spmv(x)
     ref = K @ x.ravel()
+    assert np.linalg.norm(y.ravel() - ref) <= 1e-14 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("cells, size, reorder", [
+    ("hex", (3, 2, 1), True), ("hex", (5, 3, 7), True), ("hex", (13, 5, 1), False), ("tet", (3, 2, 2), True),
+    ("tet", (5, 4, 3), False), ("hex", (190, 182, 2), False)])
+def test_block_product_edges(cells, size, reorder):
+    """Last slices of every kind (1 to 64 rows), rows of one to six
+    neighbours, and columns too far for 16-bit offsets (190 x 182 cells a
+    layer, not renumbered).  16 products and sums per row and neighbour:
+    1e-14 as above."""
+    from semo_mesh_amd.mesh import hex_mesh, tet_mesh
+    mesh = (hex_mesh if cells == "hex" else tet_mesh)(*size, jitter=0.1, seed=23)
+    case = _case()
+    if cells == "tet":
+        case.bcs = {k: v for k, v in case.bcs.items() if k in mesh.patch_names}
+        case.bcs["zmin"] = PatchBC(p_type=BC_FIXED_VALUE)
+    g = _gpu(mesh, case, reorder=reorder, tol=1e-8)
+    g.incompressiblePressureBased(1)            # a non-trivial state
+    g.assemble("coupled")
+    rb, cb, blk, _ = g.coupled_matrix()
+    K = _expand(mesh, rb, cb, blk)
+    x = np.random.default_rng(3).standard_normal((4, mesh.n_cells))
+    y = g.coupled_spmv(x)
+    g.close()
+    ref = K @ x.ravel()
+    assert len(rb) == mesh.n_cells + 2 * mesh.n_internal_faces
     assert np.linalg.norm(y.ravel() - ref) <= 1e-14 * np.linalg.norm(ref)
 
 
