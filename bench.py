@@ -414,9 +414,8 @@ def lusgs_leg(n=128, nsp=2, reps=5, cpu_n=48):
                                    "GBs": round(v["bytes"] / (v["ms"] * 1e-3) / 1e9, 1) if v["ms"] > 0 else None}
                                for k, v in prof.items()}}
             if key == "lusgs":
-                leg["sweep_levels"] = prof.get("lusgs_sweep", {}).get("count")
-                leg["note"] = ("first call levels the sweeps on the host (once per mesh); the level "
-                               "kernels are latency-bound: one launch per level")
+                leg["note"] = ("first call levels the sweeps on the host (once per mesh); a sweep is one launch, "
+                               "bound by its chain of levels")
             out[key] = leg
         hout = np.empty_like(r0)
         assert hip.hipMemcpy(hout.ctypes.data_as(C.c_void_p), dr, nbytes, 2) == 0

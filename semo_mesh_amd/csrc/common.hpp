@@ -255,17 +255,17 @@ struct semo_ctx {
     semo::DBuf<double> les_g;
     int les_model = 0;
     semo::DBuf<double> muT, kSGS, les_zero;
-    // density-based LU-SGS (linearSolver.cpp): per sweep (forward, backward)
-    // the level offsets and, in level order, one slot record per cell (the
-    // cell and the first four (neighbour, face) pairs it reads, 3 x int4),
-    // the further pairs in an overflow list; the inverted diagonal blocks
-    // [n][N*N]
+    // density-based LU-SGS (linearSolver.cpp): per sweep (forward, backward),
+    // in level order, one slot record per cell (the cell and the first four
+    // (neighbour, face) pairs it reads, 3 x int4; a level filled up to a
+    // multiple of 16), the further pairs in an overflow list; the inverted
+    // diagonal blocks; the sweeps' results [2][n][N], tickets and error word
     bool reordered = false;
     bool ls_ready = false;
-    std::vector<int> ls_lev_ptr[2];
     semo::DBuf<int4> ls_slots[2];
     semo::DBuf<int2> ls_ovf[2];
-    semo::DBuf<double> ls_dinv;
+    semo::DBuf<double> ls_dinv, ls_out;
+    semo::DBuf<int> ls_ctl;
     std::vector<double> h_ufix;     // as set, in the caller's numbering
     // per-face values of the volume-fraction "function" boundary [nbf]
     // (device face order), empty until semo_set_vf_function_points
@@ -469,7 +469,6 @@ void update_values_device(semo_ctx* c, int nsp, const double* urf, const double*
                           double* cells, double* un);
 void compress_vf_device(semo_ctx* c, double cfl, int iters, double* vf, const double* faceR_b, double* residuals);
 void linsol_device(semo_ctx* c, int method, int nsp, double time_step, const double* st, double* res);
-int lusgs_levels(semo_ctx* c, int dir);
 void flux_device(semo_ctx* c, int scheme, int n, int nsp, const double* L, const double* R, const double* nrm,
                  const double* par, double* flux);
 void les_device(semo_ctx* c, int model, const double* U, const double* V, const double* W, const double* Rho,

@@ -15,10 +15,12 @@
 // residuals of its neighbours that come before it (forward) or after it
 // (backward).  Their dependency graph is levelled on the host once per mesh:
 // a cell's forward level is one more than the largest level of its earlier
-// neighbours, so the cells of one level depend only on lower levels and are
-// updated by one launch, in any order, with the sequential sweep's result.
+// neighbours, so the cells of one level depend only on lower levels.  A sweep
+// is one launch whose wavefronts take up to 16 cells of one level at a time,
+// in level order, and wait for the neighbours' values themselves
+// (k_lusgs_sweep), with the sequential sweep's result.
 // The diagonal block (the same in both sweeps) is formed and inverted once,
-// fully parallel, and stored [n][N*N].
+// fully parallel, and stored (dinv_at).
 //
 // Cell state records, [n][12 + 3 nsp] in device order: P, U, V, W, T, rho,
 // C, Ht, dRhoDP, dHtDP, dRhoDT, dHtDT, Ur, dtPseudo, Y_0..Y_{nsp-1},
@@ -86,10 +88,12 @@ __device__ inline void construct(const double (&s)[LS<NSP>::K], double (&Pm)[4 +
 
 // getNumericalFluxJacobianUpwind (linearSolver.cpp:394-640), side "R" when
 // RIGHT, else "L": 0.5 dF/dQ of that side's state +/- 0.5 of the Roe-type
-// dissipation of the face averages (none in the species rows).
-template <int NSP, bool RIGHT>
+// dissipation of the face averages (none in the species rows).  The rows are
+// handed to `use(i, row)` one after the other, so that a caller that consumes
+// them as they come holds one row and not the matrix.
+template <int NSP, bool RIGHT, class RowF>
 __device__ inline void jacobian(const double (&L)[LS<NSP>::K], const double (&R)[LS<NSP>::K], const double n[3],
-                                double (&J)[4 + NSP][4 + NSP]) {
+                                RowF use) {
     constexpr int N = 4 + NSP;
     const double UnL = L[sU] * n[0] + L[sV] * n[1] + L[sW] * n[2];
     const double UnR = R[sU] * n[0] + R[sV] * n[1] + R[sW] * n[2];
@@ -113,74 +117,72 @@ __device__ inline void jacobian(const double (&L)[LS<NSP>::K], const double (&R)
         DRDYLR[a] = L[sY0 + NSP + a] * fgL + R[sY0 + NSP + a] * fgR;
         DHDYLR[a] = L[sY0 + 2 * NSP - 1 + a] * fgL + R[sY0 + 2 * NSP - 1 + a] * fgR;
     }
-    // the convective part, fluxLRdot
-    double F[N][N];
-#pragma unroll
-    for (int i = 0; i < N; ++i)
-#pragma unroll
-        for (int j = 0; j < N; ++j) F[i][j] = 0.0;
-    F[0][0] = DRDPLR * UnLR;
-#pragma unroll
-    for (int r = 0; r < 3; ++r) F[1 + r][0] = DRDPLR * UnLR * vel[r] + n[r];
-    F[4][0] = DRDPLR * UnLR * HtLR + RhoLR * UnLR * DHDPLR;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        F[0][1 + d] = RhoLR * n[d];
-#pragma unroll
-        for (int r = 0; r < 3; ++r)
-            F[1 + r][1 + d] = r == d ? RhoLR * n[d] * vel[r] + RhoLR * UnLR : RhoLR * n[d] * vel[r];
-        F[4][1 + d] = RhoLR * n[d] * HtLR + RhoLR * UnLR * vel[d];
-    }
-    F[0][4] = DRDTLR * UnLR;
-#pragma unroll
-    for (int r = 0; r < 3; ++r) F[1 + r][4] = DRDTLR * UnLR * vel[r];
-    F[4][4] = DRDTLR * UnLR * HtLR + RhoLR * UnLR * DHDTLR;
-#pragma unroll
-    for (int a = 0; a < NSP - 1; ++a) {
-        const int q = 5 + a;
-        F[q][0] = DRDPLR * YLR[a] * UnLR;
-#pragma unroll
-        for (int d = 0; d < 3; ++d) F[q][1 + d] = RhoLR * YLR[a] * n[d];
-        F[q][4] = DRDTLR * YLR[a] * UnLR;
-#pragma unroll
-        for (int b = 0; b < NSP - 1; ++b) F[q][5 + b] = DRDYLR[b] * YLR[a] * UnLR;
-        F[q][q] += RhoLR * UnLR;
-        F[0][q] = DRDYLR[a] * UnLR;
-#pragma unroll
-        for (int r = 0; r < 3; ++r) F[1 + r][q] = DRDYLR[a] * UnLR * vel[r];
-        F[4][q] = DRDYLR[a] * UnLR * HtLR + RhoLR * UnLR * DHDYLR[a];
-    }
-    // the dissipation, dissimat (5 x 5)
     const double dissUp = (Chat - fabs(Unhat)) / Rhohat / Chat / Chat;
     const double dissUu = Unhat / Chat;
     const double dissPp = Unhat / Chat;
     const double dissPu = (Chat - fabs(Unhat)) * Rhohat;
     const double AD = fabs(Unhat);
-    double D[5][5];
-    D[0][0] = AD * DRDPLR + dissUp * Rhohat;
 #pragma unroll
-    for (int r = 0; r < 3; ++r) D[1 + r][0] = AD * DRDPLR * vel[r] + dissUp * Rhohat * hat[r] + dissPp * n[r];
-    D[4][0] = AD * (DRDPLR * HtLR + RhoLR * DHDPLR - 1.0) + dissUp * Rhohat * Hthat + dissPp * Unhat;
+    for (int i = 0; i < N; ++i) {
+        // row i of the convective part (fluxLRdot) and of the dissipation
+        // (dissimat, 5 x 5)
+        double F[N], D[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+        if (i == 0) {
+            F[0] = DRDPLR * UnLR;
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        D[0][1 + c] = dissUu * n[c] * Rhohat;
+            for (int d = 0; d < 3; ++d) F[1 + d] = RhoLR * n[d];
+            F[4] = DRDTLR * UnLR;
 #pragma unroll
-        for (int r = 0; r < 3; ++r)
-            D[1 + r][1 + c] = r == c ? AD * RhoLR + dissUu * n[c] * Rhohat * hat[r] + dissPu * n[c] * n[r]
-                                     : dissUu * n[c] * Rhohat * hat[r] + dissPu * n[c] * n[r];
-        D[4][1 + c] = AD * RhoLR * vel[c] + dissUu * n[c] * Rhohat * Hthat + dissPu * n[c] * Unhat;
-    }
-    D[0][4] = AD * DRDTLR;
+            for (int a = 0; a < NSP - 1; ++a) F[5 + a] = DRDYLR[a] * UnLR;
+            D[0] = AD * DRDPLR + dissUp * Rhohat;
 #pragma unroll
-    for (int r = 0; r < 3; ++r) D[1 + r][4] = AD * DRDTLR * vel[r];
-    D[4][4] = AD * (DRDTLR * HtLR + RhoLR * DHDTLR);
+            for (int c = 0; c < 3; ++c) D[1 + c] = dissUu * n[c] * Rhohat;
+            D[4] = AD * DRDTLR;
+        } else if (i < 4) {
+            const int r = i - 1;
+            F[0] = DRDPLR * UnLR * vel[r] + n[r];
 #pragma unroll
-    for (int i = 0; i < N; ++i)
+            for (int d = 0; d < 3; ++d)
+                F[1 + d] = r == d ? RhoLR * n[d] * vel[r] + RhoLR * UnLR : RhoLR * n[d] * vel[r];
+            F[4] = DRDTLR * UnLR * vel[r];
+#pragma unroll
+            for (int a = 0; a < NSP - 1; ++a) F[5 + a] = DRDYLR[a] * UnLR * vel[r];
+            D[0] = AD * DRDPLR * vel[r] + dissUp * Rhohat * hat[r] + dissPp * n[r];
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+                D[1 + c] = r == c ? AD * RhoLR + dissUu * n[c] * Rhohat * hat[r] + dissPu * n[c] * n[r]
+                                  : dissUu * n[c] * Rhohat * hat[r] + dissPu * n[c] * n[r];
+            D[4] = AD * DRDTLR * vel[r];
+        } else if (i == 4) {
+            F[0] = DRDPLR * UnLR * HtLR + RhoLR * UnLR * DHDPLR;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) F[1 + d] = RhoLR * n[d] * HtLR + RhoLR * UnLR * vel[d];
+            F[4] = DRDTLR * UnLR * HtLR + RhoLR * UnLR * DHDTLR;
+#pragma unroll
+            for (int a = 0; a < NSP - 1; ++a) F[5 + a] = DRDYLR[a] * UnLR * HtLR + RhoLR * UnLR * DHDYLR[a];
+            D[0] = AD * (DRDPLR * HtLR + RhoLR * DHDPLR - 1.0) + dissUp * Rhohat * Hthat + dissPp * Unhat;
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+                D[1 + c] = AD * RhoLR * vel[c] + dissUu * n[c] * Rhohat * Hthat + dissPu * n[c] * Unhat;
+            D[4] = AD * (DRDTLR * HtLR + RhoLR * DHDTLR);
+        } else {
+            const int a = i - 5;
+            F[0] = DRDPLR * YLR[a] * UnLR;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) F[1 + d] = RhoLR * YLR[a] * n[d];
+            F[4] = DRDTLR * YLR[a] * UnLR;
+#pragma unroll
+            for (int b = 0; b < NSP - 1; ++b) F[5 + b] = DRDYLR[b] * YLR[a] * UnLR;
+            F[i] += RhoLR * UnLR;
+        }
+        double J[N];
 #pragma unroll
         for (int j = 0; j < N; ++j) {
-            const double d = (i < 5 && j < 5) ? D[i][j] : 0.0;
-            J[i][j] = RIGHT ? 0.5 * F[i][j] - 0.5 * d : 0.5 * F[i][j] + 0.5 * d;
+            const double d = (i < 5 && j < 5) ? D[j < 5 ? j : 0] : 0.0;
+            J[j] = RIGHT ? 0.5 * F[j] - 0.5 * d : 0.5 * F[j] + 0.5 * d;
         }
+        use(i, J);
+    }
 }
 
 // GaussSeidelSOR (math.cpp:141-200), in place: A's upper triangle becomes U,
@@ -261,8 +263,19 @@ __device__ inline void face_normal(const double* __restrict__ nrm, int f, bool o
     for (int a = 0; a < 3; ++a) n[a] = own_is_owner ? nrm[3 * (size_t)f + a] : -nrm[3 * (size_t)f + a];
 }
 
+// place of entry 0 of cell i's inverted diagonal block; entry e lies 64 e
+// further: 64 cells together, entry by entry, so that a wavefront's stores of
+// one entry are one run and so are a sweep unit's loads of it (cells of one
+// level are mostly consecutive)
+template <int N>
+__device__ inline size_t dinv_at(int i) { return (size_t)(i >> 6) * (64 * N * N) + (i & 63); }
+
 // LU-SGS diagonal blocks: P + 1.5 (dtau / dt) T + sum over the cell's faces
-// (ascending) of dtau / V * J_L * area, inverted, stored [n][N*N].
+// (ascending) of dtau / V * J_L * area, inverted.  FP64 arithmetic and the
+// 144-byte records of seven cells a thread bound it: 128^3, two species,
+// 770 -> 550 us once each Jacobian row was added as it was formed (212
+// registers, two wavefronts per SIMD, against 310 and one) and the blocks
+// were stored in runs.
 template <int NSP>
 __global__ __launch_bounds__(TPB) void k_lusgs_diag(int n, int nif, const int* __restrict__ cf_ptr,
                                                     const int* __restrict__ cf_idx, const int* __restrict__ owner,
@@ -286,19 +299,18 @@ __global__ __launch_bounds__(TPB) void k_lusgs_diag(int n, int nif, const int* _
         const int o = owner[f];
         double nv[3];
         face_normal(nrm, f, o == i, nv);
-        double J[N][N];
-        if (f < nif) {
-            double sn[LS<NSP>::K];
-            load_rec<NSP>(st, o == i ? nbr[f] : o, sn);
-            jacobian<NSP, false>(s, sn, nv, J);
-        } else {
-            jacobian<NSP, false>(s, s, nv, J);
-        }
         const double A = area[f];
+        // row by row, each added before the next is formed
+        auto add = [&](int a, const double (&J)[N]) {
 #pragma unroll
-        for (int a = 0; a < N; ++a)
-#pragma unroll
-            for (int c = 0; c < N; ++c) DS[a][c] += rDtauPerVol * J[a][c] * A;
+            for (int c = 0; c < N; ++c) {
+                DS[a][c] += rDtauPerVol * J[c] * A;
+                asm volatile("" : "+v"(DS[a][c]));
+            }
+        };
+        double sn[LS<NSP>::K];
+        load_rec<NSP>(st, f < nif ? (o == i ? nbr[f] : o) : i, sn);
+        jacobian<NSP, false>(s, sn, nv, add);
     }
     double M[N][N];
     {
@@ -319,7 +331,7 @@ __global__ __launch_bounds__(TPB) void k_lusgs_diag(int n, int nif, const int* _
         double X[N];
         inverse_column<N>(M, k, X);
 #pragma unroll
-        for (int j = 0; j < N; ++j) dinv[(size_t)i * N * N + j * N + k] = X[j];
+        for (int j = 0; j < N; ++j) dinv[dinv_at<N>(i) + (size_t)(j * N + k) * 64] = X[j];
     }
 }
 
@@ -333,100 +345,180 @@ __device__ inline double quad_bcast(double v) {
     return __hiloint2double(hi, lo);
 }
 
-// One level of a sweep, four lanes (a quad) per cell.  Slot t of the level
-// holds its cell, and the cell's faces toward earlier (FWD) / later cells in
-// ascending face order as (neighbour, face) pairs, the face stored as ~f when
-// the cell is the face's neighbour (normal reversed): the first four in the
-// slot's 48-byte record (one load round gives a lane its cell and its pair),
-// the rest in an overflow list.  Lane l of the quad takes pairs l, l + 4, ...: its term
-// dtau / V * (J_R r_ngb) * area; the quad adds the terms in pair order (the
-// reference's sum), then forward: r <- Dinv (r - sum), backward:
-// r <- r - Dinv sum, rows l and l + 4 on lane l.  Control flow is uniform
-// within a quad, so every DPP source lane is active.
+// A value no sweep result can be: a signaling NaN, which arithmetic quiets.
+constexpr unsigned long long LS_EMPTY = 0x7FF4A5A5C3C35A5Aull;
+// polls of one neighbour before a sweep gives up (about ten seconds): never
+// reached by the argument at k_lusgs_sweep, so that a mistake in the schedule
+// ends in an error instead of a hang
+constexpr int LS_POLL_LIMIT = 1 << 23;
+
+// words of the control array: per sweep one ticket counter for each wavefront
+// of a block, 256 bytes apart, then the error word
+constexpr int LS_STEP = 64, LS_WAVES = TPB / 64, LS_ERR = 2 * LS_WAVES * LS_STEP, LS_CTL = LS_ERR + LS_STEP;
+
+__global__ __launch_bounds__(TPB) void k_lusgs_empty(size_t n, unsigned long long* __restrict__ v,
+                                                     int* __restrict__ ctl) {
+    size_t k = (size_t)blockIdx.x * TPB + threadIdx.x;
+    if (k < LS_CTL) ctl[k] = 0;
+    if (k < n) v[k] = LS_EMPTY;
+}
+
+__device__ inline double ls_load(const double* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void ls_store(double* p, double v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// One sweep, four lanes (a quad) per cell, 16 cells of one level per unit of
+// work (slots 16 u .. 16 u + 15; the last unit of a level is filled up with
+// copies of its first slot, whose results are not stored).  Slot t holds its
+// cell, and the cell's faces toward earlier (FWD) /
+// later cells in ascending face order as (neighbour, face) pairs, the face
+// stored as ~f when the cell is the face's neighbour (normal reversed): the
+// first four in the slot's 48-byte record (one load round gives a lane its
+// cell and its pair), the rest in an overflow list.  Lane l of the quad takes
+// pairs l, l + 4, ...: its term dtau / V * (J_R r_ngb) * area; the quad adds
+// the terms in pair order (the reference's sum), then forward: r <- Dinv (r -
+// sum), backward: r <- r - Dinv sum, rows l and l + 4 on lane l.  Control
+// flow is uniform within a quad, so every DPP source lane is active.
+//
+// A lane forms its face's Jacobian first and then polls the neighbour's
+// result in `out`, which starts as LS_EMPTY: the value is its own flag, so a
+// dependency costs one store and one load through the memory side (the XCDs'
+// L2s do not share lines), not a flag and then the data, and not a launch.
+// Units are taken in level order by tickets, unit u by the wavefronts of
+// place u mod 4 in their block (one counter would be taken at 14 ns a ticket,
+// 1.9 ms a sweep at 128^3): every block has wavefronts of all four places and
+// each holds at most its current and its next, later unit, so the lowest
+// unfinished unit is always being worked on; all it waits for is finished,
+// so every wait ends whatever else runs on the device.  A unit's cells are of
+// one level: no lane waits for another lane of its wavefront.
+// Bound by that chain: 128^3 hexes (382 levels a sweep) 2.8 us a level,
+// against 6.1 us with a launch per level (4.65 -> 2.16 ms for both sweeps).
 template <int NSP, bool FWD>
-__global__ __launch_bounds__(TPB) void k_lusgs_level(int cnt, const int4* __restrict__ slots,
+__global__ __launch_bounds__(TPB) void k_lusgs_sweep(int nunits, const int4* __restrict__ slots,
                                                      const int2* __restrict__ ovf,
                                                      const double* __restrict__ nrm, const double* __restrict__ area,
                                                      const double* __restrict__ vol, const double* __restrict__ st,
-                                                     const double* __restrict__ dinv, double* __restrict__ res) {
+                                                     const double* __restrict__ dinv, const double* __restrict__ rin,
+                                                     double* out, double* __restrict__ res, int* __restrict__ ctl) {
     constexpr int N = 4 + NSP;
     static_assert(N <= 8, "two rows per lane");
-    const int gt = (int)blockIdx.x * TPB + (int)threadIdx.x;
-    const int t = gt >> 2, l = gt & 3;
-    if (t >= cnt) return;
-    // slot record: {cell, pair count, overflow offset, -}, then pairs 0..3
-    const int4 h = slots[3 * (size_t)t];
-    const int4 qq = slots[3 * (size_t)t + 1 + (l >> 1)];
-    const int i = h.x, p1 = h.y;
-    const int2 q0 = (l & 1) ? make_int2(qq.z, qq.w) : make_int2(qq.x, qq.y);
-    const int p0 = 0;
-    double s[LS<NSP>::K];
-    load_rec<NSP>(st, i, s);
-    const double rDtauPerVol = s[sDTP] / vol[i];
-    // the cell's own residual and this lane's Dinv rows do not depend on the
-    // neighbours: loaded first, in flight during the neighbour terms
-    double ri[N], D0[N], D1[N];
-    const double* Di = dinv + (size_t)i * N * N;
-#pragma unroll
-    for (int a = 0; a < N; ++a) {
-        ri[a] = res[(size_t)i * N + a];
-        D0[a] = Di[l * N + a];
-        D1[a] = l + 4 < N ? Di[(l + 4) * N + a] : 0.0;
-    }
-    double LU[N];
-#pragma unroll
-    for (int a = 0; a < N; ++a) LU[a] = 0.0;
-    for (int base = p0; base < p1; base += 4) {
-        const int p = base + l;
-        double c[N];
-#pragma unroll
-        for (int a = 0; a < N; ++a) c[a] = 0.0;
-        if (p < p1) {
-            const int2 q = p < 4 ? q0 : ovf[h.z + p - 4];
-            const int g = q.x;
-            const bool own_is_owner = q.y >= 0;
-            const int f = own_is_owner ? q.y : ~q.y;
-            double nv[3];
-            face_normal(nrm, f, own_is_owner, nv);
-            double sn[LS<NSP>::K], J[N][N], rg[N];
-            load_rec<NSP>(st, g, sn);
-#pragma unroll
-            for (int k = 0; k < N; ++k) rg[k] = res[(size_t)g * N + k];
-            const double A = area[f];
-            jacobian<NSP, true>(s, sn, nv, J);
-#pragma unroll
-            for (int a = 0; a < N; ++a) {
-                double sig = 0.0;
-#pragma unroll
-                for (int k = 0; k < N; ++k) sig += rg[k] * J[a][k];
-                c[a] = rDtauPerVol * sig * A;
-            }
+    const int lane = (int)threadIdx.x & 63, l = lane & 3;
+    const int place = (int)threadIdx.x >> 6;
+    int* ticket = ctl + ((FWD ? 0 : LS_WAVES) + place) * LS_STEP;
+    // a unit's slot records are requested while the unit before it is worked
+    // on, its ticket one unit earlier still
+    const int4* mine = slots + 3 * (lane >> 2);
+    auto take = [&] { return lane == 0 ? atomicAdd(ticket, 1) : 0; };
+    auto unit = [&](int tk) { return __builtin_amdgcn_readfirstlane(tk) * LS_WAVES + place; };
+    int u = unit(take());
+    if (u >= nunits) return;
+    // slot record: {cell, pair count, overflow offset, to be stored}, pairs 0..3
+    int4 h = mine[48 * (size_t)u], qq = mine[48 * (size_t)u + 1 + (l >> 1)];
+    int tk = take();
+    for (;;) {
+        const int i = h.x, p1 = h.y, ovf0 = h.z, act = h.w;
+        const int2 q0 = (l & 1) ? make_int2(qq.z, qq.w) : make_int2(qq.x, qq.y);
+        u = unit(tk);
+        if (u < nunits) {
+            h = mine[48 * (size_t)u];
+            qq = mine[48 * (size_t)u + 1 + (l >> 1)];
+            tk = take();
         }
+        double s[LS<NSP>::K];
+        load_rec<NSP>(st, i, s);
+        const double rDtauPerVol = s[sDTP] / vol[i];
+        // the cell's own residual and this lane's Dinv rows do not depend on
+        // the neighbours: in flight during the neighbour terms
+        double ri[N], D0[N], D1[N];
+        const double* Di = dinv + dinv_at<N>(i);
 #pragma unroll
         for (int a = 0; a < N; ++a) {
-            const double v0 = quad_bcast<0>(c[a]), v1 = quad_bcast<1>(c[a]);
-            const double v2 = quad_bcast<2>(c[a]), v3 = quad_bcast<3>(c[a]);
-            LU[a] += v0;
-            if (base + 1 < p1) LU[a] += v1;
-            if (base + 2 < p1) LU[a] += v2;
-            if (base + 3 < p1) LU[a] += v3;
+            ri[a] = rin[(size_t)i * N + a];
+            D0[a] = Di[64 * (l * N + a)];
+            D1[a] = l + 4 < N ? Di[64 * ((l + 4) * N + a)] : 0.0;
         }
-    }
-    double b[N];
+        double LU[N];
 #pragma unroll
-    for (int a = 0; a < N; ++a) b[a] = FWD ? ri[a] - LU[a] : LU[a];
+        for (int a = 0; a < N; ++a) LU[a] = 0.0;
+        for (int base = 0; base < p1; base += 4) {
+            const int p = base + l;
+            double c[N];
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {
-        const int j = l + 4 * r;
-        if (j < N) {
-            double u = 0.0;
+            for (int a = 0; a < N; ++a) c[a] = 0.0;
+            if (p < p1) {
+                const int2 q = p < 4 ? q0 : ovf[ovf0 + p - 4];
+                const int g = q.x;
+                const bool own_is_owner = q.y >= 0;
+                const int f = own_is_owner ? q.y : ~q.y;
+                double nv[3];
+                face_normal(nrm, f, own_is_owner, nv);
+                double sn[LS<NSP>::K], J[N][N], rg[N];
+                load_rec<NSP>(st, g, sn);
+                double A = area[f];
+                // formed before the wait, not sunk behind it
+                jacobian<NSP, true>(s, sn, nv, [&](int a, const double (&Ja)[N]) {
 #pragma unroll
-            for (int k = 0; k < N; ++k) u += (r == 0 ? D0[k] : D1[k]) * b[k];
-            if (FWD) res[(size_t)i * N + j] = u;
-            else res[(size_t)i * N + j] = ri[j] - u;
+                    for (int k = 0; k < N; ++k) {
+                        J[a][k] = Ja[k];
+                        asm volatile("" : "+v"(J[a][k]));
+                    }
+                });
+                for (int poll = 0;; ++poll) {
+                    bool ready = true;
+#pragma unroll
+                    for (int k = 0; k < N; ++k) rg[k] = ls_load(out + (size_t)g * N + k);
+#pragma unroll
+                    for (int k = 0; k < N; ++k)
+                        ready = ready && (unsigned long long)__double_as_longlong(rg[k]) != LS_EMPTY;
+                    if (ready) break;
+                    if (poll >= LS_POLL_LIMIT) { ctl[LS_ERR] = 1; break; }
+                    __builtin_amdgcn_s_sleep(1);
+                }
+#pragma unroll
+                for (int a = 0; a < N; ++a) {
+                    double sig = 0.0;
+#pragma unroll
+                    for (int k = 0; k < N; ++k) sig += rg[k] * J[a][k];
+                    c[a] = rDtauPerVol * sig * A;
+                }
+            }
+#pragma unroll
+            for (int a = 0; a < N; ++a) {
+                const double v0 = quad_bcast<0>(c[a]), v1 = quad_bcast<1>(c[a]);
+                const double v2 = quad_bcast<2>(c[a]), v3 = quad_bcast<3>(c[a]);
+                LU[a] += v0;
+                if (base + 1 < p1) LU[a] += v1;
+                if (base + 2 < p1) LU[a] += v2;
+                if (base + 3 < p1) LU[a] += v3;
+            }
         }
+        double b[N];
+#pragma unroll
+        for (int a = 0; a < N; ++a) b[a] = FWD ? ri[a] - LU[a] : LU[a];
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            const int j = l + 4 * r;
+            if (j < N && act) {
+                double v = 0.0;
+#pragma unroll
+                for (int k = 0; k < N; ++k) v += (r == 0 ? D0[k] : D1[k]) * b[k];
+                if (!FWD) v = ri[j] - v;
+                ls_store(out + (size_t)i * N + j, v);
+                if (!FWD) res[(size_t)i * N + j] = v;
+            }
+        }
+        if (u >= nunits) break;
     }
 }
+
+// Blocks of a sweep: one wavefront per SIMD.  Fewer leave units of the next
+// levels unprepared; more only poll, and the polls slow the values down: with
+// 128 / 192 / 256 / 384 / 512 blocks an update took 3.48 / 3.01 / 2.91 / 3.71 /
+// 3.85 ms on 128^3 hexes, 1.06 / 1.09 / 1.14 / 1.15 / 1.14 ms on 144000 tets.
+constexpr int LS_BLOCKS = 256;
 
 // lib_RCM's order in device numbering (rank[i] = position of cell i) and
 // the forward / backward level lists of the sweeps.
@@ -464,8 +556,7 @@ void lusgs_schedule(semo_ctx* c) {
             lev[i] = l;
             nlev = std::max(nlev, l + 1);
         }
-        std::vector<int>& ptr = c->ls_lev_ptr[dir];
-        ptr.assign(nlev + 1, 0);
+        std::vector<int> ptr(nlev + 1, 0);
         for (int i = 0; i < nc; ++i) ptr[lev[i] + 1]++;
         for (int l = 0; l < nlev; ++l) ptr[l + 1] += ptr[l];
         std::vector<int> cells(nc), fill(ptr.begin(), ptr.end() - 1);
@@ -473,35 +564,48 @@ void lusgs_schedule(semo_ctx* c) {
             const int i = order[dir == 0 ? p : nc - 1 - p];
             cells[fill[lev[i]]++] = i;
         }
-        // per slot: {cell, pair count, overflow offset, 0} and its first four
-        // (neighbour, face) pairs toward earlier (later) cells, ascending
-        std::vector<int4> rec(3 * (size_t)nc);
+        // per slot: {cell, pair count, overflow offset, 1} and its first four
+        // (neighbour, face) pairs toward earlier (later) cells, ascending;
+        // a level's last unit of 16 is filled with copies of its first slot,
+        // {.., 0}
+        std::vector<int4> rec;
+        rec.reserve(3 * ((size_t)nc + 16 * (size_t)nlev));
         std::vector<int2> ovf;
-        for (int t = 0; t < nc; ++t) {
-            const int i = cells[t];
-            int np = 0;
-            int2 q[4] = {};
-            const int off = (int)ovf.size();
-            for (int k = c->h_cf_ptr[i]; k < c->h_cf_ptr[i + 1]; ++k) {
-                const int f = c->h_cf_idx[k];
-                if (f >= nif) continue;
-                const bool own = c->h_owner[f] == i;
-                const int g = own ? c->h_nbr[f] : c->h_owner[f];
-                if (!(dir == 0 ? rank[g] < rank[i] : rank[g] > rank[i])) continue;
-                const int2 pq = make_int2(g, own ? f : ~f);
-                if (np < 4) q[np] = pq;
-                else ovf.push_back(pq);
-                ++np;
+        for (int l = 0; l < nlev; ++l) {
+            for (int t = ptr[l]; t < ptr[l + 1]; ++t) {
+                const int i = cells[t];
+                int np = 0;
+                int2 q[4] = {};
+                const int off = (int)ovf.size();
+                for (int k = c->h_cf_ptr[i]; k < c->h_cf_ptr[i + 1]; ++k) {
+                    const int f = c->h_cf_idx[k];
+                    if (f >= nif) continue;
+                    const bool own = c->h_owner[f] == i;
+                    const int g = own ? c->h_nbr[f] : c->h_owner[f];
+                    if (!(dir == 0 ? rank[g] < rank[i] : rank[g] > rank[i])) continue;
+                    const int2 pq = make_int2(g, own ? f : ~f);
+                    if (np < 4) q[np] = pq;
+                    else ovf.push_back(pq);
+                    ++np;
+                }
+                rec.push_back(make_int4(i, np, off, 1));
+                rec.push_back(make_int4(q[0].x, q[0].y, q[1].x, q[1].y));
+                rec.push_back(make_int4(q[2].x, q[2].y, q[3].x, q[3].y));
             }
-            rec[3 * (size_t)t] = make_int4(i, np, off, 0);
-            rec[3 * (size_t)t + 1] = make_int4(q[0].x, q[0].y, q[1].x, q[1].y);
-            rec[3 * (size_t)t + 2] = make_int4(q[2].x, q[2].y, q[3].x, q[3].y);
+            while (rec.size() % 48) {
+                const size_t first = rec.size() / 48 * 48;
+                for (int k = 0; k < 3; ++k) {
+                    int4 r = rec[first + k];
+                    if (k == 0) r.w = 0;
+                    rec.push_back(r);
+                }
+            }
         }
         if (ovf.empty()) ovf.push_back(make_int2(0, 0));
         c->ls_slots[dir].upload(rec, c->stream);
         c->ls_ovf[dir].upload(ovf, c->stream);
+        SEMO_HIP(hipStreamSynchronize(c->stream));   // rec and ovf are temporaries
     }
-    SEMO_HIP(hipStreamSynchronize(c->stream));
     c->ls_ready = true;
 }
 
@@ -521,31 +625,38 @@ void linsol_run(semo_ctx* c, int method, double time_step, const double* st, dou
         return;
     }
     lusgs_schedule(c);
-    c->ls_dinv.ensure((size_t)N * N * n);
+    c->ls_dinv.ensure((size_t)N * N * 64 * ((n + 63) / 64));
     const double sides = (double)c->h_cf_idx.size();
     SEMO_LAUNCH(c, "lusgs_diag", (double)n * (K + N * N + 3) * 8.0 + sides * (4.0 + 8.0 + 32.0 + K * 8.0),
                 k_lusgs_diag<NSP>, g, b, n, c->nif, c->d_cf_ptr.p, c->d_cf_idx.p, c->d_owner.p, c->d_nbr.p,
                 c->f_nrm.p, c->f_area.p, c->c_vol.p, st, time_step, c->ls_dinv.p);
+    // forward results, backward results; tickets and error word
+    const size_t nv = (size_t)N * n;
+    c->ls_out.ensure(2 * nv);
+    c->ls_ctl.ensure(LS_CTL);
+    SEMO_LAUNCH(c, "lusgs_empty", 16.0 * nv, k_lusgs_empty, dim3(nblk(2 * (long)nv)), b, 2 * nv,
+                reinterpret_cast<unsigned long long*>(c->ls_out.p), c->ls_ctl.p);
+    // per cell: record, Dinv, own residual read + write, slot record; per
+    // earlier (later) neighbour: its record and residual, the face's normal
+    // and area (half the sides)
+    const double bytes = (double)n * ((K + N * N + 2 * N + 1) * 8.0 + 48.0) + 0.5 * sides * ((K + N) * 8.0 + 40.0);
     for (int dir = 0; dir < 2; ++dir) {
-        const std::vector<int>& ptr = c->ls_lev_ptr[dir];
-        const int nlev = (int)ptr.size() - 1;
-        for (int l = 0; l < nlev; ++l) {
-            const int cnt = ptr[l + 1] - ptr[l];
-            if (cnt == 0) continue;
-            // per cell: record, Dinv, own residual read + write, slot record;
-            // per earlier (later) neighbour: its record and residual, the
-            // face's normal and area, the pair (half the sides)
-            const double bytes = (double)cnt * ((K + N * N + 2 * N + 1) * 8.0 + 48.0) +
-                                 0.5 * (double)cnt * (sides / n) * ((K + N) * 8.0 + 40.0);
-            const int4* slots = c->ls_slots[dir].p + 3 * (size_t)ptr[l];
-            if (dir == 0)
-                SEMO_LAUNCH(c, "lusgs_sweep", bytes, (k_lusgs_level<NSP, true>), dim3(nblk(4L * cnt)), b, cnt, slots,
-                            c->ls_ovf[0].p, c->f_nrm.p, c->f_area.p, c->c_vol.p, st, c->ls_dinv.p, res);
-            else
-                SEMO_LAUNCH(c, "lusgs_sweep", bytes, (k_lusgs_level<NSP, false>), dim3(nblk(4L * cnt)), b, cnt,
-                            slots, c->ls_ovf[1].p, c->f_nrm.p, c->f_area.p, c->c_vol.p, st, c->ls_dinv.p, res);
-        }
+        const int nu = (int)(c->ls_slots[dir].n / 48);
+        // more wavefronts than can be resident only wait for a slot
+        const dim3 gu(std::min(nblk(64L * nu), LS_BLOCKS));
+        if (dir == 0)
+            SEMO_LAUNCH(c, "lusgs_sweep", bytes, (k_lusgs_sweep<NSP, true>), gu, b, nu, c->ls_slots[0].p,
+                        c->ls_ovf[0].p, c->f_nrm.p, c->f_area.p, c->c_vol.p, st, c->ls_dinv.p,
+                        (const double*)res, c->ls_out.p, (double*)nullptr, c->ls_ctl.p);
+        else
+            SEMO_LAUNCH(c, "lusgs_sweep", bytes, (k_lusgs_sweep<NSP, false>), gu, b, nu, c->ls_slots[1].p,
+                        c->ls_ovf[1].p, c->f_nrm.p, c->f_area.p, c->c_vol.p, st, c->ls_dinv.p,
+                        (const double*)c->ls_out.p, c->ls_out.p + nv, res, c->ls_ctl.p);
     }
+    int err = 0;
+    SEMO_HIP(hipMemcpyAsync(&err, c->ls_ctl.p + LS_ERR, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    SEMO_HIP(hipStreamSynchronize(c->stream));
+    SEMO_CHECK(err == 0, SEMO_EHIP, "LU-SGS sweep: a neighbour's update did not arrive");
 }
 
 // updateValues (src/solvers/densityBased.cpp:366-512), per cell: the
@@ -622,11 +733,6 @@ void linsol_device(semo_ctx* c, int method, int nsp, double time_step, const dou
     case 4: linsol_run<4>(c, method, time_step, st, res); break;
     default: SEMO_CHECK(false, SEMO_EINVAL, "linear solver: 1 <= nsp <= 4");
     }
-}
-
-int lusgs_levels(semo_ctx* c, int dir) {
-    lusgs_schedule(c);
-    return (int)c->ls_lev_ptr[dir].size() - 1;
 }
 
 }  // namespace semo
