@@ -347,8 +347,8 @@ struct semo_ctx {
     semo::DBuf<double> kv64;                   // Krylov work (fp64)
     semo::DBuf<float> kv32;
     semo_solve_stats last_stats_mom{}, last_stats_p{}, last_stats_vf{};
-    double* pin = nullptr;                     // pinned Krylov residual slots [4]
-    hipEvent_t pev[4] = {};
+    double* pin = nullptr;                     // pinned Krylov scalars (PIPE_*)
+    hipEvent_t pev[6] = {};
     semo::AdjBufs* adj = nullptr;
     semo::Coupled* cpl = nullptr;
     // this device's copy of the no-allocation entry point's scratch
@@ -392,23 +392,31 @@ inline double cell_faces_bytes(const semo_ctx* c, double per_face) {
     } while (0)
 
 // ------------------------------------------------- Krylov convergence tests --
-// Iteration k's squared residual is copied into pinned slot k % 4 behind an
-// event.  ConvCheck reads it only once iteration k + 1 has been issued, so the
-// device has queued work while the host waits -- except near convergence:
-// when the residual history predicts that iteration k meets the tolerance,
-// k is read at once (a short stall instead of a wasted iteration).
+// Iteration k's squared residual arrives in pinned slot k % 4 behind an event:
+// the kernel that finishes the reduction stores it there itself (pipe_slot,
+// then pipe_mark), or a copy brings it (pipe_push).  ConvCheck reads it only
+// once iteration k + 1 has been issued, so the device has queued work while
+// the host waits -- except near convergence: when the residual history
+// predicts that iteration k meets the tolerance, k is read at once (a short
+// stall instead of a wasted iteration).  Slots PIPE_BB and PIPE_END carry the
+// right-hand side's squared norm and the final true residual.
+constexpr int PIPE_BB = 4, PIPE_END = 5, PIPE_SLOTS = 6;
 inline void pipe_init(semo_ctx* c) {
     if (c->pin) return;
-    SEMO_HIP(hipHostMalloc((void**)&c->pin, 4 * sizeof(double), hipHostMallocDefault));
+    SEMO_HIP(hipHostMalloc((void**)&c->pin, PIPE_SLOTS * sizeof(double), hipHostMallocDefault));
     for (hipEvent_t& e : c->pev) SEMO_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
 }
-inline void pipe_push(semo_ctx* c, const double* dscalar, int k) {
-    SEMO_HIP(hipMemcpyAsync(c->pin + (k & 3), dscalar, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    SEMO_HIP(hipEventRecord(c->pev[k & 3], c->stream));
+inline int pipe_of(int k) { return k & 3; }              // slot of iteration k
+inline double* pipe_slot(semo_ctx* c, int slot) { pipe_init(c); return c->pin + slot; }
+inline void pipe_mark(semo_ctx* c, int slot) { SEMO_HIP(hipEventRecord(c->pev[slot], c->stream)); }
+inline double pipe_read(semo_ctx* c, int slot) {
+    SEMO_HIP(hipEventSynchronize(c->pev[slot]));
+    return ((volatile double*)c->pin)[slot];
 }
-inline double pipe_pop(semo_ctx* c, int k) {
-    SEMO_HIP(hipEventSynchronize(c->pev[k & 3]));
-    return ((volatile double*)c->pin)[k & 3];
+inline void pipe_push(semo_ctx* c, const double* dscalar, int k) {
+    int s = pipe_of(k);
+    SEMO_HIP(hipMemcpyAsync(c->pin + s, dscalar, sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    pipe_mark(c, s);
 }
 // Final test of a solve, on its true FP64 relative residual: a non-finite
 // residual (NaN/Inf in the system or the iterates) or one above
@@ -428,10 +436,19 @@ struct ConvCheck {
     double lim;                 // stop when the squared residual <= lim (NaN stops too)
     int read = 0;               // last iteration whose residual was read
     double r1, r2 = -1.0;       // last two residuals read (r1 starts as |b|^2)
+    bool have_bb = true;
     ConvCheck(semo_ctx* c_, double lim_, double bb) : c(c_), lim(lim_), r1(bb) { pipe_init(c_); }
-    void take(int k) { double v = pipe_pop(c, k); r2 = r1; r1 = v; read = k; }
+    // |b|^2 is still on its way to slot PIPE_BB: it is read, and scales the
+    // squared relative tolerance, at the first test
+    ConvCheck(semo_ctx* c_, double tol2) : c(c_), lim(tol2), r1(0.0), have_bb(false) {}
+    double bb() {
+        if (!have_bb) { r1 = pipe_read(c, PIPE_BB); lim *= r1; have_bb = true; }
+        return r1;
+    }
+    void take(int k) { double v = pipe_read(c, pipe_of(k)); r2 = r1; r1 = v; read = k; }
     // after iteration `it` pushed its residual: true = stop
     bool done(int it) {
+        bb();
         if (read < it - 1) {
             take(it - 1);
             if (!(r1 > lim)) return true;         // it - 1 converged; `it` ran one step further

@@ -62,28 +62,34 @@ __device__ inline void block_partials(double (&v)[2], double* __restrict__ part)
 }
 
 // Krylov scalars in device memory (slots of c->scal)
-enum { S_RZ = 0, S_ZRO = 1, S_RR = 2, S_PQ = 4, S_X = 6, S_ALPHA = 10, S_BETA = 11, S_OMEGA = 12,
-       S_TT = 14, S_TS = 15, S_RHO = 16, S_AV = 20 };
+enum { S_RZ = 0, S_RR = 2, S_X = 6, S_ALPHA = 10, S_BETA = 11, S_OMEGA = 12,
+       S_TT = 14, S_TS = 15, S_RHO = 16, S_AV = 20,
+       S_RZ2 = 24, S_ALPHA2 = 26 };   // r.z and alpha of even / odd iterations (in-kernel totals)
 
 // what the last block does with the totals d[0], d[1]
 enum { W_STORE = 0,      // s[slot] = d0, s[slot+1] = d1
        W_FCG_ALPHA,      // d0 = p.Ap:  alpha = rz / p.Ap
-       W_FCG_BETA,       // d0 = r.z, d1 = z.r_old: Polak-Ribiere beta, rz = d0
+       W_FCG_BETA,       // d0 = r.z, d1 = z.Ap: Polak-Ribiere beta, rz = d0
+       W_FCG_START,      // d0 = r.z of the first direction: rz = d0, beta = 0
        W_BICG_INIT,      // d0 = b.b: rho = rr = b.b, beta = 0, alpha = omega = 1
        W_BICG_ALPHA,     // d0 = rh.v: alpha = rho / rh.v
        W_BICG_OMEGA,     // d0 = t.t, d1 = t.s: omega = t.s / t.t
        W_BICG_RHO };     // d0 = r.r, d1 = rh.r: beta = (rho'/rho)(alpha/omega), rho = rho'
+
+__device__ inline double fcg_alpha(double rz, double pq) { return pq != 0.0 ? rz / pq : 0.0; }
+__device__ inline double fcg_beta(double rz_old, double alpha, double zq) {
+    return rz_old != 0.0 ? -alpha * zq / rz_old : 0.0;
+}
 
 __device__ void finish_scalars(int what, int slot, const double (&d)[2], double* s) {
     switch (what) {
     case W_STORE: s[slot] = d[0]; s[slot + 1] = d[1]; break;
     // zero denominators (an exactly solved system) give zero steps, so that
     // an iteration issued past convergence leaves x unchanged
-    case W_FCG_ALPHA: s[S_PQ] = d[0]; s[S_ALPHA] = d[0] != 0.0 ? s[S_RZ] / d[0] : 0.0; break;
-    case W_FCG_BETA:
-        s[S_BETA] = s[S_RZ] != 0.0 ? (d[0] - d[1]) / s[S_RZ] : 0.0;
-        s[S_RZ] = d[0]; s[S_ZRO] = d[1];
-        break;
+    case W_FCG_ALPHA: s[S_ALPHA] = fcg_alpha(s[S_RZ], d[0]); break;
+    // z.(r - r_old) = -alpha z.Ap, so r_old is not kept
+    case W_FCG_BETA: s[S_BETA] = fcg_beta(s[S_RZ], s[S_ALPHA], d[1]); s[S_RZ] = d[0]; break;
+    case W_FCG_START: s[S_BETA] = 0.0; s[S_RZ] = d[0]; break;
     case W_BICG_INIT:
         s[S_X] = d[0]; s[S_RR] = d[0]; s[S_RHO] = d[0];
         s[S_BETA] = 0.0; s[S_ALPHA] = 1.0; s[S_OMEGA] = 1.0;
@@ -108,8 +114,9 @@ __device__ inline void reduce2(double (&v)[2], const Red& rd) { block_partials(v
 // ordered sum of nb partial pairs, then the scalar update `what`; one
 // 1024-thread block, so each thread streams only a few partials
 constexpr int FTPB = 1024;
+// host (optional): a pinned word that also gets d0, so that no copy follows
 __global__ void __launch_bounds__(FTPB) k_finish(int nb, const double* __restrict__ part, double* __restrict__ s,
-                                                 int what, int slot) {
+                                                 int what, int slot, double* __restrict__ host) {
     double a0 = 0.0, a1 = 0.0;
     const double2* p2 = reinterpret_cast<const double2*>(part);
     for (int i = threadIdx.x; i < nb; i += FTPB) { double2 v = p2[i]; a0 += v.x; a1 += v.y; }
@@ -126,7 +133,27 @@ __global__ void __launch_bounds__(FTPB) k_finish(int nb, const double* __restric
     if (threadIdx.x == 0) {
         double d[2] = {sh[0][0], sh[1][0]};
         finish_scalars(what, slot, d, s);
+        if (host) __hip_atomic_store(host, d[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
+}
+
+// The totals of nb partial pairs, formed by every block of a kernel that needs
+// them, in one order for all (256 threads each).  Up to TOTAL_MAX pairs this
+// costs no more device time than k_finish before it and saves its launch: at
+// 222650 cells (870 pairs) k_fcg_update takes 7.3 us with its own totals
+// against 5.1 + 2.8 us, k_spmv_xpby 9.7 against 7.0 + 2.8 us.
+constexpr int TOTAL_MAX = 1024;
+__device__ inline double2 block_total(int nb, const double* __restrict__ part) {
+    __shared__ double sh[2][TPB / 64];
+    double a0 = 0.0, a1 = 0.0;
+    const double2* p2 = reinterpret_cast<const double2*>(part);
+    for (int i = threadIdx.x; i < nb; i += TPB) { double2 v = p2[i]; a0 += v.x; a1 += v.y; }
+    a0 = wave_sum(a0); a1 = wave_sum(a1);
+    if ((threadIdx.x & 63) == 0) { sh[0][threadIdx.x >> 6] = a0; sh[1][threadIdx.x >> 6] = a1; }
+    __syncthreads();
+    double2 t = make_double2(0.0, 0.0);
+    for (int w = 0; w < TPB / 64; ++w) { t.x += sh[0][w]; t.y += sh[1][w]; }
+    return t;
 }
 
 // a.b (+ c.d) over a grid-stride range
@@ -380,34 +407,113 @@ __global__ void __launch_bounds__(TPB) k_spmv_dot(int n, const int* __restrict__
     reduce2(v, rd);
 }
 
-// FCG direction update fused into its product: pn = z + beta po (beta =
-// s[S_BETA]), q = A pn, partials pn.q.  po and pn are distinct buffers:
-// neighbours read po while the row writes pn.
+// Where an FCG kernel finds a scalar it needs: nb > 0 -- it forms the totals
+// of the partials itself (block_total) and one thread keeps what the next
+// kernels need in the slots of this iteration's parity; nb == 0 -- k_finish
+// left it in its slot.
+struct FcgIn {
+    const double* __restrict__ part;
+    int nb, par, first;
+};
+
+// FCG direction update fused into its product: pn = z + beta po, q = A pn,
+// partials pn.q; the first direction is z.  po and pn are distinct buffers:
+// neighbours read po while the row writes pn.  z comes as the V-cycle left
+// it: FP32 (TZ = float) from an FP32 one.
+template <class TZ>
 __global__ void __launch_bounds__(TPB) k_spmv_xpby(int n, const int* __restrict__ sl_ptr,
                                                    const int* __restrict__ col, const int16_t* __restrict__ dcol,
                                                    const double* __restrict__ val, const double* __restrict__ diag,
-                                                   const double* __restrict__ s, const double* __restrict__ z,
+                                                   double* __restrict__ s, FcgIn in, const TZ* __restrict__ z,
                                                    const double* __restrict__ po, double* __restrict__ pn,
                                                    double* __restrict__ q, Red rd) {
     int row = xcd_block() * blockDim.x + threadIdx.x;
     int sl = row >> 6, lane = row & 63;
     double v[2] = {0.0, 0.0};
+    double beta = 0.0;
+    if (in.nb) {
+        double2 t = block_total(in.nb, in.part);                  // r.z, z.Ap_old
+        if (!in.first) beta = fcg_beta(s[S_RZ2 + (in.par ^ 1)], s[S_ALPHA2 + (in.par ^ 1)], t.y);
+        if (blockIdx.x == 0 && threadIdx.x == 0) s[S_RZ2 + in.par] = t.x;
+    } else if (!in.first) {
+        beta = s[S_BETA];
+    }
     if (sl < ((n + 63) >> 6)) {
-        double beta = s[S_BETA];
         // the row's own operands are requested before the gathers
         bool own = row < n;
-        double zr = own ? z[row] : 0.0, por = own ? po[row] : 0.0, dr = own ? diag[row] : 0.0;
-        auto opnd = [&](int j) { return z[j] + beta * po[j]; };
-        double acc = dcol ? sell2_row_sum<SELL_PAIRS>(sl_ptr[sl], sl_ptr[sl + 1], lane, val,
-                                                      [&](int e) { return sell2_dcol(dcol, e, row); }, opnd)
-                          : sell2_row_sum<SELL_PAIRS>(sl_ptr[sl], sl_ptr[sl + 1], lane, val,
-                                                      [&](int e) { return sell2_col(col, e); }, opnd);
+        double zr = own ? (double)z[row] : 0.0, dr = own ? diag[row] : 0.0;
+        double por = own && !in.first ? po[row] : 0.0;
+        auto sum = [&](auto opnd) {
+            return dcol ? sell2_row_sum<SELL_PAIRS>(sl_ptr[sl], sl_ptr[sl + 1], lane, val,
+                                                    [&](int e) { return sell2_dcol(dcol, e, row); }, opnd)
+                        : sell2_row_sum<SELL_PAIRS>(sl_ptr[sl], sl_ptr[sl + 1], lane, val,
+                                                    [&](int e) { return sell2_col(col, e); }, opnd);
+        };
+        double acc = in.first ? sum([&](int j) { return (double)z[j]; })
+                              : sum([&](int j) { return (double)z[j] + beta * po[j]; });
         if (own) {
-            double pr = zr + beta * por;
+            double pr = in.first ? zr : zr + beta * por;
             pn[row] = pr;
             acc += dr * pr;
             q[row] = acc;
             v[0] = pr * acc;
+        }
+    }
+    reduce2(v, rd);
+}
+
+// the V-cycle's last step at the finest level, x + c1 D^-1 (b - A x) into z
+// (its own precision), with the dots the next direction needs: r.z and z.q
+template <class T>
+__global__ void __launch_bounds__(TPB) k_chebx_dot(RowArgs<T> a, const double* __restrict__ r,
+                                                   const double* __restrict__ q, Red rd) {
+    int row = xcd_block() * TPB + threadIdx.x;
+    int s = row >> 6, lane = row & 63;
+    double v[2] = {0.0, 0.0};
+    if (s < ((a.n + 63) >> 6)) {
+        Own<T> own{};
+        double ri = 0.0, qi = 0.0;
+        if (row < a.n) {
+            own = load_own<T, OP_CHEBX>(a, row);
+            ri = r[row]; qi = q[row];
+        }
+        auto opnd = [&](int j) { return a.x[j]; };
+        T acc = a.dcol ? sell2_row_sum<SELL_PAIRS>(a.ptr[s], a.ptr[s + 1], lane, a.val,
+                                                   [&](int e) { return sell2_dcol(a.dcol, e, row); }, opnd)
+                       : sell2_row_sum<SELL_PAIRS>(a.ptr[s], a.ptr[s + 1], lane, a.val,
+                                                   [&](int e) { return sell2_col(a.col, e); }, opnd);
+        if (row < a.n) {
+            acc += own.d * own.x;
+            T res = own.dv * (own.b - acc);
+            T di = res * a.c1;
+            T xn = own.x + di;
+            a.xo[row] = xn;
+            v[0] = ri * (double)xn; v[1] = qi * (double)xn;
+        }
+    }
+    reduce2(v, rd);
+}
+
+// |b - A x|^2 (sliced ELL, FP64), the residual itself not stored
+__global__ void __launch_bounds__(TPB) k_resid_norm(int n, const int* __restrict__ sl_ptr, const int* __restrict__ col,
+                                                    const int16_t* __restrict__ dcol, const double* __restrict__ val,
+                                                    const double* __restrict__ diag, const double* __restrict__ x,
+                                                    const double* __restrict__ b, Red rd) {
+    int row = xcd_block() * blockDim.x + threadIdx.x;
+    int s = row >> 6, lane = row & 63;
+    double v[2] = {0.0, 0.0};
+    if (s < ((n + 63) >> 6)) {
+        bool own = row < n;
+        double dr = own ? diag[row] : 0.0, xr = own ? x[row] : 0.0, br = own ? b[row] : 0.0;
+        auto opnd = [&](int j) { return x[j]; };
+        double acc = dcol ? sell2_row_sum<SELL_PAIRS>(sl_ptr[s], sl_ptr[s + 1], lane, val,
+                                                      [&](int e) { return sell2_dcol(dcol, e, row); }, opnd)
+                          : sell2_row_sum<SELL_PAIRS>(sl_ptr[s], sl_ptr[s + 1], lane, val,
+                                                      [&](int e) { return sell2_col(col, e); }, opnd);
+        if (own) {
+            acc += dr * xr;
+            double t = br - acc;
+            v[0] = t * t;
         }
     }
     reduce2(v, rd);
@@ -442,27 +548,31 @@ __device__ inline void prep_store(const Prep& pp, int i, double ri) {
     }
 }
 
-// x = 0, r = b, d0 = b.b
-__global__ void __launch_bounds__(TPB) k_fcg_init(int n, const double* __restrict__ b, double* __restrict__ x,
-                                                  double* __restrict__ r, Red rd, Prep pp) {
+// r = b, d0 = b.b
+__global__ void __launch_bounds__(TPB) k_fcg_init(int n, const double* __restrict__ b, double* __restrict__ r, Red rd,
+                                                  Prep pp) {
     int i = xcd_block() * blockDim.x + threadIdx.x;
     double v[2] = {0.0, 0.0};
-    if (i < n) { double bi = b[i]; x[i] = 0.0; r[i] = bi; v[0] = bi * bi; prep_store(pp, i, bi); }
+    if (i < n) { double bi = b[i]; r[i] = bi; v[0] = bi * bi; prep_store(pp, i, bi); }
     reduce2(v, rd);
 }
 
-// x += alpha p ; r_old = r ; r -= alpha q ; d0 = r.r
-__global__ void __launch_bounds__(TPB) k_fcg_update(int n, const double* __restrict__ s, double* __restrict__ x,
-                                                    double* __restrict__ r, double* __restrict__ rold,
-                                                    const double* __restrict__ p, const double* __restrict__ q,
-                                                    Red rd, Prep pp) {
+// x += alpha p (the first step from x = 0); r -= alpha q ; d0 = r.r
+__global__ void __launch_bounds__(TPB) k_fcg_update(int n, double* __restrict__ s, FcgIn in, double* __restrict__ x,
+                                                    double* __restrict__ r, const double* __restrict__ p,
+                                                    const double* __restrict__ q, Red rd, Prep pp) {
     int i = xcd_block() * blockDim.x + threadIdx.x;
     double v[2] = {0.0, 0.0};
+    double a;
+    if (in.nb) {
+        a = fcg_alpha(s[S_RZ2 + in.par], block_total(in.nb, in.part).x);
+        if (blockIdx.x == 0 && threadIdx.x == 0) s[S_ALPHA2 + in.par] = a;
+    } else {
+        a = s[S_ALPHA];
+    }
     if (i < n) {
-        double a = s[S_ALPHA];
-        x[i] += a * p[i];
+        x[i] = in.first ? a * p[i] : x[i] + a * p[i];
         double ri = r[i];
-        rold[i] = ri;
         ri -= a * q[i];
         r[i] = ri;
         v[0] = ri * ri;
@@ -772,9 +882,18 @@ Tags level_tags(int l, bool fp64) {
 // Chebyshev interval [lo, hi] of a level's smoother
 inline void cheb_interval(const AmgLevel& L, double& lo, double& hi) { hi = 1.1 * L.lmax; lo = hi / 10.0; }
 
+// what the last step of a V-cycle does for the FCG loop around it (degree 1):
+// its result goes to z in the V-cycle's precision, with the block partials of
+// r.z and z.q
+struct VcDot {
+    void* z;
+    const double *r, *q;
+    double* part;
+};
+
 template <class T>
 void cheb_smooth(semo_ctx* c, AmgLevel& L, T* b, int degree, bool x_zero, const double* bsrc, double* zo,
-                 const Tags& tg) {
+                 const Tags& tg, const VcDot* vd = nullptr) {
     const DevSell<T>& A = opA<T>(L);
     int n = L.n;
     T* dA = vt<T>(L); T* dB = vu<T>(L); T* r = vr<T>(L);
@@ -787,6 +906,13 @@ void cheb_smooth(semo_ctx* c, AmgLevel& L, T* b, int degree, bool x_zero, const 
                     (double)sizeof(T) * 5 * n + (bsrc ? 8.0 * n : 0.0) + (degree == 1 && zo ? 8.0 * n : 0.0),
                     k_cheb_init<T>, dim3(nblk(n)), dim3(TPB), n, vdinv<T>(L), b, bsrc, (T)(1.0 / theta), r, dA,
                     bx<T>(L).p, degree == 1 ? zo : nullptr);
+    } else if (degree == 1 && vd) {
+        RowArgs<T> a{};
+        a.n = A.n; a.ptr = A.sl_ptr.p; a.col = A.col.p; a.val = A.val.p; a.diag = A.diag.p;
+        a.dcol = A.dcol.n ? A.dcol.p : nullptr;
+        a.x = bx<T>(L).p; a.b = b; a.dinv = vdinv<T>(L); a.xo = static_cast<T*>(vd->z); a.c1 = (T)(1.0 / theta);
+        SEMO_LAUNCH(c, tg.chebx, op_bytes(A, 4) + 16.0 * n, k_chebx_dot<T>, dim3(nblk((long)A.nslices * 64)),
+                    dim3(TPB), a, vd->r, vd->q, Red{vd->part});
     } else if (degree == 1) {
         // the only step: r and y are dead, and with zo (the finest level)
         // so is the T iterate, which keeps the level's x buffer in place
@@ -821,7 +947,8 @@ void cheb_smooth(semo_ctx* c, AmgLevel& L, T* b, int degree, bool x_zero, const 
 // the kernel that produced b (the Krylov residual update at level 0, the
 // restriction below it)
 template <class T>
-void vcycle(semo_ctx* c, Amg& amg, int l, int degree, const double* bsrc, double* zo, bool prepared = false) {
+void vcycle(semo_ctx* c, Amg& amg, int l, int degree, const double* bsrc, double* zo, bool prepared = false,
+            const VcDot* vd = nullptr) {
     AmgLevel& L = amg.lv[l];
     int n = L.n;
     T* b = vb<T>(L);
@@ -859,7 +986,7 @@ void vcycle(semo_ctx* c, Amg& amg, int l, int degree, const double* bsrc, double
     }
     vcycle<T>(c, amg, l + 1, degree, nullptr, nullptr, prep_next);
     spmv<T, OP_ADD>(c, opP<T>(L), bx<T>(C).p, (const T*)nullptr, bx<T>(L).p, tg.prolong);
-    cheb_smooth<T>(c, L, b, degree, false, nullptr, zo, tg);
+    cheb_smooth<T>(c, L, b, degree, false, nullptr, zo, tg, vd);
 }
 
 // z = M^-1 r with one V-cycle in precision T.  The V-cycle is a fixed
@@ -875,8 +1002,11 @@ void sig_op(std::vector<const void*>& s, const DevSell<T>& M) {
 }
 // every device address a V-cycle in precision T passes to its kernels
 template <class T>
-std::vector<const void*> vcycle_signature(const Amg& amg, const double* r64, const double* z64) {
+std::vector<const void*> vcycle_signature(const Amg& amg, const double* r64, const double* z64, const VcDot* vd) {
     std::vector<const void*> s{r64, z64, amg.coarse_inv.p};
+    if (vd)
+        for (const void* p : {(const void*)vd->z, (const void*)vd->r, (const void*)vd->q, (const void*)vd->part})
+            s.push_back(p);
     for (const AmgLevel& L : amg.lv) {
         if (sizeof(T) == 8) {
             for (const void* p : {(const void*)L.x64.p, (const void*)L.b64.p, (const void*)L.r64.p,
@@ -896,20 +1026,21 @@ std::vector<const void*> vcycle_signature(const Amg& amg, const double* r64, con
 }
 
 template <class T>
-void precondition(semo_ctx* c, Amg& amg, const double* r64, double* z64, bool prepared = false) {
+void precondition(semo_ctx* c, Amg& amg, const double* r64, double* z64, bool prepared = false,
+                  const VcDot* vd = nullptr) {
     int deg = cheb_degree(c);
     if (!c->graphs || c->prof.on) {
-        vcycle<T>(c, amg, 0, deg, r64, z64, prepared);
+        vcycle<T>(c, amg, 0, deg, r64, z64, prepared, vd);
         return;
     }
     int prec = sizeof(T) == 4 ? 1 : 0;
-    std::vector<const void*> sig = vcycle_signature<T>(amg, r64, z64);
+    std::vector<const void*> sig = vcycle_signature<T>(amg, r64, z64, vd);
     if (!amg.vg || amg.vg_stream != c->stream || amg.vg_sig != sig || amg.vg_deg != deg || amg.vg_prec != prec ||
         amg.vg_pre != prepared) {
         amg.drop_graph();
         hipGraph_t g = nullptr;
         SEMO_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-        vcycle<T>(c, amg, 0, deg, r64, z64, prepared);
+        vcycle<T>(c, amg, 0, deg, r64, z64, prepared, vd);
         SEMO_HIP(hipStreamEndCapture(c->stream, &g));
         hipError_t e = hipGraphInstantiate(&amg.vg, g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
@@ -918,7 +1049,7 @@ void precondition(semo_ctx* c, Amg& amg, const double* r64, double* z64, bool pr
         // the capture swapped some levels' x buffers (out-of-place smoothing
         // steps): the graph holds the addresses from before the swaps, the
         // same set
-        amg.vg_sig = vcycle_signature<T>(amg, r64, z64);
+        amg.vg_sig = vcycle_signature<T>(amg, r64, z64, vd);
         SEMO_CHECK(amg.vg_sig == sig, SEMO_EHIP, "V-cycle capture changed its buffer set");
     }
     SEMO_HIP(hipGraphLaunch(amg.vg, c->stream));
@@ -935,9 +1066,14 @@ Red red_of(semo_ctx* c) { return Red{c->red.p}; }
 
 
 // sums the partials of the previous launch (nb blocks) and applies `what`
-void finish(semo_ctx* c, int nb, int what, int slot = 0) {
-    SEMO_LAUNCH(c, "krylov_finish", 16.0 * nb + 8.0, k_finish, dim3(1), dim3(FTPB), nb, c->red.p, c->scal.p, what,
-                slot);
+void finish(semo_ctx* c, int nb, int what, int slot = 0, double* host = nullptr, const double* part = nullptr) {
+    SEMO_LAUNCH(c, "krylov_finish", 16.0 * nb + 8.0, k_finish, dim3(1), dim3(FTPB), nb, part ? part : c->red.p,
+                c->scal.p, what, slot, host);
+}
+// ... and its total to the host's pinned slot
+void finish_to_host(semo_ctx* c, int nb, int what, int slot, int pslot, const double* part = nullptr) {
+    finish(c, nb, what, slot, pipe_slot(c, pslot), part);
+    pipe_mark(c, pslot);
 }
 
 // grid-stride dot products a.b (+ c.d), finished as `what`
@@ -964,15 +1100,24 @@ void spmv_dot(semo_ctx* c, const DevSell<double>& A, const double* x, double* y,
 
 // flexible (Polak-Ribiere) PCG with the AMG preconditioner.  x0 = 0,
 // stop at ||r|| <= tol ||b||.
+//
+// An iteration is the V-cycle (its last step leaves z and the dots r.z, z.q),
+// the direction and its product, the update of x and r (which also writes
+// the next V-cycle's level-0 input) and the residual's way to the host: three
+// launches and a graph, with the scalars of small systems formed where they
+// are used (block_total), five with k_finish launches for large ones.  (With
+// the dots, the scalars and the residual's copy as launches of their own and
+// r_old kept, a time step took 1.18 ms at 16^3, now 0.99; at 128^3 the V-cycle's
+// last step and the dots take 32.0 us instead of 25.4 + 9.1.)
 int fpcg(semo_ctx* c, Amg& amg, const DevSell<double>& A, const double* b, double* x, double tol, int maxit,
          bool mixed, double* relres) {
     SEMO_CHECK(A.lanes == 0, SEMO_EINVAL, "Krylov operator must be sliced ELL");
     int n = A.n;
     size_t ln = (size_t)n + 64;
     c->kv64.ensure(8 * ln);
-    double* r = c->kv64.p; double* z = r + ln; double* p = z + ln; double* q = p + ln; double* rold = q + ln;
-    // mixed precision, degree-1 smoothing, at least two levels: the kernels
-    // that produce r also write the FP32 V-cycle's level-0 input
+    double* r = c->kv64.p; double* z = r + ln; double* p = z + ln; double* q = p + ln; double* p2 = q + ln;
+    // degree-1 smoothing, at least two levels: the kernels that produce r also
+    // write the V-cycle's level-0 input, and its last step the dots
     Prep pp{};
     bool prep = cheb_degree(c) == 1 && amg.lv.size() >= 2 && amg.lv[0].n == n;
     if (prep) {
@@ -987,44 +1132,56 @@ int fpcg(semo_ctx* c, Amg& amg, const DevSell<double>& A, const double* b, doubl
             pp.c1d = 1.0 / (0.5 * (hi + lo));
         }
     }
+    int nbr = nblk(n), nbs = nblk((long)A.nslices * 64);
+    // partials of the three reductions of an iteration
+    double* part_z = c->red.p;
+    double* part_p = part_z + 2 * (size_t)std::max(nbs, RB);
+    double* part_r = part_p + 2 * (size_t)nbs;
+    bool own_totals = std::max(nbs, nbr) <= TOTAL_MAX;
+    const VcDot vd{z, r, q, part_z};
+    int nbz = prep ? nbs : rblk(n);                       // blocks of the r.z, z.q partials
+    bool z32 = prep && mixed;                             // z as the FP32 V-cycle leaves it
     auto pre = [&]() {
-        if (mixed) precondition<float>(c, amg, r, z, prep); else precondition<double>(c, amg, r, z, prep);
+        const VcDot* d = prep ? &vd : nullptr;
+        if (mixed) precondition<float>(c, amg, r, z, prep, d); else precondition<double>(c, amg, r, z, prep, d);
+        if (!prep)
+            SEMO_LAUNCH(c, "krylov_dot", 32.0 * n, k_dot, dim3(nbz), dim3(TPB), n, r, z, z, q, Red{part_z});
     };
     double prep_bytes = prep ? (mixed ? 8.0 : 16.0) * n : 0.0;     // the V-cycle's b and x written
-    SEMO_LAUNCH(c, "fcg_init", 24.0 * n + prep_bytes, k_fcg_init, dim3(nblk(n)), dim3(TPB), n, b, x, r, red_of(c), pp);
-    finish(c, nblk(n), W_STORE, S_X);
-    double bb = host_scalar(c, S_X);
-    if (bb == 0.0) { *relres = 0.0; return 0; }
-    double nb = std::sqrt(bb);
-    pre();
-    SEMO_LAUNCH(c, "fcg_copy", 16.0 * n, (k_cast<double, double>), dim3(nblk(n)), dim3(TPB), n, z, p);
-    dot_store(c, n, r, z, nullptr, nullptr, S_RZ);
+    SEMO_LAUNCH(c, "fcg_init", 16.0 * n + prep_bytes, k_fcg_init, dim3(nbr), dim3(TPB), n, b, r, Red{part_r}, pp);
+    finish_to_host(c, nbr, W_STORE, S_X, PIPE_BB, part_r);
+    ConvCheck cc(c, tol * tol);
     int it = 0;
-    ConvCheck cc(c, tol * tol * bb, bb);
-    double* p2 = rold + ln;                      // second direction buffer
+    double bb = 0.0;
     for (it = 1; it <= maxit; ++it) {
-        if (it == 1) {
-            spmv_dot(c, A, p, q, p, nullptr, W_FCG_ALPHA);                // q = A p, alpha
-        } else {                                                          // p = z + beta p; q = A p, alpha
-            int nbs = nblk((long)A.nslices * 64);
-            SEMO_LAUNCH(c, "spmv_xpby_fp64", op_bytes(A, 4), k_spmv_xpby, dim3(nbs), dim3(TPB), A.n, A.sl_ptr.p,
-                        A.col.p, A.dcol.n ? A.dcol.p : nullptr, A.val.p, A.diag.p, c->scal.p, z, p, p2, q,
-                        red_of(c));
-            finish(c, nbs, W_FCG_ALPHA);
-            std::swap(p, p2);
-        }
-        SEMO_LAUNCH(c, "fcg_update", 56.0 * n + prep_bytes, k_fcg_update, dim3(nblk(n)), dim3(TPB), n, c->scal.p, x,
-                    r, rold, p, q, red_of(c), pp);
-        finish(c, nblk(n), W_STORE, S_RR);
-        pipe_push(c, c->scal.p + S_RR, it);
-        if (cc.done(it) || it == maxit) break;
         pre();
-        dot_what(c, n, r, z, z, rold, W_FCG_BETA);                        // r.z, z.r_old -> beta
+        bool first = it == 1;
+        FcgIn in{part_z, own_totals ? nbz : 0, it & 1, first ? 1 : 0};
+        if (!own_totals) finish(c, nbz, first ? W_FCG_START : W_FCG_BETA, 0, nullptr, part_z);
+        const int16_t* dc = A.dcol.n ? A.dcol.p : nullptr;
+        // p = z + beta p, q = A p
+        if (z32)
+            SEMO_LAUNCH(c, "spmv_xpby_fp64", op_bytes(A, 3) + 4.0 * n, k_spmv_xpby<float>, dim3(nbs), dim3(TPB), n,
+                        A.sl_ptr.p, A.col.p, dc, A.val.p, A.diag.p, c->scal.p, in,
+                        reinterpret_cast<const float*>(z), p, p2, q, Red{part_p});
+        else
+            SEMO_LAUNCH(c, "spmv_xpby_fp64", op_bytes(A, 4), k_spmv_xpby<double>, dim3(nbs), dim3(TPB), n, A.sl_ptr.p,
+                        A.col.p, dc, A.val.p, A.diag.p, c->scal.p, in, z, p, p2, q, Red{part_p});
+        std::swap(p, p2);
+        in.part = part_p;
+        if (own_totals) in.nb = nbs;
+        else finish(c, nbs, W_FCG_ALPHA, 0, nullptr, part_p);
+        SEMO_LAUNCH(c, "fcg_update", 48.0 * n + prep_bytes, k_fcg_update, dim3(nbr), dim3(TPB), n, c->scal.p, in, x, r,
+                    p, q, Red{part_r}, pp);
+        finish_to_host(c, nbr, W_STORE, S_RR, pipe_of(it), part_r);
+        if (it == 1 && (bb = cc.bb()) == 0.0) { *relres = 0.0; return 0; }   // b = 0: that step left x = 0
+        if (cc.done(it)) break;
     }
     // true residual in FP64
-    spmv<double, OP_RES>(c, A, x, b, r, "true_resid_fp64");
-    dot_store(c, n, r, r, nullptr, nullptr, S_X);
-    *relres = std::sqrt(host_scalar(c, S_X)) / nb;
+    SEMO_LAUNCH(c, "true_resid_fp64", op_bytes(A, 2), k_resid_norm, dim3(nbs), dim3(TPB), n, A.sl_ptr.p, A.col.p,
+                A.dcol.n ? A.dcol.p : nullptr, A.val.p, A.diag.p, x, b, Red{part_r});
+    finish_to_host(c, nbs, W_STORE, S_X, PIPE_END, part_r);
+    *relres = std::sqrt(pipe_read(c, PIPE_END)) / std::sqrt(bb);
     return std::min(it, maxit);
 }
 
@@ -1244,9 +1401,10 @@ template void csr_upload<double>(DevSell<double>&, int, int, const std::vector<i
 template void csr_upload<float>(DevSell<float>&, int, int, const std::vector<int>&, const std::vector<int>&,
                                 const std::vector<double>&, const std::vector<double>&, int, hipStream_t);
 
-// partials for reductions over up to n rows (two values per block)
+// partials for reductions over up to n rows (two values per block, three
+// reductions at a time)
 void reduction_alloc(semo_ctx* c, long n) {
-    size_t need = 2 * (size_t)std::max(nblk(std::max<long>(n, 1) + 64), RB) + 64;
+    size_t need = 6 * (size_t)std::max(nblk(std::max<long>(n, 1) + 64), RB) + 64;
     if (c->red.n < need) c->red.alloc(need);
     if (c->scal.n < 64) c->scal.alloc(64);
 }
