@@ -221,7 +221,8 @@ void upload_csr(DevSell<T>& M, const HCsr& A, bool square, hipStream_t s, std::v
 // src_slot (optional): for every entry of A0, the slot of the device system
 // it came from (-1 on the diagonal); lets level 0 be refreshed on the device
 void amg_setup_host(semo_ctx* c, Amg& amg, const HCsr& A0, const std::vector<int>* src_slot = nullptr) {
-    amg.drop_graph();             // the level buffers are reallocated below
+    amg.graphs.drop();            // the level buffers are reallocated below
+    ++amg.builds;
     auto t0 = std::chrono::steady_clock::now();
     hipStream_t s = c->stream;
     amg.lv.clear();

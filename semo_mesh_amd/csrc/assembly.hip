@@ -1557,12 +1557,8 @@ __global__ void k_copy(size_t n, double* __restrict__ d, const double* __restric
 
 
 double finish_ratio(semo_ctx* c, int nb) {
-    std::vector<double> h(2 * (size_t)nb);
-    SEMO_HIP(hipMemcpyAsync(h.data(), c->red.p, h.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    SEMO_HIP(hipStreamSynchronize(c->stream));
-    double a = 0, b = 0;
-    for (int k = 0; k < nb; ++k) { a += h[2 * k]; b += h[2 * k + 1]; }
-    return sqrt(a) / sqrt(b);
+    double2 s = sum_to_host(c, nb, c->red.p);
+    return sqrt(s.x) / sqrt(s.y);
 }
 
 }  // namespace
@@ -1948,11 +1944,7 @@ double time_step(semo_ctx* c, int adjust) {
     SEMO_LAUNCH(c, "time_scale", cell_faces_bytes(c, 8.0) + 56.0 * c->nc + 16.0 * nb, k_time_scale, dim3(nb),
                 dim3(TPB), c->nc, k, adjust, c->d_cf_sl.p, c->d_cf_ell.p, c->f_area.p, c->c_vol.p, c->U.p, c->V.p,
                 c->W.p, c->Mu.p, c->Rho.p, c->red.p);
-    std::vector<double> h(2 * (size_t)nb);
-    SEMO_HIP(hipMemcpyAsync(h.data(), c->red.p, h.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    SEMO_HIP(hipStreamSynchronize(c->stream));
-    double minDt = 1000000.0;
-    for (int q = 0; q < nb; ++q) minDt = std::min(minDt, h[2 * q]);
+    double minDt = std::min(1000000.0, min_to_host(c, nb, c->red.p));
     if (!adjust) return c->cs.dt / minDt;
     c->cs.dt = c->cs.max_co * minDt;
     double co = c->cs.max_co;
@@ -1968,12 +1960,7 @@ double vof_update(semo_ctx* c) {
     int nb = nblk(c->nc);
     SEMO_LAUNCH(c, "vof_update", 24.0 * c->nc + 16.0 * nb, k_vof_update, dim3(nb), dim3(TPB), c->nc, c->cs.urf_vf,
                 c->Xvec.p, c->VF.p, c->red.p);
-    std::vector<double> h(2 * (size_t)nb);
-    SEMO_HIP(hipMemcpyAsync(h.data(), c->red.p, h.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    SEMO_HIP(hipStreamSynchronize(c->stream));
-    double a = 0;
-    for (int q = 0; q < nb; ++q) a += h[2 * q];
-    return sqrt(a);
+    return sqrt(sum_to_host(c, nb, c->red.p).x);
 }
 
 double momentum_update(semo_ctx* c) {

@@ -113,10 +113,10 @@ int guard(semo_ctx* c, const std::function<void()>& fn) {
         if (c) c->err.clear();
         return SEMO_OK;
     } catch (const Error& e) {
-        if (c) c->err = e.what();
+        if (c) { c->err = e.what(); ring_resync(c); }
         return e.code;
     } catch (const std::exception& e) {
-        if (c) c->err = e.what();
+        if (c) { c->err = e.what(); ring_resync(c); }
         return SEMO_EINVAL;
     }
 }
@@ -175,7 +175,8 @@ double pressure_eq(semo_ctx* c, semo_solve_stats* st, bool after_momentum = fals
 // one time step's set-up and its outer iterations, for the adjoint driver
 bool simple_setup(semo_ctx* c) {
     step_setup(c);
-    c->courant = time_step(c, c->cs.adjust_dt);
+    // a fixed time step reads no Courant number (semo_calc_time_step gives it)
+    if (c->cs.adjust_dt) c->courant = time_step(c, 1);
     for (int k = 0; k < c->cs.n_vof; ++k) volfrac_eq(c, &c->last_stats_vf);
     return step_sources(c);
 }
@@ -225,7 +226,6 @@ int semo_ctx_destroy(semo_ctx* c) {
     coupled_free(c->cpl);
     c->cpl = nullptr;
     if (c->pin) (void)hipHostFree(c->pin);
-    for (hipEvent_t e : c->pev) if (e) (void)hipEventDestroy(e);
     delete c;
     if (own) (void)hipStreamDestroy(s);
     return SEMO_OK;

@@ -7,6 +7,7 @@
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
+#include <cstring>
 #include <map>
 #include <memory>
 #include <numeric>
@@ -150,6 +151,53 @@ struct DevSell {
     size_t padded() const { return col.n; }
 };
 
+// ----------------------------------------------------------- HIP graphs -----
+// Kernel sequences captured as HIP graphs, by the device addresses (and the
+// few numbers) they were captured with: a lookup with another signature
+// captures anew, so a reallocated buffer is never reached through a stale
+// graph.  Dropped -- after the stream that may still run one -- with the
+// buffers' owner; at most eight are kept.
+struct GraphCache {
+    struct Entry {
+        std::vector<const void*> sig;
+        hipGraphExec_t exec;
+        hipStream_t stream;
+    };
+    std::vector<Entry> all;
+    void drop_first() {
+        (void)hipStreamSynchronize(all.front().stream);
+        (void)hipGraphExecDestroy(all.front().exec);
+        all.erase(all.begin());
+    }
+    void drop() { while (!all.empty()) drop_first(); }
+    GraphCache() = default;
+    GraphCache(const GraphCache&) = delete;
+    GraphCache& operator=(const GraphCache&) = delete;
+    ~GraphCache() { drop(); }
+    template <class F>
+    hipGraphExec_t get(hipStream_t s, const std::vector<const void*>& sig, F record) {
+        for (Entry& e : all)
+            if (e.stream == s && e.sig == sig) return e.exec;
+        if (all.size() >= 8) drop_first();
+        hipGraph_t g = nullptr;
+        SEMO_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+        try {
+            record();
+        } catch (...) {
+            (void)hipStreamEndCapture(s, &g);
+            if (g) (void)hipGraphDestroy(g);
+            throw;
+        }
+        SEMO_HIP(hipStreamEndCapture(s, &g));
+        hipGraphExec_t x = nullptr;
+        hipError_t e = hipGraphInstantiate(&x, g, nullptr, nullptr, 0);
+        (void)hipGraphDestroy(g);
+        SEMO_HIP(e);
+        all.push_back(Entry{sig, x, s});
+        return x;
+    }
+};
+
 // ------------------------------------------------------------ AMG level -----
 struct AmgLevel {
     int n = 0;
@@ -178,35 +226,21 @@ struct Amg {
     DBuf<int> l0_map;
     int iters_ref = -1, last_iters = -1;
     bool fresh = false;         // the last solve used a freshly built hierarchy
-    // one V-cycle captured as a HIP graph (replayed per Krylov iteration):
-    // valid for the hierarchy's buffers and the operands it was captured
-    // with.  vg_sig lists every device address the captured kernels take
-    // (operands, level vectors and operators), sorted: a replay whose current
-    // list differs re-captures, so a reallocated or swapped buffer is never
-    // reached through a stale graph.
-    hipGraphExec_t vg = nullptr;
-    hipStream_t vg_stream = nullptr;      // stream of the exec's launches
-    std::vector<const void*> vg_sig;
-    int vg_deg = 0, vg_prec = -1;
-    bool vg_pre = false;
-    // The exec's last launch may still be queued: wait for its stream before
-    // the exec (and, in the callers, the buffers it references) goes away.
-    void drop_graph() {
-        if (vg) {
-            if (vg_stream) (void)hipStreamSynchronize(vg_stream);
-            (void)hipGraphExecDestroy(vg);
-        }
-        vg = nullptr; vg_stream = nullptr; vg_sig.clear(); vg_prec = -1;
-    }
+    size_t builds = 0;          // set-ups so far (part of a captured V-cycle's key)
+    // the V-cycle, and Krylov iterations around it, captured as HIP graphs.
+    // A V-cycle's signature lists every device address its kernels take
+    // (operands, level vectors and operators), sorted: smoothing steps swap
+    // some levels' buffers at every pass, always among the same set.
+    GraphCache graphs;
     void reset() {
-        drop_graph();
+        graphs.drop();          // before the buffers they reference
         lv.clear(); nc_dense = 0; coarse_inv.release(); setup_ms = 0; built = false; key.clear();
         l0_map.release(); iters_ref = last_iters = -1; fresh = false;
     }
     Amg() = default;
     Amg(const Amg&) = delete;
     Amg& operator=(const Amg&) = delete;
-    ~Amg() { drop_graph(); }
+    ~Amg() { reset(); }
 };
 
 struct AdjBufs;                 // adjoint.hip: checkpoints and adjoint work arrays
@@ -347,8 +381,9 @@ struct semo_ctx {
     semo::DBuf<double> kv64;                   // Krylov work (fp64)
     semo::DBuf<float> kv32;
     semo_solve_stats last_stats_mom{}, last_stats_p{}, last_stats_vf{};
-    double* pin = nullptr;                     // pinned Krylov scalars (PIPE_*)
-    hipEvent_t pev[6] = {};
+    double* pin = nullptr;                     // ring of pinned words (ring_put)
+    semo::DBuf<int> d_seq;                     // words the device has stored
+    int seq = 0;                               // words the host has asked for
     semo::AdjBufs* adj = nullptr;
     semo::Coupled* cpl = nullptr;
     // this device's copy of the no-allocation entry point's scratch
@@ -391,33 +426,72 @@ inline double cell_faces_bytes(const semo_ctx* c, double per_face) {
         hipLaunchKernelGGL(kern, grid, block, (shmem), (c)->stream, __VA_ARGS__);           \
     } while (0)
 
-// ------------------------------------------------- Krylov convergence tests --
-// Iteration k's squared residual arrives in pinned slot k % 4 behind an event:
-// the kernel that finishes the reduction stores it there itself (pipe_slot,
-// then pipe_mark), or a copy brings it (pipe_push).  ConvCheck reads it only
-// once iteration k + 1 has been issued, so the device has queued work while
-// the host waits -- except near convergence: when the residual history
-// predicts that iteration k meets the tolerance, k is read at once (a short
-// stall instead of a wasted iteration).  Slots PIPE_BB and PIPE_END carry the
-// right-hand side's squared norm and the final true residual.
-constexpr int PIPE_BB = 4, PIPE_END = 5, PIPE_SLOTS = 6;
-inline void pipe_init(semo_ctx* c) {
+// ------------------------------------------------------ scalars to the host --
+// Scalars come to the host through a ring of pinned words that kernels store
+// into themselves (ring_put): the device counts the words it has stored, the
+// host those it has asked for (ring_expect, called before the launch), and it
+// polls a word until the value is there.  No copy, event or stream
+// synchronisation: a kernel's scalar is on the host 5-8 us after its launch,
+// against 26 us for a copy and a synchronisation.
+constexpr int RING = 1024;
+constexpr unsigned long long RING_EMPTY = 0x7FF4C3C35A5AA5A5ull;    // a signaling NaN: no computed value
+struct Ring {
+    double* __restrict__ host;      // null: nothing is sent
+    int* __restrict__ seq;
+};
+__device__ inline void ring_put(const Ring& r, const double* v, int n) {
+    if (!r.host) return;
+    int q = *r.seq;
+    for (int k = 0; k < n; ++k)
+        __hip_atomic_store(r.host + ((q + k) & (RING - 1)), v[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    *r.seq = q + n;
+}
+inline void ring_init(semo_ctx* c) {
     if (c->pin) return;
-    SEMO_HIP(hipHostMalloc((void**)&c->pin, PIPE_SLOTS * sizeof(double), hipHostMallocDefault));
-    for (hipEvent_t& e : c->pev) SEMO_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    c->d_seq.alloc(1);
+    SEMO_HIP(hipMemsetAsync(c->d_seq.p, 0, sizeof(int), c->stream));
+    SEMO_HIP(hipStreamSynchronize(c->stream));
+    SEMO_HIP(hipHostMalloc((void**)&c->pin, RING * sizeof(double), hipHostMallocDefault));
+    c->seq = 0;
 }
-inline int pipe_of(int k) { return k & 3; }              // slot of iteration k
-inline double* pipe_slot(semo_ctx* c, int slot) { pipe_init(c); return c->pin + slot; }
-inline void pipe_mark(semo_ctx* c, int slot) { SEMO_HIP(hipEventRecord(c->pev[slot], c->stream)); }
-inline double pipe_read(semo_ctx* c, int slot) {
-    SEMO_HIP(hipEventSynchronize(c->pev[slot]));
-    return ((volatile double*)c->pin)[slot];
+inline Ring ring_of(semo_ctx* c) { ring_init(c); return Ring{c->pin, c->d_seq.p}; }
+// the first of the next n words, emptied; the launch that stores them follows
+inline int ring_expect(semo_ctx* c, int n) {
+    ring_init(c);
+    int first = c->seq & (RING - 1);
+    for (int k = 0; k < n; ++k)
+        reinterpret_cast<volatile unsigned long long*>(c->pin)[(first + k) & (RING - 1)] = RING_EMPTY;
+    c->seq = (c->seq + n) & (RING - 1);
+    return first;
 }
-inline void pipe_push(semo_ctx* c, const double* dscalar, int k) {
-    int s = pipe_of(k);
-    SEMO_HIP(hipMemcpyAsync(c->pin + s, dscalar, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    pipe_mark(c, s);
+// after an error: the host's count follows the device's, whatever was issued
+inline void ring_resync(semo_ctx* c) {
+    if (!c->pin) return;
+    int q = 0;
+    if (hipMemcpyAsync(&q, c->d_seq.p, sizeof(int), hipMemcpyDeviceToHost, c->stream) == hipSuccess &&
+        hipStreamSynchronize(c->stream) == hipSuccess)
+        c->seq = q & (RING - 1);
 }
+// waits for word w: it has come, or the stream has ended (an error, or the
+// value arrived in between)
+inline double ring_read(semo_ctx* c, int w) {
+    volatile unsigned long long* p = reinterpret_cast<volatile unsigned long long*>(c->pin) + (w & (RING - 1));
+    for (;;) {
+        for (int k = 0; k < 2048; ++k) {
+            unsigned long long v = *p;
+            if (v != RING_EMPTY) {
+                double d;
+                memcpy(&d, &v, sizeof d);
+                return d;
+            }
+        }
+        hipError_t e = hipStreamQuery(c->stream);
+        if (e == hipErrorNotReady) continue;
+        SEMO_HIP(e);
+        SEMO_CHECK(*p != RING_EMPTY, SEMO_EHIP, "a scalar did not arrive from the device");
+    }
+}
+
 // Final test of a solve, on its true FP64 relative residual: a non-finite
 // residual (NaN/Inf in the system or the iterates) or one above
 // max(10 tol, 1e-12) is a failure, whatever stopped the iteration.  (The
@@ -431,24 +505,30 @@ inline void check_converged(double rel, double tol, const char* what) {
                                       std::to_string(rel) + ")");
 }
 
+// Convergence test of a Krylov loop.  Iteration k's squared residual is read
+// only once iteration k + 1 has been issued, so the device has queued work
+// while the host waits -- except near convergence: when the residual history
+// predicts that iteration k meets the tolerance, k is read at once (a short
+// stall instead of a wasted iteration).
 struct ConvCheck {
     semo_ctx* c;
     double lim;                 // stop when the squared residual <= lim (NaN stops too)
     int read = 0;               // last iteration whose residual was read
     double r1, r2 = -1.0;       // last two residuals read (r1 starts as |b|^2)
-    bool have_bb = true;
-    ConvCheck(semo_ctx* c_, double lim_, double bb) : c(c_), lim(lim_), r1(bb) { pipe_init(c_); }
-    // |b|^2 is still on its way to slot PIPE_BB: it is read, and scales the
+    int bb_word = -1, word[2] = {0, 0};
+    ConvCheck(semo_ctx* c_, double lim_, double bb) : c(c_), lim(lim_), r1(bb) {}
+    // |b|^2 is still on its way to a ring word: it is read, and scales the
     // squared relative tolerance, at the first test
-    ConvCheck(semo_ctx* c_, double tol2) : c(c_), lim(tol2), r1(0.0), have_bb(false) {}
+    ConvCheck(semo_ctx* c_, double tol2, int bb_word_) : c(c_), lim(tol2), r1(0.0), bb_word(bb_word_) {}
     double bb() {
-        if (!have_bb) { r1 = pipe_read(c, PIPE_BB); lim *= r1; have_bb = true; }
+        if (bb_word >= 0) { r1 = ring_read(c, bb_word); lim *= r1; bb_word = -1; }
         return r1;
     }
-    void take(int k) { double v = pipe_read(c, pipe_of(k)); r2 = r1; r1 = v; read = k; }
-    // after iteration `it` pushed its residual: true = stop
-    bool done(int it) {
+    void take(int k) { double v = ring_read(c, word[k & 1]); r2 = r1; r1 = v; read = k; }
+    // iteration `it`, whose residual comes to word w, was issued: true = stop
+    bool done(int it, int w) {
         bb();
+        word[it & 1] = w;
         if (read < it - 1) {
             take(it - 1);
             if (!(r1 > lim)) return true;         // it - 1 converged; `it` ran one step further
@@ -549,6 +629,14 @@ void solve_pressure(semo_ctx* c, const double* b, double* x, semo_solve_stats* s
 // keep_coarse(amg)), and one V-cycle of it
 void pressure_amg_update(semo_ctx* c, bool (*keep_coarse)(const Amg&));
 void pressure_vcycle(semo_ctx* c, const double* r64, double* z64, bool fp32);
+// its kernels one by one (to be captured with others), and what a graph that
+// holds them depends on
+void pressure_vcycle_kernels(semo_ctx* c, const double* r64, double* z64, bool fp32);
+std::vector<const void*> pressure_vcycle_signature(semo_ctx* c, const double* r64, const double* z64, bool fp32);
+// totals of nb partial pairs, summed on the device in a fixed order
+double2 sum_to_host(semo_ctx* c, int nb, const double* part);
+// the smallest of the pairs' first values
+double min_to_host(semo_ctx* c, int nb, const double* part);
 void solve_momentum(semo_ctx* c, int nrhs, semo_solve_stats* st);
 std::vector<std::vector<int>> aggregate_hierarchy(int n, const std::vector<int>& ptr, const std::vector<int>& col,
                                                   const std::vector<double>& val, int min_coarse);

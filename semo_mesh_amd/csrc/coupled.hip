@@ -56,7 +56,8 @@ struct Coupled {
     DBuf<double> im;
     DBuf<double> kv;                            // Krylov vectors
     DBuf<double> tp, zp;                        // Schur-complement right side / solution [n]
-    DBuf<double> part, red, sc;                 // host-summed partials; device partials, scalars
+    DBuf<double> red, sc;                       // reduction partials, scalars
+    GraphCache graphs;                          // a captured BiCGStab iteration
     int last_iters = 0;
     double last_relres = 0.0;
 };
@@ -373,14 +374,16 @@ __global__ void __launch_bounds__(TPB) k_cpl_update(int nc, double urf_p, double
 enum { C_RHO = 0, C_ALPHA, C_OMEGA, C_BETA, C_RR, C_BB, C_N };
 enum { F_STORE_BB = 0, F_RHO, F_ALPHA, F_OMEGA, F_RR, F_RESTART };
 
-__global__ void __launch_bounds__(TPB) k_cfinish(int nb, const double* __restrict__ part, double* __restrict__ sc,
-                                                 int what) {
+constexpr int CTPB = 1024;
+// the squared norms (|b|^2, |r|^2) also go to the host
+__global__ void __launch_bounds__(CTPB) k_cfinish(int nb, const double* __restrict__ part, double* __restrict__ sc,
+                                                  int what, Ring ring) {
     double a0 = 0.0, a1 = 0.0;
-    for (int i = threadIdx.x; i < nb; i += TPB) { a0 += part[2 * i]; a1 += part[2 * i + 1]; }
-    __shared__ double sh[2][TPB];
+    for (int i = threadIdx.x; i < nb; i += CTPB) { a0 += part[2 * i]; a1 += part[2 * i + 1]; }
+    __shared__ double sh[2][CTPB];
     sh[0][threadIdx.x] = a0; sh[1][threadIdx.x] = a1;
     __syncthreads();
-    for (int w = TPB / 2; w > 0; w >>= 1) {
+    for (int w = CTPB / 2; w > 0; w >>= 1) {
         if (threadIdx.x < w) { sh[0][threadIdx.x] += sh[0][threadIdx.x + w]; sh[1][threadIdx.x] += sh[1][threadIdx.x + w]; }
         __syncthreads();
     }
@@ -398,6 +401,7 @@ __global__ void __launch_bounds__(TPB) k_cfinish(int nb, const double* __restric
     case F_RESTART: sc[C_RR] = d0; sc[C_RHO] = 1.0; sc[C_ALPHA] = 1.0; sc[C_OMEGA] = 1.0; break;
     default: break;
     }
+    if (what == F_STORE_BB || what == F_RR) ring_put(ring, &d0, 1);
 }
 
 // p = r + beta (p - omega v)
@@ -463,21 +467,9 @@ __global__ void __launch_bounds__(TPB) k_cb_init(size_t n, const double* __restr
 int nb_of(size_t n) { return (int)std::min<size_t>((n + TPB - 1) / TPB, 2048); }
 
 
-double2 dot2(semo_ctx* c, Coupled& C, size_t n, const double* a, const double* b, const double* cc,
-             const double* d) {
-    int nb = nb_of(n);
-    SEMO_LAUNCH(c, "cpl_dot", (cc ? 32.0 : 16.0) * n, k_dot2v, dim3(nb), dim3(TPB), n, a, b, cc, d, C.part.p);
-    std::vector<double> h(2 * (size_t)nb);
-    SEMO_HIP(hipMemcpyAsync(h.data(), C.part.p, h.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    SEMO_HIP(hipStreamSynchronize(c->stream));
-    double2 r{0.0, 0.0};
-    for (int k = 0; k < nb; ++k) { r.x += h[2 * k]; r.y += h[2 * k + 1]; }
-    return r;
-}
-
 // z = P^-1 r with the SIMPLE-type factorisation (FP64 vectors, FP32
-// couplings and pressure V-cycle)
-void precond(semo_ctx* c, Coupled& C, const double* r, double* z) {
+// couplings and pressure V-cycle); captured: the V-cycle's kernels one by one
+void precond(semo_ctx* c, Coupled& C, const double* r, double* z, bool captured) {
     int n = C.n;
     const DevSell<double>& A = c->Amat;
     int64_t nv = (int64_t)c->pat.col.size();
@@ -490,7 +482,8 @@ void precond(semo_ctx* c, Coupled& C, const double* r, double* z) {
     else
         SEMO_LAUNCH(c, "cpl_precond_schur_rhs", (idx + 12.0) * nv + 60.0 * n, k_sp_schur_rhs<false>, dim3(nb),
                     dim3(TPB), n, A.sl_ptr.p, A.col.p, A.dcol.p, C.gc.p, nv, C.dd.p, r, C.im.p, C.tp.p);
-    pressure_vcycle(c, C.tp.p, C.zp.p, true);
+    if (captured) pressure_vcycle_kernels(c, C.tp.p, C.zp.p, true);
+    else pressure_vcycle(c, C.tp.p, C.zp.p, true);
     if (narrow)
         SEMO_LAUNCH(c, "cpl_precond_correct", (idx + 12.0) * nv + 84.0 * n, k_sp_correct<true>, dim3(nb),
                     dim3(TPB), n, A.sl_ptr.p, A.col.p, A.dcol.p, C.gc.p, nv, C.dd.p, r, C.im.p, C.zp.p, z);
@@ -532,7 +525,6 @@ void coupled_setup(semo_ctx* c, Coupled& C) {
     C.mrhs.alloc(3 * (size_t)n);
     C.kv.alloc(8 * 4 * (size_t)n);
     C.tp.alloc((size_t)n + 64); C.zp.alloc((size_t)n + 64);
-    C.part.alloc(2 * 2048 + 64);
     C.red.alloc(2 * (size_t)nblk(4 * (long)n) + 64);
     C.sc.alloc(16);
     C.gval.alloc(3 * nv); C.gval.zero(s);       // padding slots stay 0
@@ -583,8 +575,8 @@ void coupled_spmv(semo_ctx* c, const double* x, double* y) {
 
 // right-preconditioned BiCGStab, x0 = 0, stop at ||b - A x|| <= tol ||b||.
 // The Krylov scalars stay on the device; the host reads one residual per
-// iteration, one iteration behind (pinned slot + event), so the stream never
-// drains while it waits.  Restarted from the current iterate (true residual,
+// iteration, one iteration behind, so the stream never drains while it waits.
+// An iteration's 17 kernels and two V-cycles are one graph.  Restarted from the current iterate (true residual,
 // new shadow vector) when RESTART_AFTER iterations have not halved the
 // smallest residual seen since the last (re)start: in transients the
 // unrestarted iteration was seen to stall for hundreds of iterations.
@@ -598,54 +590,76 @@ void coupled_solve(semo_ctx* c, const double* b, double* x, semo_solve_stats* st
     double* sc = C.sc.p;
     int nbv = nblk((long)N);
     auto fin = [&](int nb, int what) {
-        SEMO_LAUNCH(c, "cpl_finish", 16.0 * nb + 8.0, k_cfinish, dim3(1), dim3(TPB), nb, C.red.p, sc, what);
+        SEMO_LAUNCH(c, "cpl_finish", 16.0 * nb + 8.0, k_cfinish, dim3(1), dim3(CTPB), nb, C.red.p, sc, what,
+                    ring_of(c));
     };
     auto dot = [&](const double* a_, const double* b_, const double* c_, const double* d_, int what) {
         int nb = nb_of(N);
         SEMO_LAUNCH(c, "cpl_dot", (c_ ? 32.0 : 16.0) * N, k_dot2v, dim3(nb), dim3(TPB), N, a_, b_, c_, d_, C.red.p);
         fin(nb, what);
     };
+    bool graph = c->graphs && !c->prof.on;
+    auto record = [&] {                                     // one iteration, one ring word (|r|^2)
+        dot(rh, r, nullptr, nullptr, F_RHO);
+        SEMO_LAUNCH(c, "cpl_bicg_p", 32.0 * N, k_cb_p, dim3(nbv), dim3(TPB), N, sc, r, v, p);
+        precond(c, C, p, ph, graph);
+        spmv64(c, C, ph, v);
+        dot(rh, v, nullptr, nullptr, F_ALPHA);
+        SEMO_LAUNCH(c, "cpl_bicg_s", 24.0 * N, k_cb_s, dim3(nbv), dim3(TPB), N, sc, r, v, sv);
+        precond(c, C, sv, sh, graph);
+        spmv64(c, C, sh, t);
+        dot(t, sv, t, t, F_OMEGA);
+        SEMO_LAUNCH(c, "cpl_bicg_x", 56.0 * N, k_cb_x, dim3(nbv), dim3(TPB), N, sc, ph, sh, sv, t, x, r, C.red.p);
+        fin(nbv, F_RR);
+    };
+    int wb = ring_expect(c, 1);
     SEMO_LAUNCH(c, "cpl_bicg_init", 48.0 * N, k_cb_init, dim3(nbv), dim3(TPB), N, b, x, r, rh, p, v, C.red.p);
     fin(nbv, F_STORE_BB);
-    double bb;
-    SEMO_HIP(hipMemcpyAsync(&bb, sc + C_BB, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    SEMO_HIP(hipStreamSynchronize(c->stream));
+    hipGraphExec_t exec = nullptr;
+    if (graph) {
+        std::vector<const void*> key = pressure_vcycle_signature(c, C.tp.p, C.zp.p, true);
+        BlkMat a = blk_mat(c, C);
+        for (const void* q : {(const void*)a.sl_ptr, (const void*)a.col, (const void*)a.dcol, (const void*)a.m,
+                              (const void*)a.p, (const void*)a.g, (const void*)a.md, (const void*)a.pd,
+                              (const void*)a.d, (const void*)C.gc.p, (const void*)C.dd.p, (const void*)C.im.p,
+                              (const void*)C.kv.p, (const void*)x, (const void*)C.red.p, (const void*)sc,
+                              (const void*)c->pin, (const void*)c->d_seq.p, reinterpret_cast<const void*>(N)})
+            key.push_back(q);
+        exec = C.graphs.get(c->stream, key, record);
+    }
     int it = 0;
-    if (bb > 0.0) {
-        double nb = std::sqrt(bb), tol = c->sp.tol_u;
-        ConvCheck cc(c, tol * tol * bb, bb);
-        double best = bb;
-        int since = 0;
-        for (it = 1; it <= c->sp.maxit_u; ++it) {
-            dot(rh, r, nullptr, nullptr, F_RHO);
-            SEMO_LAUNCH(c, "cpl_bicg_p", 32.0 * N, k_cb_p, dim3(nbv), dim3(TPB), N, sc, r, v, p);
-            precond(c, C, p, ph);
-            spmv64(c, C, ph, v);
-            dot(rh, v, nullptr, nullptr, F_ALPHA);
-            SEMO_LAUNCH(c, "cpl_bicg_s", 24.0 * N, k_cb_s, dim3(nbv), dim3(TPB), N, sc, r, v, sv);
-            precond(c, C, sv, sh);
-            spmv64(c, C, sh, t);
-            dot(t, sv, t, t, F_OMEGA);
-            SEMO_LAUNCH(c, "cpl_bicg_x", 56.0 * N, k_cb_x, dim3(nbv), dim3(TPB), N, sc, ph, sh, sv, t, x, r, C.red.p);
-            fin(nbv, F_RR);
-            pipe_push(c, sc + C_RR, it);
-            if (cc.done(it)) break;
-            if (cc.r1 < 0.25 * best) { best = cc.r1; since = 0; }       // squared residuals
-            else if (++since >= RESTART_AFTER) {
-                blk_product<1>(c, C, x, b, r, "cpl_blk_resid");
-                SEMO_LAUNCH(c, "cpl_bicg_restart", 32.0 * N, k_cb_restart, dim3(nbv), dim3(TPB), N, r, rh, p, v,
-                            C.red.p);
-                fin(nbv, F_RESTART);
-                since = 0;
-                best = cc.r1;
-            }
+    double tol = c->sp.tol_u;
+    ConvCheck cc(c, tol * tol, wb);
+    double bb = 0.0, best = 0.0;
+    int since = 0;
+    for (it = 1; it <= c->sp.maxit_u; ++it) {
+        int w = ring_expect(c, 1);
+        if (graph) SEMO_HIP(hipGraphLaunch(exec, c->stream));
+        else record();
+        if (it == 1) {
+            best = bb = cc.bb();
+            if (!(bb > 0.0)) break;                          // b = 0: that step left x = 0 (or b is not finite)
         }
+        if (cc.done(it, w)) break;
+        if (cc.r1 < 0.25 * best) { best = cc.r1; since = 0; }       // squared residuals
+        else if (++since >= RESTART_AFTER) {
+            blk_product<1>(c, C, x, b, r, "cpl_blk_resid");
+            SEMO_LAUNCH(c, "cpl_bicg_restart", 32.0 * N, k_cb_restart, dim3(nbv), dim3(TPB), N, r, rh, p, v, C.red.p);
+            fin(nbv, F_RESTART);
+            since = 0;
+            best = cc.r1;
+        }
+    }
+    if (bb > 0.0) {
         it = std::min(it, c->sp.maxit_u);
         // true residual
         blk_product<1>(c, C, x, b, r, "cpl_blk_resid");
-        double rr = dot2(c, C, N, r, r, nullptr, nullptr).x;
-        C.last_relres = std::sqrt(rr) / nb;
+        int nb = nb_of(N);
+        SEMO_LAUNCH(c, "cpl_dot", 16.0 * N, k_dot2v, dim3(nb), dim3(TPB), N, r, r, (const double*)nullptr,
+                    (const double*)nullptr, C.red.p);
+        C.last_relres = std::sqrt(sum_to_host(c, nb, C.red.p).x) / std::sqrt(bb);
     } else {
+        it = 0;
         C.last_relres = 0.0;
     }
     C.last_iters = it;
@@ -668,12 +682,8 @@ double coupled_update(semo_ctx* c) {
     int nb = nblk(c->nc);
     SEMO_LAUNCH(c, "cpl_update", 96.0 * c->nc + 16.0 * nb, k_cpl_update, dim3(nb), dim3(TPB), c->nc, c->cs.urf_p,
                 c->cs.urf_mom, c->cs.limit, C.x.p, c->P.p, c->U.p, c->V.p, c->W.p, c->red.p);
-    std::vector<double> h(2 * (size_t)nb);
-    SEMO_HIP(hipMemcpyAsync(h.data(), c->red.p, h.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    SEMO_HIP(hipStreamSynchronize(c->stream));
-    double a = 0, b = 0;
-    for (int k = 0; k < nb; ++k) { a += h[2 * k]; b += h[2 * k + 1]; }
-    return b > 0.0 ? std::sqrt(a) / std::sqrt(b) : std::sqrt(a);
+    double2 s = sum_to_host(c, nb, c->red.p);
+    return s.y > 0.0 ? std::sqrt(s.x) / std::sqrt(s.y) : std::sqrt(s.x);
 }
 
 // block COO (diagonal blocks first, then row by row) and rhs, device numbering

@@ -23,6 +23,7 @@
 // lib/amgcl/solver/idrs.hpp, fgmres.hpp).
 #include <chrono>
 #include <cmath>
+#include <limits>
 
 #include "common.hpp"
 
@@ -67,7 +68,8 @@ enum { S_RZ = 0, S_RR = 2, S_X = 6, S_ALPHA = 10, S_BETA = 11, S_OMEGA = 12,
        S_RZ2 = 24, S_ALPHA2 = 26 };   // r.z and alpha of even / odd iterations (in-kernel totals)
 
 // what the last block does with the totals d[0], d[1]
-enum { W_STORE = 0,      // s[slot] = d0, s[slot+1] = d1
+enum { W_NONE = -1,      // nothing is kept
+       W_STORE = 0,      // s[slot] = d0, s[slot+1] = d1
        W_FCG_ALPHA,      // d0 = p.Ap:  alpha = rz / p.Ap
        W_FCG_BETA,       // d0 = r.z, d1 = z.Ap: Polak-Ribiere beta, rz = d0
        W_FCG_START,      // d0 = r.z of the first direction: rz = d0, beta = 0
@@ -114,9 +116,9 @@ __device__ inline void reduce2(double (&v)[2], const Red& rd) { block_partials(v
 // ordered sum of nb partial pairs, then the scalar update `what`; one
 // 1024-thread block, so each thread streams only a few partials
 constexpr int FTPB = 1024;
-// host (optional): a pinned word that also gets d0, so that no copy follows
+// ring (optional): the host gets d0, and d1 where nput = 2
 __global__ void __launch_bounds__(FTPB) k_finish(int nb, const double* __restrict__ part, double* __restrict__ s,
-                                                 int what, int slot, double* __restrict__ host) {
+                                                 int what, int slot, Ring ring, int nput) {
     double a0 = 0.0, a1 = 0.0;
     const double2* p2 = reinterpret_cast<const double2*>(part);
     for (int i = threadIdx.x; i < nb; i += FTPB) { double2 v = p2[i]; a0 += v.x; a1 += v.y; }
@@ -133,8 +135,22 @@ __global__ void __launch_bounds__(FTPB) k_finish(int nb, const double* __restric
     if (threadIdx.x == 0) {
         double d[2] = {sh[0][0], sh[1][0]};
         finish_scalars(what, slot, d, s);
-        if (host) __hip_atomic_store(host, d[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        ring_put(ring, d, nput);
     }
+}
+
+// the smallest of the partials' first values
+__global__ void __launch_bounds__(FTPB) k_finish_min(int nb, const double* __restrict__ part, double start, Ring ring) {
+    double m = start;
+    for (int i = threadIdx.x; i < nb; i += FTPB) { double v = part[2 * (size_t)i]; m = v < m ? v : m; }
+    __shared__ double sh[FTPB];
+    sh[threadIdx.x] = m;
+    __syncthreads();
+    for (int w = FTPB / 2; w > 0; w >>= 1) {
+        if (threadIdx.x < w && sh[threadIdx.x + w] < sh[threadIdx.x]) sh[threadIdx.x] = sh[threadIdx.x + w];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) ring_put(ring, sh, 1);
 }
 
 // The totals of nb partial pairs, formed by every block of a kernel that needs
@@ -639,7 +655,7 @@ __global__ void __launch_bounds__(TPB) k_bicg_x(int n, const double* __restrict_
 // systems runs in lockstep, so every matrix pass serves all three.  Vectors
 // are [3][n] (component k at +k*n); the Krylov scalars of component k live
 // in slots Q_* + k of the device scalar array.
-enum { Q_RHO = 32, Q_ALPHA = 35, Q_OMEGA = 38, Q_BETA = 41, Q_BB = 44, Q_RR = 47, Q_MAXREL = 50 };
+enum { Q_RHO = 32, Q_ALPHA = 35, Q_OMEGA = 38, Q_BETA = 41, Q_BB = 44, Q_RR = 47 };
 enum { F3_INIT = 0, F3_ALPHA, F3_OMEGA, F3_RHO, F3_STORE };
 
 __device__ inline void block_partials6(double (&v)[6], double* __restrict__ part) {
@@ -657,8 +673,10 @@ __device__ inline void block_partials6(double (&v)[6], double* __restrict__ part
         }
 }
 
+// INIT and STORE send the three squared norms to the host, RHO the largest
+// relative one
 __global__ void __launch_bounds__(1024) k_finish6(int nb, const double* __restrict__ part, double* __restrict__ s,
-                                                  int what) {
+                                                  int what, Ring ring) {
     double a[6] = {0, 0, 0, 0, 0, 0};
     for (int i = threadIdx.x; i < nb; i += 1024)
         for (int q = 0; q < 6; ++q) a[q] += part[6 * i + q];
@@ -695,7 +713,8 @@ __global__ void __launch_bounds__(1024) k_finish6(int nb, const double* __restri
         default: s[Q_RR + k] = d[k]; break;
         }
     }
-    if (what == F3_RHO) s[Q_MAXREL] = mx;
+    if (what == F3_RHO) ring_put(ring, &mx, 1);
+    else if (what == F3_INIT || what == F3_STORE) ring_put(ring, d, 3);
 }
 
 __global__ void __launch_bounds__(TPB) k_bicg3_init(int n, const double* __restrict__ b, double* __restrict__ x,
@@ -826,10 +845,18 @@ __global__ void __launch_bounds__(TPB) k_dense_gemv(int n, const double* __restr
     if (lane == 0) y[row] = (T)acc;
 }
 
-__global__ void __launch_bounds__(TPB) k_neq(size_t n, const double* __restrict__ a, const double* __restrict__ b,
+// flag = 1 where some value of the na + nb differs from its key
+__global__ void __launch_bounds__(TPB) k_neq(size_t na, const double* __restrict__ a, const double* __restrict__ ka,
+                                             size_t nb, const double* __restrict__ b, const double* __restrict__ kb,
                                              int* __restrict__ flag) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n && a[i] != b[i]) *flag = 1;
+    if (i < na ? a[i] != ka[i] : (i - na < nb && b[i - na] != kb[i - na])) *flag = 1;
+}
+// the flag to the host, and cleared for the next comparison
+__global__ void k_flag_put(int* __restrict__ flag, Ring ring) {
+    double v = *flag;
+    *flag = 0;
+    ring_put(ring, &v, 1);
 }
 
 // --------------------------------------------------------------- V-cycle --
@@ -1025,67 +1052,41 @@ std::vector<const void*> vcycle_signature(const Amg& amg, const double* r64, con
     return s;
 }
 
+// what a graph of the V-cycle depends on: its addresses (sorted) and options
 template <class T>
-void precondition(semo_ctx* c, Amg& amg, const double* r64, double* z64, bool prepared = false,
-                  const VcDot* vd = nullptr) {
-    int deg = cheb_degree(c);
-    if (!c->graphs || c->prof.on) {
-        vcycle<T>(c, amg, 0, deg, r64, z64, prepared, vd);
-        return;
-    }
-    int prec = sizeof(T) == 4 ? 1 : 0;
-    std::vector<const void*> sig = vcycle_signature<T>(amg, r64, z64, vd);
-    if (!amg.vg || amg.vg_stream != c->stream || amg.vg_sig != sig || amg.vg_deg != deg || amg.vg_prec != prec ||
-        amg.vg_pre != prepared) {
-        amg.drop_graph();
-        hipGraph_t g = nullptr;
-        SEMO_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-        vcycle<T>(c, amg, 0, deg, r64, z64, prepared, vd);
-        SEMO_HIP(hipStreamEndCapture(c->stream, &g));
-        hipError_t e = hipGraphInstantiate(&amg.vg, g, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(g);
-        SEMO_HIP(e);
-        amg.vg_stream = c->stream; amg.vg_deg = deg; amg.vg_prec = prec; amg.vg_pre = prepared;
-        // the capture swapped some levels' x buffers (out-of-place smoothing
-        // steps): the graph holds the addresses from before the swaps, the
-        // same set
-        amg.vg_sig = vcycle_signature<T>(amg, r64, z64, vd);
-        SEMO_CHECK(amg.vg_sig == sig, SEMO_EHIP, "V-cycle capture changed its buffer set");
-    }
-    SEMO_HIP(hipGraphLaunch(amg.vg, c->stream));
+std::vector<const void*> vcycle_key(const semo_ctx* c, const Amg& amg, const double* r64, const double* z64,
+                                    bool prepared, const VcDot* vd) {
+    std::vector<const void*> s = vcycle_signature<T>(amg, r64, z64, vd);
+    for (size_t v : {(size_t)cheb_degree(c), sizeof(T), (size_t)prepared, (size_t)(vd != nullptr), amg.builds})
+        s.push_back(reinterpret_cast<const void*>(v));
+    return s;
 }
 
-double host_scalar(semo_ctx* c, int idx) {
-    double v;
-    SEMO_HIP(hipMemcpyAsync(&v, c->scal.p + idx, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    SEMO_HIP(hipStreamSynchronize(c->stream));
-    return v;
+template <class T>
+void precondition(semo_ctx* c, Amg& amg, const double* r64, double* z64) {
+    int deg = cheb_degree(c);
+    if (!c->graphs || c->prof.on) {
+        vcycle<T>(c, amg, 0, deg, r64, z64);
+        return;
+    }
+    std::vector<const void*> key = vcycle_key<T>(c, amg, r64, z64, false, nullptr);
+    hipGraphExec_t x = amg.graphs.get(c->stream, key, [&] { vcycle<T>(c, amg, 0, deg, r64, z64); });
+    SEMO_HIP(hipGraphLaunch(x, c->stream));
 }
 
 Red red_of(semo_ctx* c) { return Red{c->red.p}; }
 
 
 // sums the partials of the previous launch (nb blocks) and applies `what`
-void finish(semo_ctx* c, int nb, int what, int slot = 0, double* host = nullptr, const double* part = nullptr) {
+void finish(semo_ctx* c, int nb, int what, int slot = 0, const double* part = nullptr) {
     SEMO_LAUNCH(c, "krylov_finish", 16.0 * nb + 8.0, k_finish, dim3(1), dim3(FTPB), nb, part ? part : c->red.p,
-                c->scal.p, what, slot, host);
+                c->scal.p, what, slot, Ring{nullptr, nullptr}, 0);
 }
-// ... and its total to the host's pinned slot
-void finish_to_host(semo_ctx* c, int nb, int what, int slot, int pslot, const double* part = nullptr) {
-    finish(c, nb, what, slot, pipe_slot(c, pslot), part);
-    pipe_mark(c, pslot);
-}
-
-// grid-stride dot products a.b (+ c.d), finished as `what`
-void dot_what(semo_ctx* c, int n, const double* a, const double* b, const double* cc, const double* d, int what,
-              int slot = 0) {
-    int nb = rblk(n);
-    SEMO_LAUNCH(c, "krylov_dot", (cc ? 32.0 : 16.0) * n, k_dot, dim3(nb), dim3(TPB), n, a, b, cc, d, red_of(c));
-    finish(c, nb, what, slot);
-}
-// ... stored into s[slot], s[slot+1]
-void dot_store(semo_ctx* c, int n, const double* a, const double* b, const double* cc, const double* d, int slot) {
-    dot_what(c, n, a, b, cc, d, W_STORE, slot);
+// ... and sends d0 (and d1: nput = 2) to the host: the caller has asked for
+// the words (ring_expect)
+void finish_put(semo_ctx* c, int nb, int what, int slot = 0, const double* part = nullptr, int nput = 1) {
+    SEMO_LAUNCH(c, "krylov_finish", 16.0 * nb + 8.0, k_finish, dim3(1), dim3(FTPB), nb, part ? part : c->red.p,
+                c->scal.p, what, slot, ring_of(c), nput);
 }
 
 // y = A x with dots of y (see k_spmv_dot), for the fine-level sliced-ELL operator
@@ -1104,8 +1105,8 @@ void spmv_dot(semo_ctx* c, const DevSell<double>& A, const double* x, double* y,
 // An iteration is the V-cycle (its last step leaves z and the dots r.z, z.q),
 // the direction and its product, the update of x and r (which also writes
 // the next V-cycle's level-0 input) and the residual's way to the host: three
-// launches and a graph, with the scalars of small systems formed where they
-// are used (block_total), five with k_finish launches for large ones.  (With
+// kernels after the V-cycle's, with the scalars of small systems formed where
+// they are used (block_total), five with k_finish for large ones.  (With
 // the dots, the scalars and the residual's copy as launches of their own and
 // r_old kept, a time step took 1.18 ms at 16^3, now 0.99; at 128^3 the V-cycle's
 // last step and the dots take 32.0 us instead of 25.4 + 9.1.)
@@ -1141,47 +1142,86 @@ int fpcg(semo_ctx* c, Amg& amg, const DevSell<double>& A, const double* b, doubl
     const VcDot vd{z, r, q, part_z};
     int nbz = prep ? nbs : rblk(n);                       // blocks of the r.z, z.q partials
     bool z32 = prep && mixed;                             // z as the FP32 V-cycle leaves it
-    auto pre = [&]() {
-        const VcDot* d = prep ? &vd : nullptr;
-        if (mixed) precondition<float>(c, amg, r, z, prep, d); else precondition<double>(c, amg, r, z, prep, d);
+    const VcDot* d = prep ? &vd : nullptr;
+    const int16_t* dc = A.dcol.n ? A.dcol.p : nullptr;
+    double prep_bytes = prep ? (mixed ? 8.0 : 16.0) * n : 0.0;     // the V-cycle's b and x written
+    // iteration `it`: one ring word, its squared residual; the first is
+    // preceded by the start (one more word, |b|^2)
+    auto record = [&](int it) {
+        bool first = it == 1;
+        const double* po = (it & 1) ? p : p2;               // directions alternate between two buffers
+        double* pn = (it & 1) ? p2 : p;
+        if (first) {
+            SEMO_LAUNCH(c, "fcg_init", 16.0 * n + prep_bytes, k_fcg_init, dim3(nbr), dim3(TPB), n, b, r, Red{part_r},
+                        pp);
+            finish_put(c, nbr, W_NONE, 0, part_r);
+        }
+        if (mixed) vcycle<float>(c, amg, 0, cheb_degree(c), r, z, prep, d);
+        else vcycle<double>(c, amg, 0, cheb_degree(c), r, z, prep, d);
         if (!prep)
             SEMO_LAUNCH(c, "krylov_dot", 32.0 * n, k_dot, dim3(nbz), dim3(TPB), n, r, z, z, q, Red{part_z});
-    };
-    double prep_bytes = prep ? (mixed ? 8.0 : 16.0) * n : 0.0;     // the V-cycle's b and x written
-    SEMO_LAUNCH(c, "fcg_init", 16.0 * n + prep_bytes, k_fcg_init, dim3(nbr), dim3(TPB), n, b, r, Red{part_r}, pp);
-    finish_to_host(c, nbr, W_STORE, S_X, PIPE_BB, part_r);
-    ConvCheck cc(c, tol * tol);
-    int it = 0;
-    double bb = 0.0;
-    for (it = 1; it <= maxit; ++it) {
-        pre();
-        bool first = it == 1;
         FcgIn in{part_z, own_totals ? nbz : 0, it & 1, first ? 1 : 0};
-        if (!own_totals) finish(c, nbz, first ? W_FCG_START : W_FCG_BETA, 0, nullptr, part_z);
-        const int16_t* dc = A.dcol.n ? A.dcol.p : nullptr;
+        if (!own_totals) finish(c, nbz, first ? W_FCG_START : W_FCG_BETA, 0, part_z);
         // p = z + beta p, q = A p
         if (z32)
             SEMO_LAUNCH(c, "spmv_xpby_fp64", op_bytes(A, 3) + 4.0 * n, k_spmv_xpby<float>, dim3(nbs), dim3(TPB), n,
                         A.sl_ptr.p, A.col.p, dc, A.val.p, A.diag.p, c->scal.p, in,
-                        reinterpret_cast<const float*>(z), p, p2, q, Red{part_p});
+                        reinterpret_cast<const float*>(z), po, pn, q, Red{part_p});
         else
             SEMO_LAUNCH(c, "spmv_xpby_fp64", op_bytes(A, 4), k_spmv_xpby<double>, dim3(nbs), dim3(TPB), n, A.sl_ptr.p,
-                        A.col.p, dc, A.val.p, A.diag.p, c->scal.p, in, z, p, p2, q, Red{part_p});
-        std::swap(p, p2);
+                        A.col.p, dc, A.val.p, A.diag.p, c->scal.p, in, z, po, pn, q, Red{part_p});
         in.part = part_p;
         if (own_totals) in.nb = nbs;
-        else finish(c, nbs, W_FCG_ALPHA, 0, nullptr, part_p);
+        else finish(c, nbs, W_FCG_ALPHA, 0, part_p);
         SEMO_LAUNCH(c, "fcg_update", 48.0 * n + prep_bytes, k_fcg_update, dim3(nbr), dim3(TPB), n, c->scal.p, in, x, r,
-                    p, q, Red{part_r}, pp);
-        finish_to_host(c, nbr, W_STORE, S_RR, pipe_of(it), part_r);
+                    pn, q, Red{part_r}, pp);
+        finish_put(c, nbr, W_NONE, 0, part_r);
+    };
+    // The kernels of an iteration go out as one graph, the first iteration's
+    // with the start, the even and the odd ones' each their own.  (As a graph
+    // of the V-cycle between launches, an iteration of small systems waited
+    // for the switch between the two: five captured and three plain empty
+    // kernels take 34 us, eight captured ones 21 us.)
+    bool graph = c->graphs && !c->prof.on;
+    std::vector<const void*> key;
+    if (graph) {
+        ring_init(c);
+        key = mixed ? vcycle_key<float>(c, amg, r, z, prep, d) : vcycle_key<double>(c, amg, r, z, prep, d);
+        for (const void* a : {(const void*)A.sl_ptr.p, (const void*)A.col.p, (const void*)dc, (const void*)A.val.p,
+                              (const void*)A.diag.p, (const void*)c->scal.p, (const void*)r, (const void*)z,
+                              (const void*)p, (const void*)p2, (const void*)q, (const void*)x, (const void*)part_z,
+                              (const void*)part_p, (const void*)part_r, (const void*)c->pin,
+                              (const void*)c->d_seq.p, reinterpret_cast<const void*>((size_t)n)})
+            key.push_back(a);
+        key.push_back(nullptr);                              // b (first iteration), which iteration
+        key.push_back(nullptr);
+    }
+    hipGraphExec_t exec[3] = {};
+    auto issue = [&](int it) {
+        if (!graph) { record(it); return; }
+        int kind = it == 1 ? 0 : 1 + (it & 1);
+        if (!exec[kind]) {
+            key[key.size() - 2] = it == 1 ? b : nullptr;
+            key[key.size() - 1] = reinterpret_cast<const void*>((size_t)kind);
+            exec[kind] = amg.graphs.get(c->stream, key, [&] { record(it); });
+        }
+        SEMO_HIP(hipGraphLaunch(exec[kind], c->stream));
+    };
+    int it = 0, w = ring_expect(c, 2);
+    ConvCheck cc(c, tol * tol, w++);
+    double bb = 0.0;
+    for (it = 1; it <= maxit; ++it) {
+        issue(it);
         if (it == 1 && (bb = cc.bb()) == 0.0) { *relres = 0.0; return 0; }   // b = 0: that step left x = 0
-        if (cc.done(it)) break;
+        if (cc.done(it, w)) break;
+        if (it < maxit) w = ring_expect(c, 1);
     }
     // true residual in FP64
+    w = ring_expect(c, 1);
     SEMO_LAUNCH(c, "true_resid_fp64", op_bytes(A, 2), k_resid_norm, dim3(nbs), dim3(TPB), n, A.sl_ptr.p, A.col.p,
-                A.dcol.n ? A.dcol.p : nullptr, A.val.p, A.diag.p, x, b, Red{part_r});
-    finish_to_host(c, nbs, W_STORE, S_X, PIPE_END, part_r);
-    *relres = std::sqrt(pipe_read(c, PIPE_END)) / std::sqrt(bb);
+                dc, A.val.p, A.diag.p, x, b, Red{part_r});
+    finish_put(c, nbs, W_NONE, 0, part_r);
+    *relres = std::sqrt(ring_read(c, w)) / std::sqrt(bb);
     return std::min(it, maxit);
 }
 
@@ -1194,8 +1234,8 @@ void stage_vcycle(semo_ctx* c, Amg& amg, const double* r, double* z) {
     double* sr = c->mom_stage.p;
     double* sz = sr + n + 64;
     copy_d(c, sr, r, n);
-    if (c->sp.precision == SEMO_PREC_MIXED) precondition<float>(c, amg, sr, sz, false);
-    else precondition<double>(c, amg, sr, sz, false);
+    if (c->sp.precision == SEMO_PREC_MIXED) precondition<float>(c, amg, sr, sz);
+    else precondition<double>(c, amg, sr, sz);
     copy_d(c, z, sz, n);
 }
 
@@ -1208,14 +1248,14 @@ int bicgstab(semo_ctx* c, const DevSell<double>& A, const double* dinv, const do
     double* r = c->kv64.p; double* rh = r + ln; double* p = rh + ln; double* v = p + ln; double* sv = v + ln;
     double* t = sv + ln; double* ph = t + ln; double* sh = ph + ln;
     double* s = c->scal.p;
+    int w = ring_expect(c, 1);
     SEMO_LAUNCH(c, "bicg_init", 48.0 * n, k_bicg_init, dim3(nblk(n)), dim3(TPB), n, b, x, r, rh, p, v, red_of(c));
-    finish(c, nblk(n), W_BICG_INIT);
-    double bb = host_scalar(c, S_X);
-    if (bb == 0.0) { *relres = 0.0; return 0; }
-    double nb = std::sqrt(bb);
+    finish_put(c, nblk(n), W_BICG_INIT);
     int it;
-    ConvCheck cc(c, tol * tol * bb, bb);
+    ConvCheck cc(c, tol * tol, w);
+    double bb = 0.0;
     for (it = 1; it <= maxit; ++it) {
+        w = ring_expect(c, 1);
         SEMO_LAUNCH(c, "bicg_p", 48.0 * n, k_bicg_p, dim3(nblk(n)), dim3(TPB), n, s, r, v, dinv, p, ph);
         if (pre) stage_vcycle(c, *pre, p, ph);                            // ph = M^-1 p (AMG)
         spmv_dot(c, A, ph, v, rh, nullptr, W_BICG_ALPHA);                 // v = A ph, alpha
@@ -1224,13 +1264,16 @@ int bicgstab(semo_ctx* c, const DevSell<double>& A, const double* dinv, const do
         spmv_dot(c, A, sh, t, nullptr, sv, W_BICG_OMEGA);                 // t = A sh, omega
         SEMO_LAUNCH(c, "bicg_x", 64.0 * n, k_bicg_x, dim3(nblk(n)), dim3(TPB), n, s, ph, sh, sv, t, rh, x, r,
                     red_of(c));
-        finish(c, nblk(n), W_BICG_RHO);
-        pipe_push(c, c->scal.p + S_RR, it);
-        if (cc.done(it)) break;
+        finish_put(c, nblk(n), W_BICG_RHO);
+        if (it == 1 && (bb = cc.bb()) == 0.0) { *relres = 0.0; return 0; }   // b = 0: that step left x = 0
+        if (cc.done(it, w)) break;
     }
-    spmv<double, OP_RES>(c, A, x, b, r, "true_resid_fp64");
-    dot_store(c, n, r, r, nullptr, nullptr, S_X);
-    *relres = std::sqrt(host_scalar(c, S_X)) / nb;
+    int nbs = nblk((long)A.nslices * 64);
+    w = ring_expect(c, 1);
+    SEMO_LAUNCH(c, "true_resid_fp64", op_bytes(A, 2), k_resid_norm, dim3(nbs), dim3(TPB), n, A.sl_ptr.p, A.col.p,
+                A.dcol.n ? A.dcol.p : nullptr, A.val.p, A.diag.p, x, b, red_of(c));
+    finish_put(c, nbs, W_NONE);
+    *relres = std::sqrt(ring_read(c, w)) / std::sqrt(bb);
     return std::min(it, maxit);
 }
 
@@ -1251,7 +1294,8 @@ int bicgstab3(semo_ctx* c, const DevSell<double>& A, const double* dinv, const d
     double* part = c->red.p;
     const int16_t* dc = A.dcol.n ? A.dcol.p : nullptr;
     auto fin = [&](int blocks, int what) {
-        SEMO_LAUNCH(c, "bicg3_finish", 48.0 * blocks + 8.0, k_finish6, dim3(1), dim3(1024), blocks, part, s, what);
+        SEMO_LAUNCH(c, "bicg3_finish", 48.0 * blocks + 8.0, k_finish6, dim3(1), dim3(1024), blocks, part, s, what,
+                    ring_of(c));
     };
     auto spmv3 = [&](int mode, const double* xin, double* y, const double* a) {
         // matrix once, three gathered operands, three results, three dot operands
@@ -1267,37 +1311,35 @@ int bicgstab3(semo_ctx* c, const DevSell<double>& A, const double* dinv, const d
                                A.diag.p, xin, y, a, part);
     };
     SEMO_LAUNCH(c, "bicg3_init", 144.0 * n, k_bicg3_init, dim3(nb), dim3(TPB), n, b, x, r, rh, p, v, part);
+    int wb = ring_expect(c, 3);
     fin(nb, F3_INIT);
-    double bb[3];
-    SEMO_HIP(hipMemcpyAsync(bb, s + Q_BB, 3 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    SEMO_HIP(hipStreamSynchronize(c->stream));
     int it = 0;
-    if (bb[0] > 0.0 || bb[1] > 0.0 || bb[2] > 0.0) {
-        ConvCheck cc(c, tol * tol, 1.0);
-        for (it = 1; it <= maxit; ++it) {
-            SEMO_LAUNCH(c, "bicg3_p", 128.0 * n, k_bicg3_p, dim3(nb), dim3(TPB), n, s, r, v, dinv, p, ph);
-            if (pre)                                               // ph_k = M^-1 p_k (AMG)
-                for (int k = 0; k < 3; ++k) stage_vcycle(c, *pre, p + (size_t)k * n, ph + (size_t)k * n);
-            spmv3(0, ph, v, rh);                                   // v = A ph, rh.v
-            fin(nbs, F3_ALPHA);
-            SEMO_LAUNCH(c, "bicg3_s", 104.0 * n, k_bicg3_s, dim3(nb), dim3(TPB), n, s, r, v, dinv, sv, sh);
-            if (pre)
-                for (int k = 0; k < 3; ++k) stage_vcycle(c, *pre, sv + (size_t)k * n, sh + (size_t)k * n);
-            spmv3(1, sh, t, sv);                                   // t = A sh, t.s, t.t
-            fin(nbs, F3_OMEGA);
-            SEMO_LAUNCH(c, "bicg3_x", 192.0 * n, k_bicg3_x, dim3(nb), dim3(TPB), n, s, ph, sh, sv, t, rh, x, r, part);
-            fin(nb, F3_RHO);
-            pipe_push(c, s + Q_MAXREL, it);
-            if (cc.done(it)) break;
-        }
-        it = std::min(it, maxit);
+    ConvCheck cc(c, tol * tol, 1.0);
+    for (it = 1; it <= maxit; ++it) {
+        SEMO_LAUNCH(c, "bicg3_p", 128.0 * n, k_bicg3_p, dim3(nb), dim3(TPB), n, s, r, v, dinv, p, ph);
+        if (pre)                                               // ph_k = M^-1 p_k (AMG)
+            for (int k = 0; k < 3; ++k) stage_vcycle(c, *pre, p + (size_t)k * n, ph + (size_t)k * n);
+        spmv3(0, ph, v, rh);                                   // v = A ph, rh.v
+        fin(nbs, F3_ALPHA);
+        SEMO_LAUNCH(c, "bicg3_s", 104.0 * n, k_bicg3_s, dim3(nb), dim3(TPB), n, s, r, v, dinv, sv, sh);
+        if (pre)
+            for (int k = 0; k < 3; ++k) stage_vcycle(c, *pre, sv + (size_t)k * n, sh + (size_t)k * n);
+        spmv3(1, sh, t, sv);                                   // t = A sh, t.s, t.t
+        fin(nbs, F3_OMEGA);
+        SEMO_LAUNCH(c, "bicg3_x", 192.0 * n, k_bicg3_x, dim3(nb), dim3(TPB), n, s, ph, sh, sv, t, rh, x, r, part);
+        int w = ring_expect(c, 1);
+        fin(nb, F3_RHO);
+        if (cc.done(it, w)) break;
     }
+    it = std::min(it, maxit);
     // true residuals in FP64
+    int wr = ring_expect(c, 3);
     spmv3(2, x, r, b);
     fin(nbs, F3_STORE);
-    double rr[3];
-    SEMO_HIP(hipMemcpyAsync(rr, s + Q_RR, 3 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    SEMO_HIP(hipStreamSynchronize(c->stream));
+    double bb[3], rr[3];
+    for (int k = 0; k < 3; ++k) rr[k] = ring_read(c, wr + k);
+    for (int k = 0; k < 3; ++k) bb[k] = ring_read(c, wb + k);
+    if (!(bb[0] > 0.0 || bb[1] > 0.0 || bb[2] > 0.0)) it = 0;  // b = 0: that step left x = 0
     for (int k = 0; k < 3; ++k) {
         double rel = bb[k] > 0.0 ? std::sqrt(rr[k] / bb[k]) : 0.0;
         if (st) { st->iters[k] = bb[k] > 0.0 ? it : 0; st->rel_res[k] = rel; }
@@ -1421,17 +1463,14 @@ void amg_update(semo_ctx* c, Amg& amg, DBuf<double>& key_val, DBuf<double>& key_
     if (amg.built) {
         // device-side comparison with the values the hierarchy was built from
         DBuf<int>& flag = c->d_flag1;
-        flag.ensure(1);
-        zero_d(c, flag.p, sizeof(int));
-        size_t nv = c->Amat.val.n;
-        SEMO_LAUNCH(c, "amg_values_changed", 16.0 * nv, k_neq, dim3((unsigned)((nv + TPB - 1) / TPB)), dim3(TPB), nv,
-                    c->Amat.val.p, key_val.p, flag.p);
-        SEMO_LAUNCH(c, "amg_values_changed", 16.0 * c->nc, k_neq, dim3((unsigned)((c->nc + TPB - 1) / TPB)),
-                    dim3(TPB), (size_t)c->nc, c->Amat.diag.p, key_diag.p, flag.p);
-        int f = 0;
-        SEMO_HIP(hipMemcpyAsync(&f, flag.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-        SEMO_HIP(hipStreamSynchronize(c->stream));
-        rebuild = f != 0;
+        if (!flag.n) { flag.alloc(1); zero_d(c, flag.p, sizeof(int)); }
+        size_t nv = c->Amat.val.n, nd = (size_t)c->nc;
+        int w = ring_expect(c, 1);
+        SEMO_LAUNCH(c, "amg_values_changed", 16.0 * (nv + nd), k_neq, dim3((unsigned)((nv + nd + TPB - 1) / TPB)),
+                    dim3(TPB), nv, c->Amat.val.p, key_val.p, nd, c->Amat.diag.p, key_diag.p, flag.p);
+        SEMO_LAUNCH(c, "amg_values_changed", 16.0, k_flag_put, dim3(1), dim3(1), flag.p, ring_of(c));
+        double f = ring_read(c, w);
+        rebuild = f != 0.0;
     }
     // New values on the same pattern (a variable-density flow): refresh the
     // finest level on the device and keep the coarse levels, as long as the
@@ -1474,8 +1513,30 @@ void pressure_amg_update(semo_ctx* c, bool (*keep_coarse)(const Amg&)) {
 // FP64 in and out (the Schur-complement step of the coupled solver)
 void pressure_vcycle(semo_ctx* c, const double* r64, double* z64, bool fp32) {
     SEMO_CHECK(c->amg_p.built, SEMO_ESTATE, "pressure hierarchy not built");
-    if (fp32) precondition<float>(c, c->amg_p, r64, z64, false);
-    else precondition<double>(c, c->amg_p, r64, z64, false);
+    if (fp32) precondition<float>(c, c->amg_p, r64, z64);
+    else precondition<double>(c, c->amg_p, r64, z64);
+}
+void pressure_vcycle_kernels(semo_ctx* c, const double* r64, double* z64, bool fp32) {
+    SEMO_CHECK(c->amg_p.built, SEMO_ESTATE, "pressure hierarchy not built");
+    if (fp32) vcycle<float>(c, c->amg_p, 0, cheb_degree(c), r64, z64);
+    else vcycle<double>(c, c->amg_p, 0, cheb_degree(c), r64, z64);
+}
+std::vector<const void*> pressure_vcycle_signature(semo_ctx* c, const double* r64, const double* z64, bool fp32) {
+    return fp32 ? vcycle_key<float>(c, c->amg_p, r64, z64, false, nullptr)
+                : vcycle_key<double>(c, c->amg_p, r64, z64, false, nullptr);
+}
+
+double2 sum_to_host(semo_ctx* c, int nb, const double* part) {
+    int w = ring_expect(c, 2);
+    finish_put(c, nb, W_NONE, 0, part, 2);
+    double a = ring_read(c, w);
+    return make_double2(a, ring_read(c, w + 1));
+}
+double min_to_host(semo_ctx* c, int nb, const double* part) {
+    int w = ring_expect(c, 1);
+    SEMO_LAUNCH(c, "krylov_finish", 16.0 * nb + 8.0, k_finish_min, dim3(1), dim3(FTPB), nb, part,
+                std::numeric_limits<double>::infinity(), ring_of(c));
+    return ring_read(c, w);
 }
 
 // flexible CG: the coarse levels serve while the iteration count stays
