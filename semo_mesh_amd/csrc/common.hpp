@@ -497,10 +497,11 @@ inline double ring_read(semo_ctx* c, int w) {
 // max(10 tol, 1e-12) is a failure, whatever stopped the iteration.  (The
 // 1e-12 floor admits the FP64 round-off level of solves asked for tighter
 // tolerances.)
+inline double solve_limit(double tol) { return std::max(10.0 * tol, 1e-12); }
 inline void check_converged(double rel, double tol, const char* what) {
     if (!std::isfinite(rel))
         throw Error(SEMO_ENOCONV, std::string(what) + " solve produced a non-finite residual");
-    if (rel > std::max(10.0 * tol, 1e-12))
+    if (rel > solve_limit(tol))
         throw Error(SEMO_ENOCONV, std::string(what) + " solve did not converge (relative residual " +
                                       std::to_string(rel) + ")");
 }

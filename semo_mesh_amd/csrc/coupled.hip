@@ -580,7 +580,7 @@ void coupled_spmv(semo_ctx* c, const double* x, double* y) {
 // new shadow vector) when RESTART_AFTER iterations have not halved the
 // smallest residual seen since the last (re)start: in transients the
 // unrestarted iteration was seen to stall for hundreds of iterations.
-constexpr int RESTART_AFTER = 30;
+constexpr int RESTART_AFTER = 30, MAX_RESUMES = 3;
 void coupled_solve(semo_ctx* c, const double* b, double* x, semo_solve_stats* st) {
     SEMO_CHECK(c->cpl && c->cpl->built, SEMO_ESTATE, "no coupled system assembled");
     Coupled& C = *c->cpl;
@@ -627,40 +627,53 @@ void coupled_solve(semo_ctx* c, const double* b, double* x, semo_solve_stats* st
             key.push_back(q);
         exec = C.graphs.get(c->stream, key, record);
     }
+    // r = b - A x formed before: rh = r, p = v = 0 (F_RESTART keeps |r|^2)
+    auto restart = [&] {
+        SEMO_LAUNCH(c, "cpl_bicg_restart", 32.0 * N, k_cb_restart, dim3(nbv), dim3(TPB), N, r, rh, p, v, C.red.p);
+        fin(nbv, F_RESTART);
+    };
     int it = 0;
     double tol = c->sp.tol_u;
     ConvCheck cc(c, tol * tol, wb);
     double bb = 0.0, best = 0.0;
-    int since = 0;
-    for (it = 1; it <= c->sp.maxit_u; ++it) {
-        int w = ring_expect(c, 1);
-        if (graph) SEMO_HIP(hipGraphLaunch(exec, c->stream));
-        else record();
-        if (it == 1) {
-            best = bb = cc.bb();
-            if (!(bb > 0.0)) break;                          // b = 0: that step left x = 0 (or b is not finite)
+    C.last_relres = 0.0;
+    for (int attempt = 0;; ++attempt) {
+        int since = 0;
+        for (++it; it <= c->sp.maxit_u; ++it) {
+            int w = ring_expect(c, 1);
+            if (graph) SEMO_HIP(hipGraphLaunch(exec, c->stream));
+            else record();
+            if (it == 1) {
+                best = bb = cc.bb();
+                if (!(bb > 0.0)) break;                      // b = 0: that step left x = 0 (or b is not finite)
+            }
+            if (cc.done(it, w)) break;
+            if (cc.r1 < 0.25 * best) { best = cc.r1; since = 0; }       // squared residuals
+            else if (++since >= RESTART_AFTER) {
+                blk_product<1>(c, C, x, b, r, "cpl_blk_resid");
+                restart();
+                since = 0;
+                best = cc.r1;
+            }
         }
-        if (cc.done(it, w)) break;
-        if (cc.r1 < 0.25 * best) { best = cc.r1; since = 0; }       // squared residuals
-        else if (++since >= RESTART_AFTER) {
-            blk_product<1>(c, C, x, b, r, "cpl_blk_resid");
-            SEMO_LAUNCH(c, "cpl_bicg_restart", 32.0 * N, k_cb_restart, dim3(nbv), dim3(TPB), N, r, rh, p, v, C.red.p);
-            fin(nbv, F_RESTART);
-            since = 0;
-            best = cc.r1;
-        }
-    }
-    if (bb > 0.0) {
+        if (!(bb > 0.0)) { it = 0; break; }
         it = std::min(it, c->sp.maxit_u);
         // true residual
         blk_product<1>(c, C, x, b, r, "cpl_blk_resid");
         int nb = nb_of(N);
         SEMO_LAUNCH(c, "cpl_dot", 16.0 * N, k_dot2v, dim3(nb), dim3(TPB), N, r, r, (const double*)nullptr,
                     (const double*)nullptr, C.red.p);
-        C.last_relres = std::sqrt(sum_to_host(c, nb, C.red.p).x) / std::sqrt(bb);
-    } else {
-        it = 0;
-        C.last_relres = 0.0;
+        double rr = sum_to_host(c, nb, C.red.p).x;
+        C.last_relres = std::sqrt(rr) / std::sqrt(bb);
+        // the recurrence can run ahead of the residual (seen where a flow has
+        // become steady and the right-hand side is round-off): such a solve
+        // goes on from its iterate
+        if (!std::isfinite(rr) || C.last_relres <= solve_limit(tol) || it >= c->sp.maxit_u || attempt == MAX_RESUMES)
+            break;
+        restart();
+        cc = ConvCheck(c, tol * tol * bb, rr);
+        cc.read = it;
+        best = rr;
     }
     C.last_iters = it;
     if (st) {

@@ -181,6 +181,30 @@ def test_coupled_and_simple_share_the_fixed_point():
     b.close()
 
 
+def test_steady_channel_keeps_solving():
+    """A channel marched until its update is round-off (about 5e-16 of the
+    velocity): every solve still ends at its true residual, where the
+    recurrence alone stopped at 1.1e-7 of a 1e-8 solve (step 114)."""
+    from semo_mesh_amd.cases import channel_case, inlet_profile
+    from semo_mesh_amd.mesh import hex_mesh
+    from semo_mesh_amd.solver import GpuSolver
+    m = hex_mesh(20, 14, 16, lo=(1.0, 0.0, 0.0), hi=(5.0, 1.0, 1.0), jitter=0.1, seed=5, ref_face=False)
+    u_in = 0.3 * (1.4 * 287.05 * 300.0) ** 0.5
+    case = channel_case(u_in, dt=0.2 / u_in)
+    case.urf_mom, case.urf_p, case.urf_pu = 0.7, 0.3, 0.3
+    g = GpuSolver(0)
+    g.upload_mesh(m, reorder=True)
+    g.set_case(case)
+    g.set_solver("mixed", tol_p=1e-8, tol_u=1e-8, maxit_p=1000, maxit_u=1000)
+    g.set_field("U", np.full(m.n_cells, u_in))
+    g.set_boundary_velocity(inlet_profile(m, "xmin", u_in, amplitude=0.02, seed=5))
+    for _ in range(130):
+        norms = g.coupledPressureBased(5)
+        assert g.solve_stats("momentum")["rel_res"][0] <= 1e-7
+    g.close()
+    assert norms[-1] <= 1e-13
+
+
 def _bsr(rb, cb, blk, n):
     """The block COO as a scipy BSR matrix over interleaved (p, u, v, w)."""
     o = np.lexsort((cb, rb))
