@@ -561,6 +561,230 @@ __global__ void __launch_bounds__(TPB) k_lsq1g(
     g[3 * (size_t)i] = r0; g[3 * (size_t)i + 1] = r1; g[3 * (size_t)i + 2] = r2;
 }
 
+// ------------------------------------------- stencil passes over clusters --
+// The three stencil passes with a cluster's records staged in LDS
+// (clusters.hip): one workgroup per cluster, one lane per cell.  PIECES
+// 16-byte pieces of each record, each piece an array of its own, so that the
+// lanes' reads of one piece spread over all banks.  Same terms, same order,
+// same bits as k_grad_minmax / k_lsq1 / k_curv_kappa, which gather every
+// neighbour from the L2 in 128-byte lines (1.33M tets: 12 GB a pass, its
+// bandwidth).  Bound by LDS latency at 2 to 3 workgroups a CU.  us a pass,
+// gathered -> staged: 1.33M tets one field 348 -> 149, U, V, W 623 -> 382, five
+// fields 701 -> 660, curvature 587 -> 240; 19734 tets (latency) 23 -> 24, 60 -> 28,
+// 64 -> 31, 52 -> 21; 32^3 hexes U, V, W 28 -> 18, five fields 30 -> 19.
+struct ClusterK {
+    const int* __restrict__ cell;
+    const int* __restrict__ num;
+    const int* __restrict__ cnt;
+    const int* __restrict__ list;
+    const int* __restrict__ sl;
+    const uint16_t* __restrict__ ell;
+};
+
+extern __shared__ double2 clu_lds[];
+
+// stages the cluster's records (STRIDE pieces apart in src); returns the
+// list's length
+template <int PIECES, int STRIDE>
+__device__ inline int cluster_stage(const ClusterK& k, int b, const double* __restrict__ src) {
+    const double2* s2 = reinterpret_cast<const double2*>(src);
+    const int* list = k.list + (size_t)b * CL_LIST;
+    int m = k.cnt[b];
+    for (int q = threadIdx.x; q < PIECES * m; q += blockDim.x) {
+        int r = q / PIECES, pc = q - r * PIECES;
+        clu_lds[pc * m + r] = s2[(size_t)list[r] * STRIDE + pc];
+    }
+    return m;
+}
+// the cell's neighbours in stencil order, U at a time: get(u, place) reads a
+// neighbour's record into slot u, add(u) adds its terms
+template <int U, class Get, class Add>
+__device__ inline void cluster_walk(const ClusterK& k, size_t p, int n, Get get, Add add) {
+    static_assert(U % 2 == 0, "entry pairs");
+    const uint32_t* e = reinterpret_cast<const uint32_t*>(k.ell + k.sl[p >> 6]) + (p & 63);
+    uint32_t nx[U / 2];
+#pragma unroll
+    for (int u = 0; u < U / 2; ++u) nx[u] = 2 * u < n ? __builtin_nontemporal_load(e + 64 * u) : 0u;
+    for (int q = 0; q < n; q += U) {
+        uint32_t w[U / 2];
+#pragma unroll
+        for (int u = 0; u < U / 2; ++u) w[u] = nx[u];
+        e += 64 * (U / 2);
+#pragma unroll
+        for (int u = 0; u < U / 2; ++u) nx[u] = q + U + 2 * u < n ? __builtin_nontemporal_load(e + 64 * u) : 0u;
+#pragma unroll
+        for (int u = 0; u < U; ++u) get(u, (int)((w[u / 2] >> (16 * (u & 1))) & 0xffffu));
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (q + u < n) add(u);
+    }
+}
+
+__global__ void __launch_bounds__(TPB) k_lsq1_clu(ClusterK k, const int* __restrict__ bf_ptr,
+                                                  const int* __restrict__ bf_idx, const double* __restrict__ xph,
+                                                  const double* __restrict__ fxyz, const double* __restrict__ lsq,
+                                                  const double* __restrict__ faceR, int foff, double* __restrict__ g,
+                                                  const int* __restrict__ gate) {
+    if (gate && *gate == 0) return;
+    int b = xcd_block();
+    int m = cluster_stage<2, 2>(k, b, xph);
+    size_t p = (size_t)b * TPB + threadIdx.x;
+    int i = k.cell[p], n = k.num[p];
+    __syncthreads();
+    if (i < 0) return;
+    const double2* me = reinterpret_cast<const double2*>(xph + 4 * (size_t)i);
+    double2 m0 = me[0], m1 = me[1];
+    double xi = m0.x, yi = m0.y, zi = m1.x, ph = m1.y;
+    double t0 = 0, t1 = 0, t2 = 0;
+    constexpr int U = 8;
+    double2 r0[U], r1[U];
+    cluster_walk<U>(k, p, n, [&](int u, int j) { r0[u] = clu_lds[j]; r1[u] = clu_lds[m + j]; },
+                    [&](int u) {
+                        double dx = r0[u].x - xi, dy = r0[u].y - yi, dz = r1[u].x - zi;
+                        double wk = 1.0 / (dx * dx + dy * dy + dz * dz);
+                        double d = r1[u].y - ph;
+                        t0 += wk * dx * d; t1 += wk * dy * d; t2 += wk * dz * d;
+                    });
+    for (int q = bf_ptr[i]; q < bf_ptr[i + 1]; ++q) {
+        int f = bf_idx[q];
+        double dx = fxyz[3 * (size_t)f] - xi, dy = fxyz[3 * (size_t)f + 1] - yi, dz = fxyz[3 * (size_t)f + 2] - zi;
+        double wk = 1.0 / (dx * dx + dy * dy + dz * dz);
+        double d = faceR ? faceR[f - foff] - ph : 0.0;
+        t0 += wk * dx * d; t1 += wk * dy * d; t2 += wk * dz * d;
+    }
+    const double* C = lsq + 6 * (size_t)i;
+    double r0s = 0.0; r0s += C[0] * t0; r0s += C[1] * t1; r0s += C[2] * t2;
+    double r1s = 0.0; r1s += C[1] * t0; r1s += C[3] * t1; r1s += C[4] * t2;
+    double r2s = 0.0; r2s += C[2] * t0; r2s += C[4] * t1; r2s += C[5] * t2;
+    g[3 * (size_t)i] = r0s; g[3 * (size_t)i + 1] = r1s; g[3 * (size_t)i + 2] = r2s;
+}
+
+struct GradOut {
+    const double *bP, *bUR, *bVF;           // boundary faces' right values
+    double *gP, *gU, *gV, *gW, *gVF, *mxP, *mnP, *mxU, *mnU, *mxV, *mnV, *mxW, *mnW;
+};
+
+// gradients and bounds of the fields in MASK (bits P, U, V, W, VF) of one cell
+template <int MASK>
+__device__ inline void grad_cell_clu(const ClusterK& k, int m, size_t p, int i, int n, int nif, int nbf, int with_p,
+                                     const int* __restrict__ bf_ptr, const int* __restrict__ bf_idx,
+                                     const double* __restrict__ cpk, const double* __restrict__ fxyz,
+                                     const double* __restrict__ lsq, const GradOut& o) {
+    constexpr bool P2 = (MASK & 0xC) != 0, P3 = (MASK & 0x11) != 0;      // pieces [V, W] and [P, VF]
+    const double2* me = reinterpret_cast<const double2*>(cpk + 8 * (size_t)i);
+    double2 z2 = make_double2(0.0, 0.0);
+    double2 m0 = me[0], m1 = me[1], m2 = P2 ? me[2] : z2, m3 = P3 ? me[3] : z2;
+    double xi = m0.x, yi = m0.y, zi = m1.x;
+    double ph[5] = {m3.x, m1.y, m2.x, m2.y, m3.y};
+    double t[5][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
+    double mx[4] = {ph[0], ph[1], ph[2], ph[3]}, mn[4] = {ph[0], ph[1], ph[2], ph[3]};
+    constexpr int U = 4;
+    double2 rec[U][4];
+    cluster_walk<U>(k, p, n,
+                    [&](int u, int j) {
+                        rec[u][0] = clu_lds[j]; rec[u][1] = clu_lds[m + j];
+                        rec[u][2] = P2 ? clu_lds[2 * m + j] : z2;
+                        rec[u][3] = P3 ? clu_lds[3 * m + j] : z2;
+                    },
+                    [&](int u) {
+                        double dx = rec[u][0].x - xi, dy = rec[u][0].y - yi, dz = rec[u][1].x - zi;
+                        double wk = 1.0 / (dx * dx + dy * dy + dz * dz);
+                        double pj[5] = {rec[u][3].x, rec[u][1].y, rec[u][2].x, rec[u][2].y, rec[u][3].y};
+#pragma unroll
+                        for (int v = 0; v < 5; ++v)
+                            if (MASK >> v & 1) {
+                                double d = pj[v] - ph[v];
+                                t[v][0] += wk * dx * d; t[v][1] += wk * dy * d; t[v][2] += wk * dz * d;
+                            }
+#pragma unroll
+                        for (int v = 0; v < 4; ++v)
+                            if (MASK >> v & 1) { mx[v] = smax(mx[v], pj[v]); mn[v] = smin(mn[v], pj[v]); }
+                    });
+    for (int q = bf_ptr[i]; q < bf_ptr[i + 1]; ++q) {
+        int f = bf_idx[q];
+        int j = f - nif;
+        double dx = fxyz[3 * (size_t)f] - xi, dy = fxyz[3 * (size_t)f + 1] - yi, dz = fxyz[3 * (size_t)f + 2] - zi;
+        double wk = 1.0 / (dx * dx + dy * dy + dz * dz);
+#pragma unroll
+        for (int v = 0; v < 5; ++v)
+            if (MASK >> v & 1) {
+                double fr = v == 0 ? o.bP[j] : v == 4 ? o.bVF[j] : o.bUR[(size_t)(v - 1) * nbf + j];
+                double d = fr - ph[v];
+                t[v][0] += wk * dx * d; t[v][1] += wk * dy * d; t[v][2] += wk * dz * d;
+            }
+    }
+    const double* Cp = lsq + 6 * (size_t)i;
+    double C[6];
+#pragma unroll
+    for (int q = 0; q < 6; ++q) C[q] = Cp[q];
+    double* out[5] = {o.gP, o.gU, o.gV, o.gW, o.gVF};
+    double* omx[4] = {o.mxP, o.mxU, o.mxV, o.mxW};
+    double* omn[4] = {o.mnP, o.mnU, o.mnV, o.mnW};
+#pragma unroll
+    for (int v = 0; v < 5; ++v)
+        if (MASK >> v & 1) {
+            double r0 = 0.0; r0 += C[0] * t[v][0]; r0 += C[1] * t[v][1]; r0 += C[2] * t[v][2];
+            double r1 = 0.0; r1 += C[1] * t[v][0]; r1 += C[3] * t[v][1]; r1 += C[4] * t[v][2];
+            double r2 = 0.0; r2 += C[2] * t[v][0]; r2 += C[4] * t[v][1]; r2 += C[5] * t[v][2];
+            out[v][3 * (size_t)i] = r0; out[v][3 * (size_t)i + 1] = r1; out[v][3 * (size_t)i + 2] = r2;
+            if (v < 4 && (v > 0 || with_p)) { omx[v < 4 ? v : 0][i] = mx[v < 4 ? v : 0]; omn[v < 4 ? v : 0][i] = mn[v < 4 ? v : 0]; }
+        }
+}
+
+// Two wavefronts per 64 cells, each with some of the fields (MA, MB: field bits
+// of the first and the second four wavefronts): the records' LDS leaves two
+// workgroups a CU (one with five fields), and twice the wavefronts hide its
+// latency.
+template <int MA, int MB>
+__global__ void __launch_bounds__(2 * TPB) k_grad_minmax_clu(
+    ClusterK k, int nif, int nbf, int with_p, const int* __restrict__ bf_ptr, const int* __restrict__ bf_idx,
+    const double* __restrict__ cpk, const double* __restrict__ fxyz, const double* __restrict__ lsq, GradOut o) {
+    constexpr int PC = ((MA | MB) & 0x11) ? 4 : 3;
+    int b = xcd_block();
+    int m = cluster_stage<PC, 4>(k, b, cpk);
+    size_t p = (size_t)b * TPB + (threadIdx.x & (TPB - 1));
+    int i = k.cell[p], n = k.num[p];
+    __syncthreads();
+    if (i < 0) return;
+    if (threadIdx.x < TPB) grad_cell_clu<MA>(k, m, p, i, n, nif, nbf, with_p, bf_ptr, bf_idx, cpk, fxyz, lsq, o);
+    else grad_cell_clu<MB>(k, m, p, i, n, nif, nbf, with_p, bf_ptr, bf_idx, cpk, fxyz, lsq, o);
+}
+
+__global__ void __launch_bounds__(TPB) k_curv_kappa_clu(ClusterK k, const double* __restrict__ xn,
+                                                        const double* __restrict__ kinv, double* __restrict__ kappa) {
+    int b = xcd_block();
+    int m = cluster_stage<3, 4>(k, b, xn);
+    size_t p = (size_t)b * TPB + threadIdx.x;
+    int i = k.cell[p], n = k.num[p];
+    __syncthreads();
+    if (i < 0) return;
+    const double2* me = reinterpret_cast<const double2*>(xn + 8 * (size_t)i);
+    double2 m0 = me[0], m1 = me[1], m2 = me[2];
+    double ci[3] = {m0.x, m0.y, m1.x}, ni[3] = {m1.y, m2.x, m2.y};
+    double r[3] = {0, 0, 0};
+    constexpr int U = 4;
+    double2 o[U][3];
+    cluster_walk<U>(k, p, n,
+                    [&](int u, int j) {
+#pragma unroll
+                        for (int q = 0; q < 3; ++q) o[u][q] = clu_lds[q * m + j];
+                    },
+                    [&](int u) {
+                        double cj[3] = {o[u][0].x, o[u][0].y, o[u][1].x}, nj[3] = {o[u][1].y, o[u][2].x, o[u][2].y};
+#pragma unroll
+                        for (int a = 0; a < 3; ++a) {
+                            double d = cj[a] - ci[a];
+                            double dv = nj[a] - ni[a];
+                            r[a] += 1.0 * d * dv;
+                        }
+                    });
+    const double* v = kinv + 6 * (size_t)i;
+    double g0 = v[0] * r[0] + v[1] * r[1] + v[2] * r[2];
+    double g1 = v[1] * r[0] + v[3] * r[1] + v[4] * r[2];
+    double g2 = v[2] * r[0] + v[4] * r[1] + v[5] * r[2];
+    kappa[i] = -(g0 + g1 + g2);
+}
+
 __global__ void __launch_bounds__(TPB) k_minmax1(int nc, const int* __restrict__ st_ptr,
                                                  const int* __restrict__ st_idx, const double* __restrict__ phi,
                                                  double* __restrict__ mx, double* __restrict__ mn) {
@@ -1577,6 +1801,21 @@ double lsq1_bytes(const semo_ctx* c) {
 }
 }  // namespace
 
+namespace {
+ClusterK cluster_k(const semo_ctx* c) {
+    const Clusters& K = c->clu;
+    return ClusterK{K.cell.p, K.num.p, K.cnt.p, K.list.p, K.sl.p, K.ell.p};
+}
+// Clusters serve a pass of `pieces` 16-byte pieces a record when they were
+// built (stencil_clusters), their lists fit -- CLU_LDS bytes a workgroup at
+// most, one workgroup a CU -- and no lane count was asked for.
+constexpr size_t CLU_LDS = 100 * 1024;
+size_t cluster_lds(const semo_ctx* c, int pieces) { return 16 * (size_t)pieces * c->clu.most; }
+bool use_clusters(const semo_ctx* c, int pieces) {
+    return c->clu.ok && c->lsq_lanes == 0 && cluster_lds(c, pieces) <= CLU_LDS;
+}
+}  // namespace
+
 void fields_alloc(semo_ctx* c) {
     size_t n = c->nc, nb = c->nbf;
     for (DBuf<double>* b : {&c->P, &c->U, &c->V, &c->W, &c->VF, &c->Rho, &c->Mu, &c->oldP, &c->oldU,
@@ -1599,6 +1838,7 @@ void fields_alloc(semo_ctx* c) {
     c->cpk.alloc(8 * n);
     SEMO_LAUNCH(c, "setup_pack_xyz", 88.0 * c->nc, k_pack_xyz, dim3(nblk(c->nc)), dim3(TPB), c->nc, c->c_xyz.p,
                 c->cpk.p);
+    stencil_clusters(c);
     c->Qm3.alloc(n); c->Qm3.zero(c->stream);
     c->fVFL.alloc(std::max(c->nif, 1)); c->fVFR.alloc(std::max(c->nif, 1));
     c->c_maxA.alloc(n);
@@ -1729,7 +1969,18 @@ void grad_minmax(semo_ctx* c, bool with_p, bool uvw_only) {
                     c->f_xyz.p, c->c_lsq.p, c->bP.p, c->bUR.p, c->bVF.p, c->gP.p, c->gU.p, c->gV.p, c->gW.p, c->gVF.p,
                     c->mxP.p, c->mnP.p, c->mxU.p, c->mnU.p, c->mxV.p, c->mnV.p, c->mxW.p, c->mnW.p);
     };
-    if (narrow) {
+    auto go_clu = [&](auto kern, int pieces) {
+        double cb = bytes - (narrow ? 2.0 : 4.0) * S + 2.0 * S + 4.0 * (double)c->clu.total;
+        GradOut o{c->bP.p, c->bUR.p, c->bVF.p, c->gP.p, c->gU.p, c->gV.p, c->gW.p, c->gVF.p, c->mxP.p, c->mnP.p,
+                  c->mxU.p, c->mnU.p, c->mxV.p, c->mnV.p, c->mxW.p, c->mnW.p};
+        SEMO_LAUNCH_LDS(c, tag, cb, kern, dim3(c->clu.n), dim3(2 * TPB), cluster_lds(c, pieces), cluster_k(c), c->nif,
+                        c->nbf, (with_p && !uvw_only) ? 1 : 0, c->d_bf_ptr.p, c->d_bf_idx.p, c->cpk.p, c->f_xyz.p,
+                        c->c_lsq.p, o);
+    };
+    if (use_clusters(c, uvw_only ? 3 : 4)) {
+        if (uvw_only) go_clu(k_grad_minmax_clu<0x6, 0x8>, 3);        // U, V | W
+        else go_clu(k_grad_minmax_clu<0xE, 0x11>, 4);                // U, V, W | P, VF
+    } else if (narrow) {
         if (uvw_only) go(k_grad_minmax<3, int16_t>, c->d_st_dl.p);
         else go(k_grad_minmax<5, int16_t>, c->d_st_dl.p);
     } else {
@@ -1847,7 +2098,10 @@ void lsq1_launch(semo_ctx* c, const double* xph, const double* faceR, int foff, 
     const int* bp = c->d_bf_ptr.p;
     const int* bi = c->d_bf_idx.p;
     dim3 tb(TPB), gb(nblk((long)n * G));
-    if (c->d_st_dl.n) {
+    if (use_clusters(c, 2)) {
+        SEMO_LAUNCH_LDS(c, "lsq1", lsq1_bytes(c) + 4.0 * (double)c->clu.total, k_lsq1_clu, dim3(c->clu.n), tb,
+                        cluster_lds(c, 2), cluster_k(c), bp, bi, xph, c->f_xyz.p, c->c_lsq.p, faceR, foff, g, gate);
+    } else if (c->d_st_dl.n) {
         const int16_t* st = c->d_st_dl.p;
         if (G == 4)
             SEMO_LAUNCH(c, "lsq1", lsq1_bytes(c), (k_lsq1g<int16_t, 4, 2>), gb, tb, n, sl, st, c->d_st_ptr.p, bp, bi,
@@ -1919,7 +2173,11 @@ bool surface_tension(semo_ctx* c) {
     SEMO_LAUNCH(c, "curv_normal", 48.0 * n, k_curv_normal, gb, tb, n, 1, c->cgrad.p, c->cnrm.p);
     c->xn.ensure(8 * (size_t)n);
     SEMO_LAUNCH(c, "curv_pack", 112.0 * n, k_pack_xn, gb, tb, n, c->c_xyz.p, c->cnrm.p, c->xn.p);
-    if (c->d_st_dl.n)
+    if (use_clusters(c, 3))
+        SEMO_LAUNCH_LDS(c, "curv_kappa", 2.0 * (double)c->d_st_idx.n + 4.0 * (double)c->clu.total + 104.0 * n,
+                        k_curv_kappa_clu, dim3(c->clu.n), tb, cluster_lds(c, 3), cluster_k(c), c->xn.p, c->kinv.p,
+                        c->kappa.p);
+    else if (c->d_st_dl.n)
         SEMO_LAUNCH(c, "curv_kappa", 2.0 * (double)c->d_st_idx.n + 48.0 * n + 48.0 * n + 8.0 * n,
                     k_curv_kappa<int16_t>, gb, tb, n, c->d_st_sl.p, c->d_st_dl.p, c->xn.p, c->kinv.p, c->kappa.p);
     else

@@ -120,8 +120,8 @@ struct Profiler {
 // CSR instead (lanes > 0): sl_ptr then holds the n+1 row offsets and `lanes`
 // consecutive lanes of a wavefront share one row.
 constexpr int SL = 64;
-// lanes per cell of the one-field LSQ pass when not set: 4 from this
-// average stencil length on, else 1
+// average stencil length from which stencils count as long: the cluster passes
+// serve them at any size, and of the others 4 lanes share a cell (else 1)
 constexpr double LSQ_LANES_LONG_STENCIL = 40.0;
 // Inside a slice the entries go in pairs: pair m (entries 2m, 2m+1 of each
 // row) of the 64 rows is 128 consecutive elements, row r's two at 2r, 2r+1,
@@ -243,6 +243,20 @@ struct Amg {
     ~Amg() { reset(); }
 };
 
+// ------------------------------------------------------- stencil clusters ---
+// Workgroups of 256 cells that lie together in space (clusters.hip): the cells
+// (ascending; -1 past the last), their stencil lengths, the distinct cells
+// they and their stencils touch (CL_LIST apart, cnt of them), and the
+// stencils as 16-bit places in that list, sliced ELL in entry pairs.
+constexpr int CL_LIST = 2048;
+struct Clusters {
+    bool ok = false;            // every cluster's list fits
+    int n = 0, most = 0;        // clusters; the longest list
+    int64_t total = 0;          // list entries
+    DBuf<int> cell, num, cnt, list, sl;
+    DBuf<uint16_t> ell;
+};
+
 struct AdjBufs;                 // adjoint.hip: checkpoints and adjoint work arrays
 struct Coupled;                 // coupled.hip: block (4x4) system and its AMG
 
@@ -277,6 +291,8 @@ struct semo_ctx {
     // the same slices as int16 offsets neighbour - cell, -32768 padding; empty
     // when some neighbour lies further than 32767 from its cell
     semo::DBuf<int16_t> d_st_dl;
+    semo::Clusters clu;                    // the same stencils over compact cell clusters
+    double bb_lo[3] = {}, bb_hi[3] = {};   // bounding box of the points
     // per-face fixedValue-U values [3][nbf] (device face order), empty: the
     // patches' uniform values
     semo::DBuf<double> b_ufix;
@@ -550,6 +566,8 @@ SellPattern sell_from_csr(int n, int ncols, const std::vector<int>& ptr, const s
                           std::vector<int>* pos_of_csr);
 // geometry.hip
 void geometry_compute(semo_ctx* c);
+// clusters.hip
+void stencil_clusters(semo_ctx* c);
 // assembly.hip
 void fields_alloc(semo_ctx* c);
 void eos_transport(semo_ctx* c, const double* bR);

@@ -343,6 +343,11 @@ void mesh_setup(semo_ctx* c, const semo_mesh_desc* m, int reorder) {
     // ---- uploads
     hipStream_t s = c->stream;
     c->d_pts.upload(m->points, 3 * (size_t)np, s);
+    for (int a = 0; a < 3; ++a) c->bb_lo[a] = c->bb_hi[a] = m->points[a];
+    for (size_t k = 0; k < 3 * (size_t)np; ++k) {
+        c->bb_lo[k % 3] = std::min(c->bb_lo[k % 3], m->points[k]);
+        c->bb_hi[k % 3] = std::max(c->bb_hi[k % 3], m->points[k]);
+    }
     c->d_owner.upload(c->h_owner, s);
     c->d_nbr.upload(c->h_nbr, s);
     c->d_fptr.upload(fptr, s);
