@@ -185,75 +185,121 @@ __device__ inline void jacobian(const double (&L)[LS<NSP>::K], const double (&R)
     }
 }
 
+// Division of several numbers by the same b: y = 1 / b once, then per
+// quotient q = a y corrected by its exact remainder (Markstein, IBM J. Res.
+// Dev. 34 (1990) 111), three operations instead of a division of some twelve.
+// The quotient is a / b as rounded by the division while no step leaves the
+// normal range: the divisor is checked (div_ok), a quotient that overflows or
+// starts from a non-finite a is found by the caller among its results, which
+// are then formed again with plain divisions.  Below 1e-292 the last bit may
+// differ.
+template <bool PLAIN>
+__device__ inline double quot(double a, double b, double y) {
+    if constexpr (PLAIN) return a / b;
+    const double q = a * y;
+    return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+}
+__device__ inline bool div_ok(double b) { return fabs(b) > 0x1p-900 && fabs(b) < 0x1p900; }
+
 // GaussSeidelSOR (math.cpp:141-200), in place: A's upper triangle becomes U,
 // its strict lower triangle the multipliers L (which the reference keeps in
-// a separate matrix; the elimination never reads them back).
-template <int N>
-__device__ inline void lu_nopivot(double (&A)[N][N]) {
+// a separate matrix; the elimination never reads them back).  Y: the
+// reciprocals of U's diagonal.  False if quot needs PLAIN for one of them.
+template <int N, bool PLAIN>
+__device__ inline bool lu_nopivot(double (&A)[N][N], double (&Y)[N]) {
+    bool ok = true;
 #pragma unroll
-    for (int k = 0; k < N - 1; ++k)
+    for (int k = 0; k < N; ++k) {
+        if constexpr (!PLAIN) { Y[k] = 1.0 / A[k][k]; ok = ok && div_ok(A[k][k]); }
 #pragma unroll
         for (int i = k + 1; i < N; ++i) {
-            const double coeff = A[i][k] / A[k][k];
+            const double coeff = quot<PLAIN>(A[i][k], A[k][k], Y[k]);
 #pragma unroll
             for (int j = k + 1; j < N; ++j) A[i][j] = A[i][j] - coeff * A[k][j];
             A[i][k] = coeff;
         }
+    }
+    return ok;
 }
 
 // Column k of the inverse: forward substitution of the unit vector e_k
-// through L, back substitution through U.
-template <int N>
-__device__ inline void inverse_column(const double (&A)[N][N], int k, double (&X)[N]) {
+// through L, back substitution through U.  The zeros above row k stay zero:
+// without PLAIN their products are left out (a non-finite L shows in its own
+// column).  k_lusgs_diag keeps PLAIN: at 256 registers the second pass over a
+// cell that the check needs costs it a wavefront per SIMD.
+template <int N, bool PLAIN>
+__device__ inline void inverse_column(const double (&A)[N][N], const double (&Y)[N], int k, double (&X)[N]) {
     double Dv[N];
 #pragma unroll
     for (int i = 0; i < N; ++i) {
         Dv[i] = i == k ? 1.0 : 0.0;
 #pragma unroll
-        for (int j = 0; j < i; ++j) Dv[i] = Dv[i] - A[i][j] * Dv[j];
+        for (int j = 0; j < i; ++j)
+            if (PLAIN || j >= k) Dv[i] = Dv[i] - A[i][j] * Dv[j];
     }
-    X[N - 1] = Dv[N - 1] / A[N - 1][N - 1];
+    X[N - 1] = quot<PLAIN>(Dv[N - 1], A[N - 1][N - 1], Y[N - 1]);
 #pragma unroll
     for (int i = N - 2; i >= 0; --i) {
         X[i] = Dv[i];
 #pragma unroll
         for (int j = N - 1; j >= i + 1; --j) X[i] = X[i] - A[i][j] * X[j];
-        X[i] = X[i] / A[i][i];
+        X[i] = quot<PLAIN>(X[i], A[i][i], Y[i]);
     }
+}
+
+// use(k, X) for the columns of A's inverse; false: to be done again with PLAIN
+template <int N, bool PLAIN, class Use>
+__device__ inline bool inverse(double (&A)[N][N], Use use) {
+    double Y[N];
+    bool ok = lu_nopivot<N, PLAIN>(A, Y);
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        double X[N];
+        inverse_column<N, PLAIN>(A, Y, k, X);
+        if constexpr (!PLAIN)
+#pragma unroll
+            for (int j = 0; j < N; ++j) ok = ok && __builtin_isfinite(X[j]);
+        use(k, X);
+    }
+    return ok;
 }
 
 // calcLinearSolver (SINGLE false) / calcSingleLinearSolver (SINGLE true):
 // one thread per cell; the inverse's columns are applied as they come, which
-// is the reference's k-ordered sum sum_k Ainv[j][k] b[k].
+// is the reference's k-ordered sum sum_k Ainv[j][k] b[k].  Bound by FP64
+// arithmetic (some 2400 operations a cell with three species, 70 divisions
+// among them, against 280 bytes): with seven reciprocals in place of the
+// divisions and the substitutions' zeros left out 309,690 cells take 20.8 us
+// against 27, their bytes 14.
 template <int NSP, bool SINGLE>
 __global__ __launch_bounds__(TPB) void k_linsol_point(int n, const double* __restrict__ st, double time_step,
                                                       double* __restrict__ res) {
     constexpr int N = 4 + NSP;
     const int i = xcd_block() * TPB + (int)threadIdx.x;
     if (i >= n) return;
-    double s[LS<NSP>::K];
-    load_rec<NSP>(st, i, s);
-    double A[N][N];
-    {
-        double Pm[N][N], Tm[N][N];
-        construct<NSP>(s, Pm, Tm);
-        const double f = 1.5 * s[sDTP] / time_step;
+    double out[N];
+    auto cell = [&](auto plain) {
+        double s[LS<NSP>::K];
+        load_rec<NSP>(st, i, s);
+        double A[N][N];
+        {
+            double Pm[N][N], Tm[N][N];
+            construct<NSP>(s, Pm, Tm);
+            const double f = 1.5 * s[sDTP] / time_step;
 #pragma unroll
-        for (int a = 0; a < N; ++a)
+            for (int a = 0; a < N; ++a)
 #pragma unroll
-            for (int c = 0; c < N; ++c) A[a][c] = SINGLE ? Tm[a][c] : Pm[a][c] + f * Tm[a][c];
-    }
-    double b[N], out[N];
+                for (int c = 0; c < N; ++c) A[a][c] = SINGLE ? Tm[a][c] : Pm[a][c] + f * Tm[a][c];
+        }
+        double b[N];
 #pragma unroll
-    for (int a = 0; a < N; ++a) { b[a] = res[(size_t)i * N + a]; out[a] = 0.0; }
-    lu_nopivot<N>(A);
+        for (int a = 0; a < N; ++a) { b[a] = res[(size_t)i * N + a]; out[a] = 0.0; }
+        return inverse<N, decltype(plain)::value>(A, [&](int k, const double (&X)[N]) {
 #pragma unroll
-    for (int k = 0; k < N; ++k) {
-        double X[N];
-        inverse_column<N>(A, k, X);
-#pragma unroll
-        for (int j = 0; j < N; ++j) out[j] += X[j] * b[k];
-    }
+            for (int j = 0; j < N; ++j) out[j] += X[j] * b[k];
+        });
+    };
+    if (!cell(std::false_type{})) cell(std::true_type{});
 #pragma unroll
     for (int a = 0; a < N; ++a) res[(size_t)i * N + a] = out[a];
 }
@@ -325,14 +371,10 @@ __global__ __launch_bounds__(TPB) void k_lusgs_diag(int n, int nif, const int* _
                 M[a][c] += DS[a][c];
             }
     }
-    lu_nopivot<N>(M);
-#pragma unroll
-    for (int k = 0; k < N; ++k) {
-        double X[N];
-        inverse_column<N>(M, k, X);
+    inverse<N, true>(M, [&](int k, const double (&X)[N]) {
 #pragma unroll
         for (int j = 0; j < N; ++j) dinv[dinv_at<N>(i) + (size_t)(j * N + k) * 64] = X[j];
-    }
+    });
 }
 
 // Broadcast within each quad of lanes (DPP quad_perm): every lane gets lane

@@ -71,6 +71,31 @@ def test_linsol_vs_reference(name, reorder):
         g.close()
 
 
+@pytest.mark.parametrize("nsp", [1, 2, 3, 4])
+def test_point_blocks_outside_the_shared_reciprocals(oracle_lib, nsp):
+    """Blocks whose pivots are zero, overflow or lie outside [2^-900, 2^900]
+    take plain divisions, among cells that do not: the oracle's results,
+    infinities and NaN included."""
+    m = hex_mesh(13, 5, 4, jitter=0.1, seed=5)
+    o = oracle_lib.Oracle(m, cavity_case())
+    st = linsol_states(m, nsp, 11, vol=o.get("cell_volume"))
+    r0 = linsol_residuals(m.n_cells, nsp, 12)
+    st[::7, 8] = 0.0; st[::7, 10] = 0.0          # no compressibility: singular blocks
+    st[1::7, 5] *= 1e-290                        # density below the range
+    st[2::7, 5] *= 1e290
+    st[3::7, 7] = np.inf
+    g = _gpu(m, False)
+    try:
+        for method in ("point", "single"):
+            with np.errstate(all="ignore"):
+                ref = o.linear_solver(method, nsp, 1e-3, st, r0)
+            out = _run(g, method, 1e-3, st, r0)
+            assert not np.isfinite(ref).all() and np.isfinite(ref[4::7]).all()
+            assert np.array_equal(out, ref, equal_nan=True), method
+    finally:
+        g.close()
+
+
 @pytest.mark.parametrize("kind", ["hex20", "tet886"])
 def test_lusgs_vs_oracle(oracle_lib, kind):
     m = hex_mesh(20, 20, 20, jitter=0.1, seed=5) if kind == "hex20" else \
