@@ -146,7 +146,9 @@ struct BlkMat {
     int64_t nv;
 };
 
-// OP 0: y = A x;  OP 1: y = b - A x.  One lane per block row: a wavefront's
+// OP 0: y = A x;  OP 1: y = b - A x;  OP 2: y = A x with block partials of
+// y.w, OP 3 also of y.y (the rows are in registers: 1.05M cells 79 us and 86 /
+// 81 us with the dots, which cost 14 us each as passes of their own).  One lane per block row: a wavefront's
 // load of each of the five value arrays is one contiguous 1 KB run, a
 // neighbour costs one 32-byte gather.  Bound by HBM: 40 B per off-diagonal
 // block and 128 B per row with the vectors, against 132 B and 192 B when full
@@ -155,10 +157,17 @@ struct BlkMat {
 // rest are added in the same order.
 template <int OP, bool NARROW>
 __global__ void __launch_bounds__(TPB) k_blk(int n, BlkMat a, const double* __restrict__ x,
-                                             const double* __restrict__ b, double* __restrict__ y) {
+                                             const double* __restrict__ b, double* __restrict__ y,
+                                             const double* __restrict__ w, double* __restrict__ part) {
     int row = xcd_block() * TPB + threadIdx.x;
     int s = row >> 6, lane = row & (SL - 1);
-    if (s >= (n + SL - 1) / SL) return;
+    bool in = s < (n + SL - 1) / SL;
+    if constexpr (OP < 2) { if (!in) return; }
+    double2 wa = make_double2(0.0, 0.0), wb = wa;
+    if (OP >= 2 && row < n) {
+        wa = *reinterpret_cast<const double2*>(w + 4 * (size_t)row);
+        wb = *reinterpret_cast<const double2*>(w + 4 * (size_t)row + 2);
+    }
     double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
     if (row < n) {
         size_t N = (size_t)n;
@@ -170,10 +179,10 @@ __global__ void __launch_bounds__(TPB) k_blk(int n, BlkMat a, const double* __re
         s2 = a.d[4 * N + row] * xa.x + dm * xb.x;
         s3 = a.d[5 * N + row] * xa.x + dm * xb.y;
     }
-    int end = a.sl_ptr[s + 1];
+    int end = in ? a.sl_ptr[s + 1] : 0;
     const double* g1 = a.g + a.nv;
     const double* g2 = g1 + a.nv;
-    for (int e = a.sl_ptr[s] + 2 * lane; e < end; e += 2 * SL) {
+    for (int e = in ? a.sl_ptr[s] + 2 * lane : 0; e < end; e += 2 * SL) {
         int2 j = pat_cols<NARROW>(a.col, a.dcol, e, row);
         double2 q = *reinterpret_cast<const double2*>(a.p + e);
         double2 m = *reinterpret_cast<const double2*>(a.m + e);
@@ -193,14 +202,24 @@ __global__ void __launch_bounds__(TPB) k_blk(int n, BlkMat a, const double* __re
         s2 += c1.y * v0.x + m.y * v1.x;
         s3 += c2.y * v0.x + m.y * v1.y;
     }
-    if (row >= n) return;
+    if constexpr (OP < 2) { if (row >= n) return; }
     if constexpr (OP == 1) {
         double2 ba = *reinterpret_cast<const double2*>(b + 4 * (size_t)row);
         double2 bb = *reinterpret_cast<const double2*>(b + 4 * (size_t)row + 2);
         s0 = ba.x - s0; s1 = ba.y - s1; s2 = bb.x - s2; s3 = bb.y - s3;
     }
-    *reinterpret_cast<double2*>(y + 4 * (size_t)row) = make_double2(s0, s1);
-    *reinterpret_cast<double2*>(y + 4 * (size_t)row + 2) = make_double2(s2, s3);
+    if (OP < 2 || row < n) {
+        *reinterpret_cast<double2*>(y + 4 * (size_t)row) = make_double2(s0, s1);
+        *reinterpret_cast<double2*>(y + 4 * (size_t)row + 2) = make_double2(s2, s3);
+    }
+    if constexpr (OP >= 2) {
+        double yw = 0.0, yy = 0.0;
+        if (row < n) {
+            yw = s0 * wa.x + s1 * wa.y + s2 * wb.x + s3 * wb.y;
+            if (OP == 3) yy = s0 * s0 + s1 * s1 + s2 * s2 + s3 * s3;
+        }
+        block_sum2(yw, yy, part);
+    }
 }
 
 // ------------------------------------------ SIMPLE-type block preconditioner --
@@ -334,17 +353,12 @@ __global__ void __launch_bounds__(TPB) k_sp_correct(int n, const int* __restrict
 }
 
 // ----------------------------------------------------------- Krylov kernels --
-// two dot products, block partials (fixed order): part[2b] = a.b, part[2b+1] = c.d
-__global__ void __launch_bounds__(TPB) k_dot2v(size_t n, const double* __restrict__ a, const double* __restrict__ b,
-                                               const double* __restrict__ c, const double* __restrict__ d,
-                                               double* __restrict__ part) {
+// |a|^2, block partials (fixed order) in part[2b]
+__global__ void __launch_bounds__(TPB) k_norm2(size_t n, const double* __restrict__ a, double* __restrict__ part) {
     size_t i = (size_t)xcd_block() * blockDim.x + threadIdx.x;
-    double s0 = 0.0, s1 = 0.0;
-    for (size_t k = i; k < n; k += (size_t)gridDim.x * blockDim.x) {
-        s0 += a[k] * b[k];
-        if (c) s1 += c[k] * d[k];
-    }
-    block_sum2(s0, s1, part);
+    double s = 0.0;
+    for (size_t k = i; k < n; k += (size_t)gridDim.x * blockDim.x) s += a[k] * a[k];
+    block_sum2(s, 0.0, part);
 }
 
 // P += urf_p x0, U += urf_u x(1..3), clipped; partial sums of |dx|^2 and |x_new|^2
@@ -372,7 +386,7 @@ __global__ void __launch_bounds__(TPB) k_cpl_update(int nc, double urf_p, double
 // device scalars of the block BiCGStab (zero denominators give zero steps,
 // so that an iteration issued past convergence leaves x unchanged)
 enum { C_RHO = 0, C_ALPHA, C_OMEGA, C_BETA, C_RR, C_BB, C_N };
-enum { F_STORE_BB = 0, F_RHO, F_ALPHA, F_OMEGA, F_RR, F_RESTART };
+enum { F_STORE_BB = 0, F_ALPHA, F_OMEGA, F_RR, F_RESTART };
 
 constexpr int CTPB = 1024;
 // the squared norms (|b|^2, |r|^2) also go to the host
@@ -390,15 +404,16 @@ __global__ void __launch_bounds__(CTPB) k_cfinish(int nb, const double* __restri
     if (threadIdx.x != 0) return;
     double d0 = sh[0][0], d1 = sh[1][0];
     switch (what) {
-    case F_STORE_BB: sc[C_BB] = d0; sc[C_RR] = d0; sc[C_RHO] = 1.0; sc[C_ALPHA] = 1.0; sc[C_OMEGA] = 1.0; break;
-    case F_RHO:      // d0 = rh.r
-        sc[C_BETA] = (sc[C_RHO] != 0.0 && sc[C_OMEGA] != 0.0) ? (d0 / sc[C_RHO]) * (sc[C_ALPHA] / sc[C_OMEGA]) : 0.0;
-        sc[C_RHO] = d0;
-        break;
+    // a (re)start: rh = r, so rho = |r|^2, and p = r by beta = 0 (p = v = 0)
+    case F_STORE_BB: sc[C_BB] = d0; [[fallthrough]];
+    case F_RESTART: sc[C_RR] = d0; sc[C_RHO] = d0; sc[C_BETA] = 0.0; sc[C_OMEGA] = 1.0; break;
     case F_ALPHA: sc[C_ALPHA] = d0 != 0.0 ? sc[C_RHO] / d0 : 0.0; break;     // d0 = rh.v
     case F_OMEGA: sc[C_OMEGA] = d1 != 0.0 ? d0 / d1 : 0.0; break;            // d0 = t.s, d1 = t.t
-    case F_RR: sc[C_RR] = d0; break;
-    case F_RESTART: sc[C_RR] = d0; sc[C_RHO] = 1.0; sc[C_ALPHA] = 1.0; sc[C_OMEGA] = 1.0; break;
+    case F_RR:       // d0 = r.r, d1 = rh.r
+        sc[C_RR] = d0;
+        sc[C_BETA] = (sc[C_RHO] != 0.0 && sc[C_OMEGA] != 0.0) ? (d1 / sc[C_RHO]) * (sc[C_ALPHA] / sc[C_OMEGA]) : 0.0;
+        sc[C_RHO] = d1;
+        break;
     default: break;
     }
     if (what == F_STORE_BB || what == F_RR) ring_put(ring, &d0, 1);
@@ -418,21 +433,24 @@ __global__ void __launch_bounds__(TPB) k_cb_s(size_t n, const double* __restrict
     if (i >= n) return;
     s[i] = r[i] - sc[C_ALPHA] * v[i];
 }
-// x += alpha ph + omega sh; r = s - omega t; partials of r.r
+// x += alpha ph + omega sh; r = s - omega t; partials of r.r and of rh.r for
+// the next direction (1.05M cells: 34 us without it, 41 with; a pass of its
+// own 14 and one more finish)
 __global__ void __launch_bounds__(TPB) k_cb_x(size_t n, const double* __restrict__ sc, const double* __restrict__ ph,
                                               const double* __restrict__ sh, const double* __restrict__ s,
-                                              const double* __restrict__ t, double* __restrict__ x,
-                                              double* __restrict__ r, double* __restrict__ part) {
+                                              const double* __restrict__ t, const double* __restrict__ rh,
+                                              double* __restrict__ x, double* __restrict__ r,
+                                              double* __restrict__ part) {
     size_t i = (size_t)xcd_block() * blockDim.x + threadIdx.x;
-    double rr = 0.0;
+    double rr = 0.0, hr = 0.0;
     if (i < n) {
         double a = sc[C_ALPHA], w = sc[C_OMEGA];
         x[i] += a * ph[i] + w * sh[i];
         double ri = s[i] - w * t[i];
         r[i] = ri;
-        rr = ri * ri;
+        rr = ri * ri; hr = rh[i] * ri;
     }
-    block_sum2(rr, 0.0, part);
+    block_sum2(rr, hr, part);
 }
 // restart from the current x (r = b - A x already formed): rh = r,
 // p = v = 0; partials of r.r
@@ -497,15 +515,17 @@ BlkMat blk_mat(semo_ctx* c, const Coupled& C) {
     return BlkMat{A.sl_ptr.p, A.col.p, A.dcol.p, C.mval.p, C.pval.p, C.gval.p, C.mdiag.p, C.pdiag.p, C.dval.p,
                   (int64_t)c->pat.col.size()};
 }
-// y = A x (OP 0) or y = b - A x (OP 1)
+// y = A x (OP 0), y = b - A x (OP 1), y = A x with partials of y.w (OP 2) and
+// also of y.y (OP 3)
 template <int OP>
-void blk_product(semo_ctx* c, Coupled& C, const double* x, const double* b, double* y, const char* tag) {
+void blk_product(semo_ctx* c, Coupled& C, const double* x, const double* b, double* y, const char* tag,
+                 const double* w = nullptr) {
     bool narrow = c->Amat.dcol.p != nullptr;
     double bytes = (40.0 + (narrow ? 2.0 : 4.0)) * C.nnzb + (64.0 + 64.0 + (OP ? 32.0 : 0.0)) * C.n;
     dim3 g(nblk((long)c->pat.nslices * SL)), t(TPB);
     BlkMat a = blk_mat(c, C);
-    if (narrow) SEMO_LAUNCH(c, tag, bytes, (k_blk<OP, true>), g, t, C.n, a, x, b, y);
-    else SEMO_LAUNCH(c, tag, bytes, (k_blk<OP, false>), g, t, C.n, a, x, b, y);
+    if (narrow) SEMO_LAUNCH(c, tag, bytes, (k_blk<OP, true>), g, t, C.n, a, x, b, y, w, C.red.p);
+    else SEMO_LAUNCH(c, tag, bytes, (k_blk<OP, false>), g, t, C.n, a, x, b, y, w, C.red.p);
 }
 void spmv64(semo_ctx* c, Coupled& C, const double* x, double* y) {
     blk_product<0>(c, C, x, nullptr, y, "cpl_blk_spmv");
@@ -576,7 +596,7 @@ void coupled_spmv(semo_ctx* c, const double* x, double* y) {
 // right-preconditioned BiCGStab, x0 = 0, stop at ||b - A x|| <= tol ||b||.
 // The Krylov scalars stay on the device; the host reads one residual per
 // iteration, one iteration behind, so the stream never drains while it waits.
-// An iteration's 17 kernels and two V-cycles are one graph.  Restarted from the current iterate (true residual,
+// An iteration's 11 kernels and two V-cycles are one graph.  Restarted from the current iterate (true residual,
 // new shadow vector) when RESTART_AFTER iterations have not halved the
 // smallest residual seen since the last (re)start: in transients the
 // unrestarted iteration was seen to stall for hundreds of iterations.
@@ -593,23 +613,18 @@ void coupled_solve(semo_ctx* c, const double* b, double* x, semo_solve_stats* st
         SEMO_LAUNCH(c, "cpl_finish", 16.0 * nb + 8.0, k_cfinish, dim3(1), dim3(CTPB), nb, C.red.p, sc, what,
                     ring_of(c));
     };
-    auto dot = [&](const double* a_, const double* b_, const double* c_, const double* d_, int what) {
-        int nb = nb_of(N);
-        SEMO_LAUNCH(c, "cpl_dot", (c_ ? 32.0 : 16.0) * N, k_dot2v, dim3(nb), dim3(TPB), N, a_, b_, c_, d_, C.red.p);
-        fin(nb, what);
-    };
+    int nbp = nblk((long)c->pat.nslices * SL);              // blocks of a product
     bool graph = c->graphs && !c->prof.on;
     auto record = [&] {                                     // one iteration, one ring word (|r|^2)
-        dot(rh, r, nullptr, nullptr, F_RHO);
         SEMO_LAUNCH(c, "cpl_bicg_p", 32.0 * N, k_cb_p, dim3(nbv), dim3(TPB), N, sc, r, v, p);
         precond(c, C, p, ph, graph);
-        spmv64(c, C, ph, v);
-        dot(rh, v, nullptr, nullptr, F_ALPHA);
+        blk_product<2>(c, C, ph, nullptr, v, "cpl_blk_spmv", rh);
+        fin(nbp, F_ALPHA);
         SEMO_LAUNCH(c, "cpl_bicg_s", 24.0 * N, k_cb_s, dim3(nbv), dim3(TPB), N, sc, r, v, sv);
         precond(c, C, sv, sh, graph);
-        spmv64(c, C, sh, t);
-        dot(t, sv, t, t, F_OMEGA);
-        SEMO_LAUNCH(c, "cpl_bicg_x", 56.0 * N, k_cb_x, dim3(nbv), dim3(TPB), N, sc, ph, sh, sv, t, x, r, C.red.p);
+        blk_product<3>(c, C, sh, nullptr, t, "cpl_blk_spmv", sv);
+        fin(nbp, F_OMEGA);
+        SEMO_LAUNCH(c, "cpl_bicg_x", 64.0 * N, k_cb_x, dim3(nbv), dim3(TPB), N, sc, ph, sh, sv, t, rh, x, r, C.red.p);
         fin(nbv, F_RR);
     };
     int wb = ring_expect(c, 1);
@@ -661,8 +676,7 @@ void coupled_solve(semo_ctx* c, const double* b, double* x, semo_solve_stats* st
         // true residual
         blk_product<1>(c, C, x, b, r, "cpl_blk_resid");
         int nb = nb_of(N);
-        SEMO_LAUNCH(c, "cpl_dot", 16.0 * N, k_dot2v, dim3(nb), dim3(TPB), N, r, r, (const double*)nullptr,
-                    (const double*)nullptr, C.red.p);
+        SEMO_LAUNCH(c, "cpl_norm2", 8.0 * N, k_norm2, dim3(nb), dim3(TPB), N, r, C.red.p);
         double rr = sum_to_host(c, nb, C.red.p).x;
         C.last_relres = std::sqrt(rr) / std::sqrt(bb);
         // the recurrence can run ahead of the residual (seen where a flow has

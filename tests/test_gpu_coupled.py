@@ -165,6 +165,28 @@ def test_coupled_multilevel_solve():
     assert res <= 1e-9
 
 
+@pytest.mark.parametrize("size", [(7, 3, 3), (8, 4, 2), (13, 5, 1), (16, 8, 2), (19, 9, 3)])
+def test_coupled_solve_edges(size):
+    """The iteration's dot products ride in the products and the update: last
+    slices of 63, 64 and 1 rows, one whole block and three blocks with a
+    ragged last.  The solve stops at its tolerance 1e-10 by the recurrence;
+    the true residual may lie a few units above."""
+    from semo_mesh_amd.mesh import hex_mesh
+    mesh = hex_mesh(*size, jitter=0.1, seed=29)
+    g = _gpu(mesh, _case(), tol=1e-10)
+    g.incompressiblePressureBased(1)
+    g.assemble("coupled")
+    rb, cb, blk, rhs = g.coupled_matrix()
+    K = _expand(mesh, rb, cb, blk)
+    for _ in range(2):                       # the second with the kept graph
+        x = g.coupled_solve(rhs)
+        its = g.last_stats.iters[0]
+        res = np.linalg.norm(rhs.ravel() - K @ x.ravel()) / np.linalg.norm(rhs.ravel())
+        assert its > 0 and res <= 4e-10
+    assert not g.coupled_solve(np.zeros_like(rhs)).any()
+    g.close()
+
+
 def test_coupled_and_simple_share_the_fixed_point():
     mesh = cavity_mesh(6, jitter=0.1, seed=19)
     a = _gpu(mesh, _case(0.3))
