@@ -55,20 +55,30 @@ void need_case(semo_ctx* c) {
 }
 
 // cell arrays: caller numbering <-> device numbering
+// cell values to and from the caller's order, which the device applies
+// (k_reorder): the host copies the caller's array as it is
 void to_dev(semo_ctx* c, DBuf<double>& d, const double* h, int comps) {
-    std::vector<double> t((size_t)c->nc * comps);
-    for (int i = 0; i < c->nc; ++i)
-        for (int k = 0; k < comps; ++k) t[(size_t)i * comps + k] = h[(size_t)c->perm[i] * comps + k];
-    d.upload(t, c->stream);
-    SEMO_HIP(hipStreamSynchronize(c->stream));   // t is a temporary
+    size_t n = (size_t)c->nc * comps;
+    if (!c->d_inv.n) {
+        d.upload(h, n, c->stream);
+    } else {
+        c->io.ensure(n);
+        SEMO_HIP(hipMemcpyAsync(c->io.p, h, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+        d.alloc(n);
+        reorder_in(c, c->io.p, d.p, comps);
+    }
+    SEMO_HIP(hipStreamSynchronize(c->stream));   // h is the caller's
 }
-void from_dev(semo_ctx* c, const double* dptr, double* h, int comps, size_t stride_block = 0) {
-    std::vector<double> t((size_t)c->nc * comps);
-    SEMO_HIP(hipMemcpyAsync(t.data(), dptr, t.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+void from_dev(semo_ctx* c, const double* dptr, double* h, int comps) {
+    size_t n = (size_t)c->nc * comps;
+    const double* src = dptr;
+    if (c->d_inv.n) {
+        c->io.ensure(n);
+        reorder_out(c, c->io.p, dptr, comps);
+        src = c->io.p;
+    }
+    SEMO_HIP(hipMemcpyAsync(h, src, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     SEMO_HIP(hipStreamSynchronize(c->stream));
-    for (int i = 0; i < c->nc; ++i)
-        for (int k = 0; k < comps; ++k) h[(size_t)c->perm[i] * comps + k] = t[(size_t)i * comps + k];
-    (void)stride_block;
 }
 void face_from_dev(semo_ctx* c, const DBuf<double>& d, double* h, int comps, bool odd) {
     std::vector<double> t(d.n);

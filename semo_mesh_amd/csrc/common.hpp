@@ -275,6 +275,8 @@ struct semo_ctx {
     bool has_mesh = false;
     int np = 0, nc = 0, nf = 0, nif = 0, nbf = 0, npatch = 0;
     std::vector<int> perm, inv;            // cells: new->old, old->new
+    semo::DBuf<int> d_inv;                 // inv, where cells are renumbered
+    semo::DBuf<double> io;                 // a field in the caller's order on its way in or out
     std::vector<int> fperm;                // faces: new->old
     std::vector<int8_t> fflip;
     std::vector<int> patch_start, patch_nfaces;
@@ -629,6 +631,8 @@ double* noalloc_scratch(int device);
 void lsq1_noalloc(semo_ctx* c, const double* phi, const double* faceR_b, double* grad);
 void minmax_standalone(semo_ctx* c, const double* d_phi, double* d_mx, double* d_mn);
 void copy_d(semo_ctx* c, double* dst, const double* src, size_t n);
+void reorder_out(semo_ctx* c, double* a, const double* d, int comps);
+void reorder_in(semo_ctx* c, const double* a, double* d, int comps);
 // `bytes` bytes at p (a multiple of 4) set to zero by a kernel on the
 // context's stream, tagged "fill" (a HIP memset would run untagged)
 void zero_d(semo_ctx* c, void* p, size_t bytes);

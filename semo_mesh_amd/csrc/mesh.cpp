@@ -348,6 +348,8 @@ void mesh_setup(semo_ctx* c, const semo_mesh_desc* m, int reorder) {
         c->bb_lo[k % 3] = std::min(c->bb_lo[k % 3], m->points[k]);
         c->bb_hi[k % 3] = std::max(c->bb_hi[k % 3], m->points[k]);
     }
+    if (reorder) c->d_inv.upload(c->inv, s);
+    else c->d_inv.release();
     c->d_owner.upload(c->h_owner, s);
     c->d_nbr.upload(c->h_nbr, s);
     c->d_fptr.upload(fptr, s);

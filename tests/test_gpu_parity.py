@@ -450,3 +450,27 @@ def test_gauss_green_vs_reference(name, reorder):
         else:
             assert np.array_equal(a, b), f
     g.close()
+
+
+@pytest.mark.parametrize("reorder", [False, True])
+@pytest.mark.parametrize("size", [(2, 1, 1), (16, 16, 1), (257, 1, 1), (19, 9, 3)])
+def test_fields_keep_the_callers_order(size, reorder):
+    """A field set and read back is the caller's, bit for bit; three
+    components of a cell (centres, which the mesh orders itself) come back
+    with their cell."""
+    from semo_mesh_amd.mesh import hex_mesh
+    from semo_mesh_amd.solver import GpuSolver
+    m = hex_mesh(*size)
+    g = GpuSolver(0)
+    g.upload_mesh(m, reorder=reorder)
+    a = np.random.default_rng(5).standard_normal(m.n_cells)
+    a[0] = -0.0
+    g.set_field("P", a); g.set_field("U", -a)
+    assert g.get_field("P").tobytes() == a.tobytes() and g.get_field("U").tobytes() == (-a).tobytes()
+    perm, inv = g.permutation()
+    assert reorder or np.array_equal(perm, np.arange(m.n_cells))
+    x = g.get_field("cell_xyz")
+    i = np.arange(m.n_cells)
+    ref = (np.stack([i % size[0], i // size[0] % size[1], i // (size[0] * size[1])], 1) + 0.5) / np.array(size)
+    g.close()
+    np.testing.assert_allclose(x, ref, rtol=0, atol=1e-12)
