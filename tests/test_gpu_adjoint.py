@@ -23,7 +23,7 @@ import numpy as np
 import pytest
 
 from semo_mesh_amd.cases import cavity_case
-from semo_mesh_amd.mesh import cavity_mesh
+from semo_mesh_amd.mesh import cavity_mesh, hex_mesh
 
 pytestmark = pytest.mark.gpu
 
@@ -190,6 +190,42 @@ def test_adjoint_vs_cpu_adjoint(oracle_lib, n, physics):
           f"max |dJ/dalpha| {np.abs(gc).max():.3e}")
     assert abs(J - Jc) <= 1e-10 * abs(Jc)
     assert rel <= 1e-10
+
+
+@pytest.mark.parametrize("size", [(7, 3, 3), (16, 4, 4), (19, 9, 3)])
+def test_adjoint_edges_vs_cpu_adjoint(oracle_lib, size):
+    """The stencil passes' last slices (63, 64 and 1 cells), stencils of 7 to
+    26 neighbours; bar as above."""
+    mesh = hex_mesh(*size, jitter=0.1, seed=41)
+    alpha = 10.0 * np.random.default_rng(7).random(mesh.n_cells)
+    g = _gpu(mesh, _case(), alpha, reorder=False)
+    J, grad = g.adjointAlphaP(3, W)
+    g.close()
+    o = oracle_lib.AdjointOracle(mesh, _case())
+    o.set_solver(1e-14, 20000)
+    o.set("alphaP", alpha)
+    Jc, gc = o.adjoint(3, W)
+    assert abs(J - Jc) <= 1e-10 * abs(Jc)
+    assert np.linalg.norm(grad - gc) <= 1e-10 * np.linalg.norm(gc)
+
+
+def test_adjoint_of_far_neighbours():
+    """Layers of 33,124 cells, not renumbered: 32-bit stencil indices, where
+    the renumbered mesh has 16-bit offsets.  Each to solves of 1e-12, whose
+    error the pressure system's condition (below 1e4 over two layers)
+    multiplies."""
+    mesh = hex_mesh(182, 182, 2, jitter=0.1, seed=43)
+    alpha = 10.0 * np.random.default_rng(9).random(mesh.n_cells)
+    out = []
+    for reorder in (False, True):
+        g = _gpu(mesh, _case(), alpha, reorder)
+        g.set_solver("fp64", tol_p=1e-12, tol_u=1e-12, maxit_p=300, maxit_u=1000)
+        out.append(g.adjointAlphaP(2, W))
+        g.close()
+    (ja, ga), (jb, gb) = out
+    print("J", ja, jb, "gradient rel L2", np.linalg.norm(ga - gb) / np.linalg.norm(gb))
+    assert abs(ja - jb) <= 1e-8 * abs(jb)
+    assert np.linalg.norm(ga - gb) <= 1e-8 * np.linalg.norm(gb)
 
 
 def test_darcy_term_definition():
