@@ -381,9 +381,10 @@ __global__ void __launch_bounds__(TPB) k_adj_mom_cell(
 
 // ----------------------------------------------- LSQ + stencil bounds reverse --
 // arg max / arg min over {i} + stencil(i) with the forward's tie rule (the
-// first maximum in stencil order, the cell itself first).  One pass over the stencil in its sliced-ELL layout for all NB fields, four
-// neighbours' values requested together: 262,144 cells 91 us (a pass per
-// field over the CSR list) -> 33 us, 29 for three fields.
+// first maximum in stencil order, the cell itself first).  One pass over the
+// stencil in its sliced-ELL layout for all NB fields, four neighbours' values
+// requested together: 262,144 cells 91 us (a pass per field over the CSR list)
+// -> 33 us, 29 for three fields.
 template <class IDX>
 __device__ inline int st_cell(const IDX* __restrict__ st_ell, int e, int end, int i) {
     if (e >= end) return -1;

@@ -596,10 +596,11 @@ void coupled_spmv(semo_ctx* c, const double* x, double* y) {
 // right-preconditioned BiCGStab, x0 = 0, stop at ||b - A x|| <= tol ||b||.
 // The Krylov scalars stay on the device; the host reads one residual per
 // iteration, one iteration behind, so the stream never drains while it waits.
-// An iteration's 11 kernels and two V-cycles are one graph.  Restarted from the current iterate (true residual,
-// new shadow vector) when RESTART_AFTER iterations have not halved the
-// smallest residual seen since the last (re)start: in transients the
-// unrestarted iteration was seen to stall for hundreds of iterations.
+// An iteration's 12 kernels and two V-cycles are one graph.  Restarted from
+// the current iterate (true residual, new shadow vector) when RESTART_AFTER
+// iterations have not halved the smallest residual seen since the last
+// (re)start: in transients the unrestarted iteration was seen to stall for
+// hundreds of iterations.
 constexpr int RESTART_AFTER = 30, MAX_RESUMES = 3;
 void coupled_solve(semo_ctx* c, const double* b, double* x, semo_solve_stats* st) {
     SEMO_CHECK(c->cpl && c->cpl->built, SEMO_ESTATE, "no coupled system assembled");

@@ -1,0 +1,67 @@
+"""The pressure solver's flexible CG at the sizes where its scalars change
+hands, and the host's ring of residuals past its end."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _system(n, width, seed):
+    """Five-point Laplacian plus 1e-2 on n cells in rows of `width`."""
+    rng = np.random.default_rng(seed)
+    r, c, v = [], [], []
+    diag = np.full(n, 1e-2)
+    for off in (1, width):
+        i = np.arange(n - off)
+        if off == 1:
+            i = i[(i + 1) % width != 0]
+        w = 1.0 + 0.2 * rng.random(i.size)
+        for a, b in ((i, i + off), (i + off, i)):
+            r.append(a); c.append(b); v.append(-w)
+        diag += np.bincount(i, w, n) + np.bincount(i + off, w, n)
+    r.append(np.arange(n)); c.append(np.arange(n)); v.append(diag)
+    return np.concatenate(r), np.concatenate(c), np.concatenate(v), rng.standard_normal(n)
+
+
+def _solver(precision):
+    from semo_mesh_amd.cases import cavity_case
+    from semo_mesh_amd.mesh import hex_mesh
+    from semo_mesh_amd.solver import GpuSolver
+    g = GpuSolver(0)
+    g.upload_mesh(hex_mesh(2, 2, 2))
+    g.set_case(cavity_case())
+    g.set_solver(precision, tol_p=1e-9, tol_u=1e-9, maxit_p=200, maxit_u=200)
+    return g
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("n", [262079, 262144, 262145, 262401])
+def test_totals_on_both_sides_of_the_block_limit(n, precision):
+    """Up to 1024 blocks of 256 rows each block sums the partials itself,
+    beyond a kernel does.  The recurrence stops at 1e-9; its distance from the
+    true residual is round-off of the iterates, far below a factor of 2."""
+    r, c, v, b = _system(n, 509, 3)
+    g = _solver(precision)
+    x = g.solveAMGCL("pressure", r, c, v, b)
+    its = g.last_stats.iters[0]
+    g.close()
+    res = np.linalg.norm(b - np.bincount(r, v * x[c], n)) / np.linalg.norm(b)
+    print(n, precision, its, res)
+    assert 2 < its < 60 and res <= 2e-9
+
+
+def test_ring_of_residuals_wraps():
+    """Solves until well over 1024 residuals have passed through the ring:
+    each gives the first one's bits."""
+    r, c, v, b = _system(3001, 53, 5)
+    g = _solver("fp64")
+    first, total = None, 0
+    for _ in range(400):
+        x = g.solveAMGCL("pressure", r, c, v, b)
+        total += g.last_stats.iters[0]
+        first = x if first is None else first
+        assert np.array_equal(x, first)
+        if total > 2500:
+            break
+    g.close()
+    assert total > 1100
