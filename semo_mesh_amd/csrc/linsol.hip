@@ -398,6 +398,7 @@ constexpr int LS_POLL_LIMIT = 1 << 23;
 // of a block, 256 bytes apart, then the error word
 constexpr int LS_STEP = 64, LS_WAVES = TPB / 64, LS_ERR = 2 * LS_WAVES * LS_STEP, LS_CTL = LS_ERR + LS_STEP;
 
+// the results emptied, tickets and error word cleared: max(n, LS_CTL) threads
 __global__ __launch_bounds__(TPB) void k_lusgs_empty(size_t n, unsigned long long* __restrict__ v,
                                                      int* __restrict__ ctl) {
     size_t k = (size_t)blockIdx.x * TPB + threadIdx.x;
@@ -676,7 +677,7 @@ void linsol_run(semo_ctx* c, int method, double time_step, const double* st, dou
     const size_t nv = (size_t)N * n;
     c->ls_out.ensure(2 * nv);
     c->ls_ctl.ensure(LS_CTL);
-    SEMO_LAUNCH(c, "lusgs_empty", 16.0 * nv, k_lusgs_empty, dim3(nblk(2 * (long)nv)), b, 2 * nv,
+    SEMO_LAUNCH(c, "lusgs_empty", 16.0 * nv, k_lusgs_empty, dim3(nblk(std::max(2 * (long)nv, (long)LS_CTL))), b, 2 * nv,
                 reinterpret_cast<unsigned long long*>(c->ls_out.p), c->ls_ctl.p);
     // per cell: record, Dinv, own residual read + write, slot record; per
     // earlier (later) neighbour: its record and residual, the face's normal

@@ -117,6 +117,25 @@ def test_lusgs_vs_oracle(oracle_lib, kind):
             assert np.array_equal(out, ref)
 
 
+@pytest.mark.parametrize("nsp", [1, 2, 3, 4])
+@pytest.mark.parametrize("size", [(2, 1, 1), (2, 2, 2), (5, 5, 1), (13, 2, 1), (17, 3, 1), (13, 2, 2)])
+def test_lusgs_of_a_few_cells(oracle_lib, size, nsp):
+    """2 to 52 cells, fewer result values than the sweeps have control words:
+    every call on a context starts from cleared tickets, other states in the
+    middle one."""
+    m = hex_mesh(*size, jitter=0.1, seed=5)
+    o = oracle_lib.Oracle(m, cavity_case())
+    vol = o.get("cell_volume")
+    g = _gpu(m, False)
+    try:
+        for seed in (11, 13, 11):
+            st, r0 = linsol_states(m, nsp, seed, vol=vol), linsol_residuals(m.n_cells, nsp, seed + 1)
+            ref = o.linear_solver("lusgs", nsp, 1e-3, st, r0)
+            assert np.array_equal(g.calcLinearSolverLUSGS(1e-3, st, r0), ref)
+    finally:
+        g.close()
+
+
 def test_lusgs_large_vs_oracle(oracle_lib):
     """96^3 jittered hex (884,736 cells), both storage orders against the
     oracle's sequential sweeps."""
