@@ -156,14 +156,15 @@ struct DevSell {
 // few numbers) they were captured with: a lookup with another signature
 // captures anew, so a reallocated buffer is never reached through a stale
 // graph.  Dropped -- after the stream that may still run one -- with the
-// buffers' owner; at most eight are kept.
+// buffers' owner; at most eight are kept, the ones used last: a solve holds up
+// to three of them over the captures of the others.
 struct GraphCache {
     struct Entry {
         std::vector<const void*> sig;
         hipGraphExec_t exec;
         hipStream_t stream;
     };
-    std::vector<Entry> all;
+    std::vector<Entry> all;         // by last use
     void drop_first() {
         (void)hipStreamSynchronize(all.front().stream);
         (void)hipGraphExecDestroy(all.front().exec);
@@ -176,8 +177,11 @@ struct GraphCache {
     ~GraphCache() { drop(); }
     template <class F>
     hipGraphExec_t get(hipStream_t s, const std::vector<const void*>& sig, F record) {
-        for (Entry& e : all)
-            if (e.stream == s && e.sig == sig) return e.exec;
+        for (auto e = all.begin(); e != all.end(); ++e)
+            if (e->stream == s && e->sig == sig) {
+                std::rotate(e, e + 1, all.end());
+                return all.back().exec;
+            }
         if (all.size() >= 8) drop_first();
         hipGraph_t g = nullptr;
         SEMO_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
