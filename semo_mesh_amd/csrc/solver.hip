@@ -1197,6 +1197,11 @@ int fpcg(semo_ctx* c, Amg& amg, const DevSell<double>& A, const double* b, doubl
                               (const void*)part_p, (const void*)part_r, (const void*)c->pin,
                               (const void*)c->d_seq.p, reinterpret_cast<const void*>((size_t)n)})
             key.push_back(a);
+        // where an iteration leaves the next one's V-cycle its b and start: the
+        // V-cycle's own list is sorted, and smoothing of another degree swaps
+        // the level's x with a work array
+        for (const void* a : {(const void*)pp.b32, (const void*)pp.x32, (const void*)pp.b64, (const void*)pp.x64})
+            key.push_back(a);
         key.push_back(nullptr);                              // b (first iteration), which iteration
         key.push_back(nullptr);
     }

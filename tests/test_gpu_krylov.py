@@ -65,3 +65,45 @@ def test_ring_of_residuals_wraps():
             break
     g.close()
     assert total > 1100
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_smoother_degree_changed_between_solves(precision):
+    """Iterations are kept as graphs that hand the next V-cycle its start, and
+    degree-2 smoothing swaps the buffers it lies in.  Whatever was solved
+    before, with one or two iterations (not every graph captured) or more, a
+    solve from the same state gives the first one's bits."""
+    from semo_mesh_amd.cases import cavity_case
+    from semo_mesh_amd.mesh import cavity_mesh
+    from semo_mesh_amd.solver import GpuSolver
+    m = cavity_mesh(16, jitter=0.1, seed=29)
+    rng = np.random.default_rng(3)
+    state = {f: 1e-2 * rng.standard_normal(m.n_cells) for f in "PUVW"}
+
+    def solve(g, degree, tol=1e-10):
+        for f, v in state.items():
+            g.set_field(f, v)
+        g.set_solver(precision, tol_p=tol, tol_u=1e-10, maxit_p=200, maxit_u=200, cheb_degree=degree)
+        g.calcPressureEq()
+        assert g.last_stats.n_levels >= 2
+        return g.last_stats.iters[0], g.get_field("P")
+
+    def fresh(history, degree):
+        g = GpuSolver(0)
+        g.upload_mesh(m, reorder=True)
+        g.set_case(cavity_case())
+        g.set_solver(precision, tol_p=1e-10, tol_u=1e-10, cheb_degree=5)
+        g.incompressiblePressureBased(1)
+        for d, tol in history:
+            its, _ = solve(g, d, tol)
+            print(d, tol, its)
+        out = solve(g, degree)
+        g.close()
+        return out
+
+    for history in ([(1, 0.09), (2, 0.09)], [(1, 0.3), (2, 0.3)], [(1, 0.3), (2, 1e-10)],
+                    [(2, 0.3), (1, 0.09), (3, 0.09)], [(d, t) for t in (0.3, 1e-10) for d in (1, 2, 3, 4, 1)]):
+        for degree in (1, 2):
+            its, p = fresh([], degree)
+            got, q = fresh(history, degree)
+            assert 3 < its < 60 and got == its and np.array_equal(p, q), (history, degree, its, got)
