@@ -661,7 +661,7 @@ void coupled_solve(semo_ctx* c, const double* b, double* x, semo_solve_stats* st
             else record();
             if (it == 1) {
                 best = bb = cc.bb();
-                if (!(bb > 0.0)) break;                      // b = 0: that step left x = 0 (or b is not finite)
+                if (!(bb > 0.0)) break;                      // b = 0, or not finite
             }
             if (cc.done(it, w)) break;
             if (cc.r1 < 0.25 * best) { best = cc.r1; since = 0; }       // squared residuals
@@ -672,7 +672,11 @@ void coupled_solve(semo_ctx* c, const double* b, double* x, semo_solve_stats* st
                 best = cc.r1;
             }
         }
-        if (!(bb > 0.0)) { it = 0; break; }
+        if (!(bb > 0.0)) {
+            zero_d(c, x, N * sizeof(double));                // 0 * z is NaN where the preconditioner overflows
+            it = 0;
+            break;
+        }
         it = std::min(it, c->sp.maxit_u);
         // true residual
         blk_product<1>(c, C, x, b, r, "cpl_blk_resid");

@@ -1103,6 +1103,10 @@ void spmv_dot(semo_ctx* c, const DevSell<double>& A, const double* x, double* y,
     finish(c, nb, what);
 }
 
+// x = 0 for b = 0: the iteration issued before |b|^2 arrived leaves 0 * z, NaN
+// where the preconditioner overflows
+void zero_x(semo_ctx* c, double* x, size_t n) { zero_d(c, x, n * sizeof(double)); }
+
 // flexible (Polak-Ribiere) PCG with the AMG preconditioner.  x0 = 0,
 // stop at ||r|| <= tol ||b||.
 //
@@ -1221,7 +1225,7 @@ int fpcg(semo_ctx* c, Amg& amg, const DevSell<double>& A, const double* b, doubl
     double bb = 0.0;
     for (it = 1; it <= maxit; ++it) {
         issue(it);
-        if (it == 1 && (bb = cc.bb()) == 0.0) { *relres = 0.0; return 0; }   // b = 0: that step left x = 0
+        if (it == 1 && (bb = cc.bb()) == 0.0) { zero_x(c, x, n); *relres = 0.0; return 0; }
         if (cc.done(it, w)) break;
         if (it < maxit) w = ring_expect(c, 1);
     }
@@ -1274,7 +1278,7 @@ int bicgstab(semo_ctx* c, const DevSell<double>& A, const double* dinv, const do
         SEMO_LAUNCH(c, "bicg_x", 64.0 * n, k_bicg_x, dim3(nblk(n)), dim3(TPB), n, s, ph, sh, sv, t, rh, x, r,
                     red_of(c));
         finish_put(c, nblk(n), W_BICG_RHO);
-        if (it == 1 && (bb = cc.bb()) == 0.0) { *relres = 0.0; return 0; }   // b = 0: that step left x = 0
+        if (it == 1 && (bb = cc.bb()) == 0.0) { zero_x(c, x, n); *relres = 0.0; return 0; }
         if (cc.done(it, w)) break;
     }
     int nbs = nblk((long)A.nslices * 64);
@@ -1348,7 +1352,7 @@ int bicgstab3(semo_ctx* c, const DevSell<double>& A, const double* dinv, const d
     double bb[3], rr[3];
     for (int k = 0; k < 3; ++k) rr[k] = ring_read(c, wr + k);
     for (int k = 0; k < 3; ++k) bb[k] = ring_read(c, wb + k);
-    if (!(bb[0] > 0.0 || bb[1] > 0.0 || bb[2] > 0.0)) it = 0;  // b = 0: that step left x = 0
+    if (!(bb[0] > 0.0 || bb[1] > 0.0 || bb[2] > 0.0)) { zero_x(c, x, 3 * (size_t)n); it = 0; }
     for (int k = 0; k < 3; ++k) {
         double rel = bb[k] > 0.0 ? std::sqrt(rr[k] / bb[k]) : 0.0;
         if (st) { st->iters[k] = bb[k] > 0.0 ? it : 0; st->rel_res[k] = rel; }

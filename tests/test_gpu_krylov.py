@@ -107,3 +107,16 @@ def test_smoother_degree_changed_between_solves(precision):
             its, p = fresh([], degree)
             got, q = fresh(history, degree)
             assert 3 < its < 60 and got == its and np.array_equal(p, q), (history, degree, its, got)
+
+
+@pytest.mark.parametrize("equation, precision, scale", [
+    ("pressure", "fp64", 1.0), ("pressure", "mixed", 1.0), ("pressure", "mixed", 1e40),
+    ("momentum", "fp64", 1.0), ("momentum", "fp64", 1e-311)])
+def test_zero_right_side_gives_zero(equation, precision, scale):
+    """Also where the preconditioner overflows its type (entries above FP32's
+    range, diagonals whose reciprocal is infinite) and no residual says so."""
+    r, c, v, _ = _system(3001, 53, 5)
+    g = _solver(precision)
+    x = g.solveAMGCL(equation, r, c, v * scale, np.zeros(3001))
+    g.close()
+    assert not x.any() and not np.isnan(x).any()
