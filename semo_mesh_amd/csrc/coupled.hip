@@ -385,8 +385,8 @@ __global__ void __launch_bounds__(TPB) k_cpl_update(int nc, double urf_p, double
 
 // device scalars of the block BiCGStab (zero denominators give zero steps,
 // so that an iteration issued past convergence leaves x unchanged)
-enum { C_RHO = 0, C_ALPHA, C_OMEGA, C_BETA, C_RR, C_BB, C_N };
-enum { F_STORE_BB = 0, F_ALPHA, F_OMEGA, F_RR, F_RESTART };
+enum { C_RHO = 0, C_ALPHA, C_OMEGA, C_BETA };
+enum { F_START = 0, F_ALPHA, F_OMEGA, F_RR, F_RESTART };
 
 constexpr int CTPB = 1024;
 // the squared norms (|b|^2, |r|^2) also go to the host
@@ -405,18 +405,17 @@ __global__ void __launch_bounds__(CTPB) k_cfinish(int nb, const double* __restri
     double d0 = sh[0][0], d1 = sh[1][0];
     switch (what) {
     // a (re)start: rh = r, so rho = |r|^2, and p = r by beta = 0 (p = v = 0)
-    case F_STORE_BB: sc[C_BB] = d0; [[fallthrough]];
-    case F_RESTART: sc[C_RR] = d0; sc[C_RHO] = d0; sc[C_BETA] = 0.0; sc[C_OMEGA] = 1.0; break;
+    case F_START:
+    case F_RESTART: sc[C_RHO] = d0; sc[C_BETA] = 0.0; sc[C_OMEGA] = 1.0; break;
     case F_ALPHA: sc[C_ALPHA] = d0 != 0.0 ? sc[C_RHO] / d0 : 0.0; break;     // d0 = rh.v
     case F_OMEGA: sc[C_OMEGA] = d1 != 0.0 ? d0 / d1 : 0.0; break;            // d0 = t.s, d1 = t.t
     case F_RR:       // d0 = r.r, d1 = rh.r
-        sc[C_RR] = d0;
         sc[C_BETA] = (sc[C_RHO] != 0.0 && sc[C_OMEGA] != 0.0) ? (d1 / sc[C_RHO]) * (sc[C_ALPHA] / sc[C_OMEGA]) : 0.0;
         sc[C_RHO] = d1;
         break;
     default: break;
     }
-    if (what == F_STORE_BB || what == F_RR) ring_put(ring, &d0, 1);
+    if (what == F_START || what == F_RR) ring_put(ring, &d0, 1);
 }
 
 // p = r + beta (p - omega v)
@@ -630,7 +629,7 @@ void coupled_solve(semo_ctx* c, const double* b, double* x, semo_solve_stats* st
     };
     int wb = ring_expect(c, 1);
     SEMO_LAUNCH(c, "cpl_bicg_init", 48.0 * N, k_cb_init, dim3(nbv), dim3(TPB), N, b, x, r, rh, p, v, C.red.p);
-    fin(nbv, F_STORE_BB);
+    fin(nbv, F_START);
     hipGraphExec_t exec = nullptr;
     if (graph) {
         std::vector<const void*> key = pressure_vcycle_signature(c, C.tp.p, C.zp.p, true);
@@ -643,7 +642,7 @@ void coupled_solve(semo_ctx* c, const double* b, double* x, semo_solve_stats* st
             key.push_back(q);
         exec = C.graphs.get(c->stream, key, record);
     }
-    // r = b - A x formed before: rh = r, p = v = 0 (F_RESTART keeps |r|^2)
+    // r = b - A x formed before: rh = r, p = v = 0, rho = |r|^2
     auto restart = [&] {
         SEMO_LAUNCH(c, "cpl_bicg_restart", 32.0 * N, k_cb_restart, dim3(nbv), dim3(TPB), N, r, rh, p, v, C.red.p);
         fin(nbv, F_RESTART);

@@ -433,10 +433,12 @@ __device__ inline void ls_store(double* p, double v) {
 // Units are taken in level order by tickets, unit u by the wavefronts of
 // place u mod 4 in their block (one counter would be taken at 14 ns a ticket,
 // 1.9 ms a sweep at 128^3): every block has wavefronts of all four places and
-// each holds at most its current and its next, later unit, so the lowest
-// unfinished unit is always being worked on; all it waits for is finished,
-// so every wait ends whatever else runs on the device.  A unit's cells are of
-// one level: no lane waits for another lane of its wavefront.
+// each holds, besides its current unit, at most two later ones of the same
+// counter.  So the lowest unfinished unit is some wavefront's current one or
+// is come to without a wait: what lies before it on its counter is finished,
+// as is all it waits for.  Every wait ends, whatever else runs on the device.
+// A unit's cells are of one level: no lane waits for another lane of its
+// wavefront.
 // Bound by that chain: 128^3 hexes (382 levels a sweep) 2.8 us a level,
 // against 6.1 us with a launch per level (4.65 -> 2.16 ms for both sweeps).
 template <int NSP, bool FWD>

@@ -63,17 +63,16 @@ __device__ inline void block_partials(double (&v)[2], double* __restrict__ part)
 }
 
 // Krylov scalars in device memory (slots of c->scal)
-enum { S_RZ = 0, S_RR = 2, S_X = 6, S_ALPHA = 10, S_BETA = 11, S_OMEGA = 12,
+enum { S_RZ = 0, S_ALPHA = 10, S_BETA = 11, S_OMEGA = 12,
        S_TT = 14, S_TS = 15, S_RHO = 16, S_AV = 20,
        S_RZ2 = 24, S_ALPHA2 = 26 };   // r.z and alpha of even / odd iterations (in-kernel totals)
 
 // what the last block does with the totals d[0], d[1]
-enum { W_NONE = -1,      // nothing is kept
-       W_STORE = 0,      // s[slot] = d0, s[slot+1] = d1
+enum { W_NONE = 0,       // nothing is kept
        W_FCG_ALPHA,      // d0 = p.Ap:  alpha = rz / p.Ap
        W_FCG_BETA,       // d0 = r.z, d1 = z.Ap: Polak-Ribiere beta, rz = d0
        W_FCG_START,      // d0 = r.z of the first direction: rz = d0, beta = 0
-       W_BICG_INIT,      // d0 = b.b: rho = rr = b.b, beta = 0, alpha = omega = 1
+       W_BICG_INIT,      // d0 = b.b: rho = b.b, beta = 0, alpha = omega = 1
        W_BICG_ALPHA,     // d0 = rh.v: alpha = rho / rh.v
        W_BICG_OMEGA,     // d0 = t.t, d1 = t.s: omega = t.s / t.t
        W_BICG_RHO };     // d0 = r.r, d1 = rh.r: beta = (rho'/rho)(alpha/omega), rho = rho'
@@ -83,9 +82,8 @@ __device__ inline double fcg_beta(double rz_old, double alpha, double zq) {
     return rz_old != 0.0 ? -alpha * zq / rz_old : 0.0;
 }
 
-__device__ void finish_scalars(int what, int slot, const double (&d)[2], double* s) {
+__device__ void finish_scalars(int what, const double (&d)[2], double* s) {
     switch (what) {
-    case W_STORE: s[slot] = d[0]; s[slot + 1] = d[1]; break;
     // zero denominators (an exactly solved system) give zero steps, so that
     // an iteration issued past convergence leaves x unchanged
     case W_FCG_ALPHA: s[S_ALPHA] = fcg_alpha(s[S_RZ], d[0]); break;
@@ -93,13 +91,12 @@ __device__ void finish_scalars(int what, int slot, const double (&d)[2], double*
     case W_FCG_BETA: s[S_BETA] = fcg_beta(s[S_RZ], s[S_ALPHA], d[1]); s[S_RZ] = d[0]; break;
     case W_FCG_START: s[S_BETA] = 0.0; s[S_RZ] = d[0]; break;
     case W_BICG_INIT:
-        s[S_X] = d[0]; s[S_RR] = d[0]; s[S_RHO] = d[0];
+        s[S_RHO] = d[0];
         s[S_BETA] = 0.0; s[S_ALPHA] = 1.0; s[S_OMEGA] = 1.0;
         break;
     case W_BICG_ALPHA: s[S_AV] = d[0]; s[S_ALPHA] = d[0] != 0.0 ? s[S_RHO] / d[0] : 0.0; break;
     case W_BICG_OMEGA: s[S_TT] = d[0]; s[S_TS] = d[1]; s[S_OMEGA] = d[0] != 0.0 ? d[1] / d[0] : 0.0; break;
     case W_BICG_RHO:
-        s[S_RR] = d[0];
         s[S_BETA] = (s[S_RHO] != 0.0 && s[S_OMEGA] != 0.0) ? (d[1] / s[S_RHO]) * (s[S_ALPHA] / s[S_OMEGA]) : 0.0;
         s[S_RHO] = d[1];
         break;
@@ -118,7 +115,7 @@ __device__ inline void reduce2(double (&v)[2], const Red& rd) { block_partials(v
 constexpr int FTPB = 1024;
 // ring (optional): the host gets d0, and d1 where nput = 2
 __global__ void __launch_bounds__(FTPB) k_finish(int nb, const double* __restrict__ part, double* __restrict__ s,
-                                                 int what, int slot, Ring ring, int nput) {
+                                                 int what, Ring ring, int nput) {
     double a0 = 0.0, a1 = 0.0;
     const double2* p2 = reinterpret_cast<const double2*>(part);
     for (int i = threadIdx.x; i < nb; i += FTPB) { double2 v = p2[i]; a0 += v.x; a1 += v.y; }
@@ -134,7 +131,7 @@ __global__ void __launch_bounds__(FTPB) k_finish(int nb, const double* __restric
     }
     if (threadIdx.x == 0) {
         double d[2] = {sh[0][0], sh[1][0]};
-        finish_scalars(what, slot, d, s);
+        finish_scalars(what, d, s);
         ring_put(ring, d, nput);
     }
 }
@@ -659,7 +656,7 @@ __global__ void __launch_bounds__(TPB) k_bicg_x(int n, const double* __restrict_
 // systems runs in lockstep, so every matrix pass serves all three.  Vectors
 // are [3][n] (component k at +k*n); the Krylov scalars of component k live
 // in slots Q_* + k of the device scalar array.
-enum { Q_RHO = 32, Q_ALPHA = 35, Q_OMEGA = 38, Q_BETA = 41, Q_BB = 44, Q_RR = 47 };
+enum { Q_RHO = 32, Q_ALPHA = 35, Q_OMEGA = 38, Q_BETA = 41, Q_BB = 44 };
 enum { F3_INIT = 0, F3_ALPHA, F3_OMEGA, F3_RHO, F3_STORE };
 
 __device__ inline void block_partials6(double (&v)[6], double* __restrict__ part) {
@@ -699,13 +696,12 @@ __global__ void __launch_bounds__(1024) k_finish6(int nb, const double* __restri
     for (int k = 0; k < 3; ++k) {
         switch (what) {
         case F3_INIT:
-            s[Q_BB + k] = d[k]; s[Q_RR + k] = d[k]; s[Q_RHO + k] = d[k];
+            s[Q_BB + k] = d[k]; s[Q_RHO + k] = d[k];
             s[Q_ALPHA + k] = 1.0; s[Q_OMEGA + k] = 1.0; s[Q_BETA + k] = 0.0;
             break;
         case F3_ALPHA: s[Q_ALPHA + k] = d[k] != 0.0 ? s[Q_RHO + k] / d[k] : 0.0; break;
         case F3_OMEGA: s[Q_OMEGA + k] = d[3 + k] != 0.0 ? d[k] / d[3 + k] : 0.0; break;
         case F3_RHO: {
-            s[Q_RR + k] = d[k];
             double rho = s[Q_RHO + k], om = s[Q_OMEGA + k];
             s[Q_BETA + k] = (rho != 0.0 && om != 0.0) ? (d[3 + k] / rho) * (s[Q_ALPHA + k] / om) : 0.0;
             s[Q_RHO + k] = d[3 + k];
@@ -714,7 +710,7 @@ __global__ void __launch_bounds__(1024) k_finish6(int nb, const double* __restri
             mx = (rel > mx || rel != rel) ? rel : mx;
             break;
         }
-        default: s[Q_RR + k] = d[k]; break;
+        default: break;
         }
     }
     if (what == F3_RHO) ring_put(ring, &mx, 1);
@@ -1082,15 +1078,15 @@ Red red_of(semo_ctx* c) { return Red{c->red.p}; }
 
 
 // sums the partials of the previous launch (nb blocks) and applies `what`
-void finish(semo_ctx* c, int nb, int what, int slot = 0, const double* part = nullptr) {
+void finish(semo_ctx* c, int nb, int what, const double* part = nullptr) {
     SEMO_LAUNCH(c, "krylov_finish", 16.0 * nb + 8.0, k_finish, dim3(1), dim3(FTPB), nb, part ? part : c->red.p,
-                c->scal.p, what, slot, Ring{nullptr, nullptr}, 0);
+                c->scal.p, what, Ring{nullptr, nullptr}, 0);
 }
 // ... and sends d0 (and d1: nput = 2) to the host: the caller has asked for
 // the words (ring_expect)
-void finish_put(semo_ctx* c, int nb, int what, int slot = 0, const double* part = nullptr, int nput = 1) {
+void finish_put(semo_ctx* c, int nb, int what, const double* part = nullptr, int nput = 1) {
     SEMO_LAUNCH(c, "krylov_finish", 16.0 * nb + 8.0, k_finish, dim3(1), dim3(FTPB), nb, part ? part : c->red.p,
-                c->scal.p, what, slot, ring_of(c), nput);
+                c->scal.p, what, ring_of(c), nput);
 }
 
 // y = A x with dots of y (see k_spmv_dot), for the fine-level sliced-ELL operator
@@ -1162,14 +1158,14 @@ int fpcg(semo_ctx* c, Amg& amg, const DevSell<double>& A, const double* b, doubl
         if (first) {
             SEMO_LAUNCH(c, "fcg_init", 16.0 * n + prep_bytes, k_fcg_init, dim3(nbr), dim3(TPB), n, b, r, Red{part_r},
                         pp);
-            finish_put(c, nbr, W_NONE, 0, part_r);
+            finish_put(c, nbr, W_NONE, part_r);
         }
         if (mixed) vcycle<float>(c, amg, 0, cheb_degree(c), r, z, prep, d);
         else vcycle<double>(c, amg, 0, cheb_degree(c), r, z, prep, d);
         if (!prep)
             SEMO_LAUNCH(c, "krylov_dot", 32.0 * n, k_dot, dim3(nbz), dim3(TPB), n, r, z, z, q, Red{part_z});
         FcgIn in{part_z, own_totals ? nbz : 0, it & 1, first ? 1 : 0};
-        if (!own_totals) finish(c, nbz, first ? W_FCG_START : W_FCG_BETA, 0, part_z);
+        if (!own_totals) finish(c, nbz, first ? W_FCG_START : W_FCG_BETA, part_z);
         // p = z + beta p, q = A p
         if (z32)
             SEMO_LAUNCH(c, "spmv_xpby_fp64", op_bytes(A, 3) + 4.0 * n, k_spmv_xpby<float>, dim3(nbs), dim3(TPB), n,
@@ -1180,10 +1176,10 @@ int fpcg(semo_ctx* c, Amg& amg, const DevSell<double>& A, const double* b, doubl
                         A.col.p, dc, A.val.p, A.diag.p, c->scal.p, in, z, po, pn, q, Red{part_p});
         in.part = part_p;
         if (own_totals) in.nb = nbs;
-        else finish(c, nbs, W_FCG_ALPHA, 0, part_p);
+        else finish(c, nbs, W_FCG_ALPHA, part_p);
         SEMO_LAUNCH(c, "fcg_update", 48.0 * n + prep_bytes, k_fcg_update, dim3(nbr), dim3(TPB), n, c->scal.p, in, x, r,
                     pn, q, Red{part_r}, pp);
-        finish_put(c, nbr, W_NONE, 0, part_r);
+        finish_put(c, nbr, W_NONE, part_r);
     };
     // The kernels of an iteration go out as one graph, the first iteration's
     // with the start, the even and the odd ones' each their own.  (As a graph
@@ -1233,7 +1229,7 @@ int fpcg(semo_ctx* c, Amg& amg, const DevSell<double>& A, const double* b, doubl
     w = ring_expect(c, 1);
     SEMO_LAUNCH(c, "true_resid_fp64", op_bytes(A, 2), k_resid_norm, dim3(nbs), dim3(TPB), n, A.sl_ptr.p, A.col.p,
                 dc, A.val.p, A.diag.p, x, b, Red{part_r});
-    finish_put(c, nbs, W_NONE, 0, part_r);
+    finish_put(c, nbs, W_NONE, part_r);
     *relres = std::sqrt(ring_read(c, w)) / std::sqrt(bb);
     return std::min(it, maxit);
 }
@@ -1541,7 +1537,7 @@ std::vector<const void*> pressure_vcycle_signature(semo_ctx* c, const double* r6
 
 double2 sum_to_host(semo_ctx* c, int nb, const double* part) {
     int w = ring_expect(c, 2);
-    finish_put(c, nb, W_NONE, 0, part, 2);
+    finish_put(c, nb, W_NONE, part, 2);
     double a = ring_read(c, w);
     return make_double2(a, ring_read(c, w + 1));
 }
