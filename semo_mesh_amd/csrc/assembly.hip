@@ -569,8 +569,8 @@ __global__ void __launch_bounds__(TPB) k_lsq1g(
 // same bits as k_grad_minmax / k_lsq1 / k_curv_kappa, which gather every
 // neighbour from the L2 in 128-byte lines (1.33M tets: 12 GB a pass, its
 // bandwidth).  Bound by LDS latency at 2 to 3 workgroups a CU.  us a pass,
-// gathered -> staged: 1.33M tets one field 348 -> 149, U, V, W 623 -> 382, five
-// fields 701 -> 660, curvature 587 -> 240; 19734 tets (latency) 23 -> 24, 60 -> 28,
+// gathered -> staged: 1.33M tets one field 348 -> 165, U, V, W 623 -> 378, five
+// fields 701 -> 678, curvature 587 -> 234; 19734 tets (latency) 23 -> 24, 60 -> 28,
 // 64 -> 31, 52 -> 21; 32^3 hexes U, V, W 28 -> 18, five fields 30 -> 19.
 struct ClusterK {
     const int* __restrict__ cell;
