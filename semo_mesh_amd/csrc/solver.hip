@@ -1323,6 +1323,7 @@ int bicgstab3(semo_ctx* c, const DevSell<double>& A, const double* dinv, const d
     int wb = ring_expect(c, 3);
     fin(nb, F3_INIT);
     int it = 0;
+    double bb[3] = {0.0, 0.0, 0.0};
     ConvCheck cc(c, tol * tol, 1.0);
     for (it = 1; it <= maxit; ++it) {
         SEMO_LAUNCH(c, "bicg3_p", 128.0 * n, k_bicg3_p, dim3(nb), dim3(TPB), n, s, r, v, dinv, p, ph);
@@ -1338,6 +1339,10 @@ int bicgstab3(semo_ctx* c, const DevSell<double>& A, const double* dinv, const d
         SEMO_LAUNCH(c, "bicg3_x", 192.0 * n, k_bicg3_x, dim3(nb), dim3(TPB), n, s, ph, sh, sv, t, rh, x, r, part);
         int w = ring_expect(c, 1);
         fin(nb, F3_RHO);
+        if (it == 1) {                       // later iterations' words come around to these
+            for (int k = 0; k < 3; ++k) bb[k] = ring_read(c, wb + k);
+            if (!(bb[0] > 0.0 || bb[1] > 0.0 || bb[2] > 0.0)) break;
+        }
         if (cc.done(it, w)) break;
     }
     it = std::min(it, maxit);
@@ -1345,9 +1350,8 @@ int bicgstab3(semo_ctx* c, const DevSell<double>& A, const double* dinv, const d
     int wr = ring_expect(c, 3);
     spmv3(2, x, r, b);
     fin(nbs, F3_STORE);
-    double bb[3], rr[3];
+    double rr[3];
     for (int k = 0; k < 3; ++k) rr[k] = ring_read(c, wr + k);
-    for (int k = 0; k < 3; ++k) bb[k] = ring_read(c, wb + k);
     if (!(bb[0] > 0.0 || bb[1] > 0.0 || bb[2] > 0.0)) { zero_x(c, x, 3 * (size_t)n); it = 0; }
     for (int k = 0; k < 3; ++k) {
         double rel = bb[k] > 0.0 ? std::sqrt(rr[k] / bb[k]) : 0.0;

@@ -120,3 +120,42 @@ def test_zero_right_side_gives_zero(equation, precision, scale):
     x = g.solveAMGCL(equation, r, c, v * scale, np.zeros(3001))
     g.close()
     assert not x.any() and not np.isnan(x).any()
+
+
+def test_momentum_residuals_past_the_rings_end():
+    """A diffusion-dominated momentum system of a long column of cells, more
+    than 1024 lockstep iterations: the relative residuals are those of the
+    exported system, of which summing in another order changes 2e-10
+    (measured; bar 1e-3)."""
+    from semo_mesh_amd.cases import BC_FIXED_VALUE, BC_ZERO_GRADIENT, PatchBC, cavity_case
+    from semo_mesh_amd.mesh import hex_mesh
+    from semo_mesh_amd.solver import GpuSolver
+    m = hex_mesh(5000, 1, 1)
+    case = cavity_case(dt=1e-3)
+    free = PatchBC(u_type=BC_ZERO_GRADIENT)
+    case.bcs = {k: free for k in case.bcs}
+    case.bcs["pref"] = PatchBC(p_type=BC_FIXED_VALUE, u_type=BC_ZERO_GRADIENT)
+    case.bcs["xmin"] = PatchBC(u_type=BC_FIXED_VALUE, u_value=(1.0, 0.5, 0.2))
+    case.bcs["xmax"] = PatchBC(u_type=BC_FIXED_VALUE)
+    g = GpuSolver(0)
+    g.upload_mesh(m)
+    g.set_case(case)
+    g.set_momentum_solver("jacobi")
+    g.set_solver("mixed", tol_p=1e-2, tol_u=1e-8)
+    g.incompressiblePressureBased(1)
+    case.dt, case.mu = 1e6, (1e3, 1e3)
+    g.set_case(case)
+    g.set_solver("fp64", tol_u=1e-8, maxit_u=20000)
+    rng = np.random.default_rng(3)
+    for f in "UVW":
+        g.set_field(f, rng.standard_normal(m.n_cells))
+    g.calcMomentumEqs()
+    st = g.last_stats
+    r, c, v, b = g.matrix("momentum")
+    x = [g.get_field(f) for f in ("x0", "x1", "x2")]
+    g.close()
+    print(st.iters[0], list(st.rel_res))
+    assert st.iters[0] > 1100
+    for k in range(3):
+        rel = np.linalg.norm(b[k] - np.bincount(r, v * x[k][c], m.n_cells)) / np.linalg.norm(b[k])
+        assert abs(st.rel_res[k] - rel) <= 1e-3 * rel
