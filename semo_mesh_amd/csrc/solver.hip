@@ -912,6 +912,7 @@ inline void cheb_interval(const AmgLevel& L, double& lo, double& hi) { hi = 1.1 
 // what the last step of a V-cycle does for the FCG loop around it (degree 1):
 // its result goes to z in the V-cycle's precision, with the block partials of
 // r.z and z.q
+// (the finest operator sliced ELL)
 struct VcDot {
     void* z;
     const double *r, *q;
@@ -1122,7 +1123,9 @@ int fpcg(semo_ctx* c, Amg& amg, const DevSell<double>& A, const double* b, doubl
     c->kv64.ensure(8 * ln);
     double* r = c->kv64.p; double* z = r + ln; double* p = z + ln; double* q = p + ln; double* p2 = q + ln;
     // degree-1 smoothing, at least two levels: the kernels that produce r also
-    // write the V-cycle's level-0 input, and its last step the dots
+    // write the V-cycle's level-0 input, and its last step the dots, where the
+    // finest operator is sliced ELL (rows of more than ten or very unequal
+    // numbers of neighbours are CSR: k_row smooths, k_dot follows)
     Prep pp{};
     bool prep = cheb_degree(c) == 1 && amg.lv.size() >= 2 && amg.lv[0].n == n;
     if (prep) {
@@ -1144,9 +1147,10 @@ int fpcg(semo_ctx* c, Amg& amg, const DevSell<double>& A, const double* b, doubl
     double* part_r = part_p + 2 * (size_t)nbs;
     bool own_totals = std::max(nbs, nbr) <= TOTAL_MAX;
     const VcDot vd{z, r, q, part_z};
-    int nbz = prep ? nbs : rblk(n);                       // blocks of the r.z, z.q partials
-    bool z32 = prep && mixed;                             // z as the FP32 V-cycle leaves it
-    const VcDot* d = prep ? &vd : nullptr;
+    bool fused = prep && (mixed ? amg.lv[0].A32.lanes : amg.lv[0].A64.lanes) == 0;
+    int nbz = fused ? nbs : rblk(n);                      // blocks of the r.z, z.q partials
+    bool z32 = fused && mixed;                            // z as the FP32 V-cycle leaves it
+    const VcDot* d = fused ? &vd : nullptr;
     const int16_t* dc = A.dcol.n ? A.dcol.p : nullptr;
     double prep_bytes = prep ? (mixed ? 8.0 : 16.0) * n : 0.0;     // the V-cycle's b and x written
     // iteration `it`: one ring word, its squared residual; the first is
@@ -1162,7 +1166,7 @@ int fpcg(semo_ctx* c, Amg& amg, const DevSell<double>& A, const double* b, doubl
         }
         if (mixed) vcycle<float>(c, amg, 0, cheb_degree(c), r, z, prep, d);
         else vcycle<double>(c, amg, 0, cheb_degree(c), r, z, prep, d);
-        if (!prep)
+        if (!fused)
             SEMO_LAUNCH(c, "krylov_dot", 32.0 * n, k_dot, dim3(nbz), dim3(TPB), n, r, z, z, q, Red{part_z});
         FcgIn in{part_z, own_totals ? nbz : 0, it & 1, first ? 1 : 0};
         if (!own_totals) finish(c, nbz, first ? W_FCG_START : W_FCG_BETA, part_z);

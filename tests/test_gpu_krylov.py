@@ -50,6 +50,47 @@ def test_totals_on_both_sides_of_the_block_limit(n, precision):
     assert 2 < its < 60 and res <= 2e-9
 
 
+def _dense_stencil(m, ragged):
+    """Every cell of an m^3 grid coupled to its 26 neighbours or, ragged, to
+    its six and every 64th cell also to 24 further ones."""
+    rng = np.random.default_rng(11)
+    n = m ** 3
+    idx = np.arange(n).reshape(m, m, m)
+    pairs = []
+    for dz, dy, dx in np.ndindex(3, 3, 3):
+        d = np.array([dz, dy, dx]) - 1
+        if tuple(d) <= (0, 0, 0) or (ragged and np.abs(d).sum() > 1):
+            continue
+        lo, hi = np.maximum(-d, 0), m - np.maximum(d, 0)
+        i = idx[lo[0]:hi[0], lo[1]:hi[1], lo[2]:hi[2]].ravel()
+        pairs.append((i, i + d @ (m * m, m, 1), 1.0 / (d @ d)))
+    if ragged:
+        i = np.repeat(np.arange(0, n, 64), 24)
+        j = (i + 2 + np.arange(i.size) % 24) % n
+        pairs.append((i, j, 0.01))
+    r, c, v = [np.arange(n)], [np.arange(n)], [np.full(n, 1e-2)]
+    for i, j, w in pairs:
+        w = w * (1.0 + 0.2 * rng.random(i.size))
+        r += [i, j, i, j]; c += [j, i, i, j]; v += [-w, -w, w, w]
+    return np.concatenate(r), np.concatenate(c), np.concatenate(v), rng.standard_normal(n)
+
+
+@pytest.mark.parametrize("ragged", [False, True])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_finest_level_with_long_or_unequal_rows(precision, ragged):
+    """Rows of 26 neighbours, and slices with one long row among short ones:
+    the hierarchy keeps its finest operator in CSR, the Krylov product in
+    sliced ELL.  Smoothed aggregation takes 13 iterations."""
+    r, c, v, b = _dense_stencil(12, ragged)
+    g = _solver(precision)
+    x = g.solveAMGCL("pressure", r, c, v, b)
+    its, levels = g.last_stats.iters[0], g.last_stats.n_levels
+    g.close()
+    res = np.linalg.norm(b - np.bincount(r, v * x[c], b.size)) / np.linalg.norm(b)
+    print(precision, ragged, its, levels, res)
+    assert levels >= 2 and its <= 20 and res <= 2e-9
+
+
 def test_ring_of_residuals_wraps():
     """Solves until well over 1024 residuals have passed through the ring:
     each gives the first one's bits."""
