@@ -477,7 +477,8 @@ inline void ring_init(semo_ctx* c) {
     c->seq = 0;
 }
 inline Ring ring_of(semo_ctx* c) { ring_init(c); return Ring{c->pin, c->d_seq.p}; }
-// the first of the next n words, emptied; the launch that stores them follows
+// the first of the next n words, emptied; the launch that stores them follows.
+// They are read before RING more are asked for.
 inline int ring_expect(semo_ctx* c, int n) {
     ring_init(c);
     int first = c->seq & (RING - 1);
